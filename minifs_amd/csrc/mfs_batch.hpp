@@ -43,6 +43,8 @@ struct BatchSolve {
     const typename Real<R>::vec4* fgeo_r;
     R *gx, *gy, *gz;
     const int* snode;             // tetrahedral meshes: slot nodes (nullptr otherwise)
+    const int *snb, *depmask;     // slot neighbours; boundary slots of the gradient
+    const typename Real<R>::vec4* sgeo;  // slot geometry (gradient)
     const double4* sgeo64;        // FP64 slot geometry, distances and sides (residual kernel)
     const double* sdn;
     const int* sflip;
@@ -56,7 +58,7 @@ __global__ __launch_bounds__(kBlock) void k_b_flux_ts(const BatchSolve<R>* __res
     const BatchSolve<R>& S = T[cell_solve[blockIdx.x]];
     const int lb = (int)blockIdx.x - S.blk0_cell;
     const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;  // XCD-aware inside the solve
-    flux_ts_slot_body<MAXF == 4 ? 4 : 8, MIXED>(lg * kBlock + (int)threadIdx.x, S.nC, S.sw.snb, S.sgeo64, S.sdn,
+    flux_ts_slot_body<MAXF == 4 ? 4 : 8, MIXED>(lg * kBlock + (int)threadIdx.x, S.nC, S.snb, S.sgeo64, S.sdn,
                                                 S.sflip, S.q, S.vol, S.res, S.dt, S.diag, S.part + lb, S.nblk_cell, S.K,
                                                 S.cfl, S.cfl_min, S.q32, S.diag32);
 }
@@ -79,7 +81,7 @@ __global__ __launch_bounds__(kBlock) void k_b_clamp(const BatchSolve<R>* __restr
                     S.ratio_dtmax, S.K, S.q32 ? S.diag32 : nullptr);
 }
 
-template <bool FWD, int LPC, typename R>
+template <bool FWD, int MAXD, typename R>
 __global__ __launch_bounds__(kSweepBlock) void k_b_sweep(const BatchSolve<R>* __restrict__ T,
                                                         const int2* __restrict__ items, int nitems, int* tickets,
                                                         int* tickets_next, int ngroups) {
@@ -87,23 +89,21 @@ __global__ __launch_bounds__(kSweepBlock) void k_b_sweep(const BatchSolve<R>* __
     // Item i belongs to ticket group i mod ngroups; the waves of the
     // workgroups of group g take its items in order from the group's
     // counter, as in the single-solve sweep.
-    if (blockIdx.x == 0 && threadIdx.x < kTicketGroups) tickets_next[threadIdx.x * kTicketStride] = 0;
+    clear_tickets(tickets_next);
     const int grp = (int)blockIdx.x % ngroups;
     int* const ctr = tickets + grp * kTicketStride;
-    const int lane = (int)threadIdx.x & 63;
-    int tk = 0;
-    if (lane == 0) tk = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    tk = __shfl(tk, 0, 64);
+    int tk = __builtin_amdgcn_readfirstlane(take_ticket(ctr));
     while (true) {
         const int it = grp + ngroups * tk;
         if (it >= nitems) return;
         int next = 0;
-        if (lane == 0) next = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const int2 su = items[it];
         const SweepArgs<R>& A = T[su.x].sw;
-        if (__hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-            (void)sweep_chunk<FWD, LPC, R, false>(A, T[su.x].K, FWD ? su.y : A.nchunks - 1 - su.y);
-        tk = __shfl(next, 0, 64);
+        if (__hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+            next = take_ticket(ctr);  // the solve has failed: its chunks are passed over
+        else
+            (void)sweep_chunk<FWD, MAXD, R, kWideChunks>(A, T[su.x].K, su.y, ctr, next);
+        tk = __builtin_amdgcn_readfirstlane(next);
     }
 }
 
@@ -124,7 +124,7 @@ __global__ __launch_bounds__(kBlock) void k_b_grad(const BatchSolve<R>* __restri
     const int lb = (int)blockIdx.x - S.blk0_cell;
     const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
     if (MAXF == 4 && S.snode)
-        grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.sw.snb, S.sw.sgeo, S.snode, S.sw.depmask,
+        grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask,
                          S.qnew, S.qn, S.vol, S.gx, S.gy, S.gz);
     else
         grad_body<MAXF, R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn,
@@ -185,7 +185,7 @@ __global__ __launch_bounds__(kBlock) void k_b_grad_claim(const BatchSolve<R>* __
         const int lb = gb - S.blk0_cell;
         const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
         if (MAXF == 4 && S.snode)
-            grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.sw.snb, S.sw.sgeo, S.snode, S.sw.depmask,
+            grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask,
                              S.qnew, S.qn, S.vol, S.gx, S.gy, S.gz);
         else
             grad_body<MAXF, R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn,
@@ -211,12 +211,12 @@ __global__ __launch_bounds__(kBlock) void k_b_grad_flux_ts(const BatchSolve<R>* 
     const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
     const int c = lg * kBlock + (int)threadIdx.x;
     if (MAXF == 4 && S.snode)
-        grad_tet_body<R>(c, S.nC, S.n, S.sw.snb, S.sw.sgeo, S.snode, S.sw.depmask, S.qnew, S.qn, S.vol, S.gx, S.gy,
+        grad_tet_body<R>(c, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask, S.qnew, S.qn, S.vol, S.gx, S.gy,
                          S.gz);
     else
         grad_body<MAXF, R>(c, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn, S.btype, S.qnew, S.qn, S.vol,
                            S.gx, S.gy, S.gz);
-    flux_ts_slot_body<MAXF == 4 ? 4 : 8, MIXED>(c, S1.nC, S1.sw.snb, S1.sgeo64, S1.sdn, S1.sflip, S1.q, S1.vol,
+    flux_ts_slot_body<MAXF == 4 ? 4 : 8, MIXED>(c, S1.nC, S1.snb, S1.sgeo64, S1.sdn, S1.sflip, S1.q, S1.vol,
                                                 S1.res, S1.dt, S1.diag, S1.part + lb, S1.nblk_cell, S1.K, S1.cfl,
                                                 S1.cfl_min, S1.q32, S1.diag32);
 }

@@ -77,9 +77,19 @@ struct mfs_ctx {
     std::vector<int> node_of_dev;  // host: device node -> mesh node
     std::vector<int> cell_of_dev;  // host: device cell -> mesh cell
     // sweeps
-    int4* crun = nullptr;       // per position of the flat order: first cell, count, rep fwd, rep bwd
-    int* pos = nullptr;         // per chunk (device order): its position in the flat order
-    int* tile_chunk = nullptr;  // ntiles+1: first chunk of each tile
+    // per direction (forward, backward): the schedule and the dependency
+    // tables (SweepLayout in mfs_prep.hpp)
+    struct Sweep {
+        int nchunk = 0;
+        int tail = 0;               // chunks of the thin tail
+        int4* crec = nullptr;
+        int* dnb = nullptr;
+        double4* dgeo = nullptr;    // FP64 operator
+        float4* dgeo32 = nullptr;   // FP32 operator (mixed precision)
+        int* tile_chunk = nullptr;
+        int* pos = nullptr;
+    } sweep[2];
+    unsigned short* cdep = nullptr;  // per cell and direction: first dependency in the chunk, count
     int* snb = nullptr;         // lpc per device cell: neighbour across the slot's face
     double4* sgeo = nullptr;    // lpc per device cell: normal away from the cell, area
     float4* sgeo32 = nullptr;   // the same in FP32 (mixed precision)
@@ -103,17 +113,17 @@ struct mfs_ctx {
     bool gpend[2] = {false, false};
     int gradient_stream = 1;  // 1: on the solver stream (fused with the next residual pass), 2-5: second stream
     int cell0 = 0;  // device id of mesh cell 0
-    int nchunk = 0, lpc = 4;
+    int lpc = 4;  // slots per cell of the slot tables
     int nlev = 0;
     int sweep_grid = 0;  // resident workgroups of the sweep launch
-    // The sweeps' thin tail: positions [tail_u, nchunk) of the flat order
-    // are the longest run of thin levels (at most kThinLevelChunks chunks
-    // each) that ends the order.  With tail_grid > 0 each sweep runs as two
-    // launches, its wide levels on sweep_grid workgroups and its tail on
-    // tail_grid, so that other work can fill the CUs the tail leaves idle.
-    int tail_u = 0;
+    // The sweeps' thin tail: the longest run of thin levels that ends the
+    // forward order.  With tail_grid > 0 each sweep runs as two launches, its
+    // wide levels on sweep_grid workgroups and its tail on tail_grid, so that
+    // other work can fill the CUs the tail leaves idle.
     int tail_grid = 0;
-    int tail_cells = 0;  // cells of the chunks at positions [tail_u, nchunk)
+    bool all_thin = false;  // every level is thin
+    int tail_chunks = 0;  // its width in groups of 64/lpc cells per tile
+    int tail_cells = 0;
     int compute_units = 0;  // CUs of the device
     // reductions and history
     double* part = nullptr;  // 8 * nblk, value-major: 5 squared-norm partials, dt min, dt max, spare

@@ -104,12 +104,11 @@ constexpr int kDefaultGradientStreamMixed = 5;
 // 14.20/14.59/14.52, mixed precision 11.73/12.00/11.47.
 constexpr int kDefaultBatchGradientStreamFP64 = 1;
 constexpr int kDefaultBatchGradientStreamMixed = 4;
-// The sweeps' thin tail runs as a launch of its own on this many
-// workgroups (a thin level has at most 64 chunks), when it holds at least
-// kMinTailChunks chunks.  6.0M cells, FP64, gradient mode 5, ms per
-// iteration for 32/64/128/256 workgroups: 4.08/4.04/4.05/4.05.
+// The sweeps' thin tail runs as a launch of its own on this many workgroups
+// of kThinWaves waves, all on one XCD (k_sweep_xcd; a thin level has at most
+// 64 groups of cells), when it holds at least kMinTailChunks of them.
 constexpr int kDefaultTailGrid = 64;
-constexpr int kMinTailChunks = 256;
+constexpr int kThinWaves = 2;  // waves per workgroup of an XCD-local launch of thin levels
 
 #include "mfs_kernels.hpp"
 #include "mfs_sweep.hpp"
@@ -665,58 +664,74 @@ bool launch_diag(mfs_ctx* ctx, bool clamp_only) {
 
 // Whether the sweeps run as two launches each (wide levels, thin tail).
 bool sweep_split(const mfs_ctx* ctx) {
-    return !ctx->sweep_by_tiles && ctx->tail_grid > 0 && ctx->tail_u < ctx->nchunk;
+    return !ctx->sweep_by_tiles && ctx->tail_grid > 0 && ctx->tail_chunks > 0;
 }
 
 // Workgroups of the thin-tail launch of a split sweep.
 int tail_workgroups(const mfs_ctx* ctx) {
-    const int units = (ctx->nchunk - ctx->tail_u + ctx->sweep_waves - 1) / ctx->sweep_waves;
+    const int units = (ctx->tail_chunks + ctx->sweep_waves - 1) / ctx->sweep_waves;
     return std::max(1, std::min({ctx->tail_grid, ctx->sweep_grid, units}));
 }
 
-// The two sweeps and the update.  `after` is enqueued after the forward
-// sweep, or, with at_tail on a split sweep, after its wide levels, before
-// its thin tail.
-template <int LPC, typename R>
-bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_tail) {
-    dev::SweepArgs<R> A;
+// The sweeps' arguments for an iteration that starts from state buffer `cur`;
+// the launch fills in its tickets and its range.
+template <typename R>
+void sweep_args(dev::SweepArgs<R>& A, const mfs_ctx* ctx, int cur) {
+    A = dev::SweepArgs<R>{};
     A.nC = ctx->nC;
     A.nq = ctx->nC + ctx->nB;
-    A.nchunks = ctx->nchunk;
     A.ntiles = ctx->ntiles;
-    A.tile_chunk = ctx->tile_chunk;
-    A.pos = ctx->pos;
-    A.flat = ctx->sweep_by_tiles ? 0 : 1;
-    A.crun = ctx->crun;
-    A.snb = ctx->snb;
+    for (int d = 0; d < 2; ++d) {
+        const mfs_ctx::Sweep& S = ctx->sweep[d];
+        A.dir[d].nchunks = S.nchunk;
+        A.dir[d].crec = S.crec;
+        A.dir[d].dnb = S.dnb;
+        A.dir[d].tile_chunk = S.tile_chunk;
+        A.dir[d].pos = S.pos;
+        if constexpr (sizeof(R) == sizeof(double))
+            A.dir[d].dgeo = S.dgeo;
+        else
+            A.dir[d].dgeo = S.dgeo32;
+    }
+    A.cdep = ctx->cdep;
     if constexpr (sizeof(R) == sizeof(double)) {
-        A.sgeo = ctx->sgeo;
-        A.q = ctx->q[ctx->cur];
+        A.q = ctx->q[cur];
         A.diag = ctx->diag;
         A.dqf = ctx->dqf;
         A.dqb = ctx->dq;
     } else {
-        A.sgeo = ctx->sgeo32;
         A.q = ctx->q32;
         A.diag = ctx->diag32;
         A.dqf = ctx->dqf32;
         A.dqb = ctx->dq32;
     }
-    A.q64 = ctx->q[ctx->cur];
+    A.q64 = ctx->q[cur];
     A.res = ctx->res;
-    A.qout = ctx->q[1 - ctx->cur];
+    A.qout = ctx->q[1 - cur];
     A.err = ctx->err;
-    A.depmask = ctx->depmask;
     A.cell0 = ctx->cell0;
-    const dim3 block(64 * ctx->sweep_waves);
-    const int units = A.flat ? (A.nchunks + ctx->sweep_waves - 1) / ctx->sweep_waves : A.ntiles;
+}
+
+// The two sweeps and the update.  `after` is enqueued after the forward
+// sweep, or, with at_tail on a split sweep, after its wide levels, before
+// its thin tail.
+template <int MAXD, typename R>
+bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_tail) {
+    dev::SweepArgs<R> A;
+    sweep_args(A, ctx, ctx->cur);
+    const bool flat = !ctx->sweep_by_tiles;
+    const int nf = ctx->sweep[0].nchunk, nb = ctx->sweep[1].nchunk;
+    const int units = flat ? (std::max(nf, nb) + ctx->sweep_waves - 1) / ctx->sweep_waves : A.ntiles;
     const dim3 grid((unsigned)std::max(1, std::min(ctx->sweep_grid, units)));
     // A split sweep runs its wide levels on the resident grid and its thin
     // tail on a small one: the forward sweep ends with the tail and the
     // backward sweep starts with it.
     const bool split = sweep_split(ctx);
-    const int nt = A.nchunks - ctx->tail_u;  // steps of the tail
+    const int wf = nf - ctx->sweep[0].tail, tb = ctx->sweep[1].tail;  // forward: wide chunks; backward: tail chunks
     const dim3 tgrid((unsigned)(split ? tail_workgroups(ctx) : 1));
+    // A mesh of thin levels only runs its sweeps on one XCD whole.
+    const bool local = flat && !split && ctx->all_thin;
+    const dim3 lgrid(std::min<unsigned>(grid.x, dev::kDefaultTailGrid));
     // Each launch takes its tickets from one counter set and zeroes the
     // other for the next launch.  The launches of an iteration alternate
     // between the two sets and are even in number, so every iteration's
@@ -724,29 +739,37 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     int* const tk[2] = {ctx->tickets, ctx->tickets + kTicketGroups * kTicketStride};
     int set = 0;
     // ev0 / ev1: the timing events that this launch's start / end set
-    auto launch = [&](const void* fn, dim3 g, int ubeg, int uend, const char* what, hipEvent_t ev0,
+    auto launch = [&](const void* fn, bool thin, dim3 g, int ubeg, int uend, const char* what, hipEvent_t ev0,
                       hipEvent_t ev1) {
         A.ubeg = ubeg;
         A.uend = uend;
         A.ngroups = std::min(kTicketGroups, (int)g.x);
-        A.run_shift = g.x == grid.x ? dev::kWideRunShift : 0;
+        A.run_shift = dev::kWideRunShift;
         A.tickets = tk[set];
         A.tickets_next = tk[1 - set];
         set ^= 1;
-        void* args[] = {&A, &ctx->K};
-        return hip_ok(ctx, hipExtLaunchKernel(fn, g, block, args, 0, ctx->stream, ev0, ev1, 0), what);
+        int join = (int)g.x;
+        void* args[] = {&A, &ctx->K, &join};
+        if (thin) g.x *= dev::kXcd;  // one XCD's share of the grid takes part
+        const int waves = thin ? dev::kThinWaves : ctx->sweep_waves;
+        return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(64 * waves), args, dev::stage_bytes(waves), ctx->stream, ev0,
+                                             ev1, 0), what);
     };
     SweepTurn turn(ctx->device, ctx->stream);
     if (turn.error()) return sweep_turn_failed(ctx, turn.error());
     {
         SweepTimes t(ctx, split);
-        const void* fwd = (const void*)dev::k_sweep<true, LPC, R>;
+        const void* fwd = local  ? (const void*)dev::k_sweep_xcd<true, MAXD, R>
+                          : flat ? (const void*)dev::k_sweep<true, MAXD, R, dev::kAnyChunks>
+                                 : (const void*)dev::k_sweep_tiles<true, MAXD, R>;
         if (split) {
-            if (!launch(fwd, grid, 0, ctx->tail_u, "k_sweep<fwd>", t.start(0), t.stop(0))) return false;
-            if (at_tail && after && !after()) return false;
-            if (!launch(fwd, tgrid, ctx->tail_u, A.nchunks, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
+            if (!launch((const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>, false, grid, 0, wf, "k_sweep<fwd>",
+                        t.start(0), t.stop(0)))
                 return false;
-        } else if (!launch(fwd, grid, 0, A.nchunks, "k_sweep<fwd>", t.start(0), t.stop(0))) {
+            if (at_tail && after && !after()) return false;
+            if (!launch((const void*)dev::k_sweep_xcd<true, MAXD, R>, true, tgrid, wf, nf, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
+                return false;
+        } else if (!launch(fwd, local, local ? lgrid : grid, 0, nf, "k_sweep<fwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("fwd_sweep", "fwd_sweep_wide", "fwd_sweep_tail");
@@ -754,12 +777,16 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     if ((!at_tail || !split) && after && !after()) return false;
     {
         SweepTimes t(ctx, split);
-        const void* bwd = (const void*)dev::k_sweep<false, LPC, R>;
+        const void* bwd = local  ? (const void*)dev::k_sweep_xcd<false, MAXD, R>
+                          : flat ? (const void*)dev::k_sweep<false, MAXD, R, dev::kAnyChunks>
+                                 : (const void*)dev::k_sweep_tiles<false, MAXD, R>;
         if (split) {
-            if (!launch(bwd, tgrid, 0, nt, "k_sweep<bwd> (thin tail)", t.start(0), t.stop(0)) ||
-                !launch(bwd, grid, nt, A.nchunks, "k_sweep<bwd>", t.start(1), t.stop(1)))
+            if (!launch((const void*)dev::k_sweep_xcd<false, MAXD, R>, true, tgrid, 0, tb,
+                        "k_sweep<bwd> (thin tail)", t.start(0), t.stop(0)) ||
+                !launch((const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>, false, grid, tb, nb, "k_sweep<bwd>",
+                        t.start(1), t.stop(1)))
                 return false;
-        } else if (!launch(bwd, grid, 0, A.nchunks, "k_sweep<bwd>", t.start(0), t.stop(0))) {
+        } else if (!launch(bwd, local, local ? lgrid : grid, 0, nb, "k_sweep<bwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("bwd_sweep", "bwd_sweep_tail", "bwd_sweep_wide");
@@ -770,10 +797,10 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
 }
 bool launch_sweeps(mfs_ctx* ctx, const std::function<bool()>& after = nullptr, bool at_tail = false) {
     if (ctx->precision == MFS_MIXED)
-        return ctx->lpc == 4 ? launch_sweeps_t<4, float>(ctx, after, at_tail)
-                             : launch_sweeps_t<8, float>(ctx, after, at_tail);
-    return ctx->lpc == 4 ? launch_sweeps_t<4, double>(ctx, after, at_tail)
-                         : launch_sweeps_t<8, double>(ctx, after, at_tail);
+        return ctx->maxf == 4 ? launch_sweeps_t<4, float>(ctx, after, at_tail)
+                              : launch_sweeps_t<6, float>(ctx, after, at_tail);
+    return ctx->maxf == 4 ? launch_sweeps_t<4, double>(ctx, after, at_tail)
+                          : launch_sweeps_t<6, double>(ctx, after, at_tail);
 }
 
 // CalculateGradient: node values, then the gradient.  With `next` set (the
@@ -924,13 +951,21 @@ void free_all(mfs_ctx* ctx) {
         }
 }
 
-template <int LPC, typename R>
+// Workgroups per CU that every sweep kernel of the context allows.
+template <int MAXD, typename R>
 int sweep_occupancy(int* per_cu, int block) {
-    int a = 0, b = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, dev::k_sweep<true, LPC, R>, block, 0) != hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&b, dev::k_sweep<false, LPC, R>, block, 0) != hipSuccess)
-        return -1;
-    *per_cu = std::min(a, b);
+    const void* fn[] = {(const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>,
+                        (const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>,
+                        (const void*)dev::k_sweep<true, MAXD, R, dev::kAnyChunks>,
+                        (const void*)dev::k_sweep<false, MAXD, R, dev::kAnyChunks>,
+                        (const void*)dev::k_sweep_tiles<true, MAXD, R>,
+                        (const void*)dev::k_sweep_tiles<false, MAXD, R>};
+    *per_cu = 1 << 20;
+    for (const void* f : fn) {
+        int n = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, block, dev::stage_bytes(block / 64)) != hipSuccess) return -1;
+        *per_cu = std::min(*per_cu, n);
+    }
     return 0;
 }
 
@@ -1016,16 +1051,15 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     ctx->K.phiq = 1. / 0.5;
     ctx->K.betq = 1.0 + ctx->K.alpq * ctx->K.phiq;
     ctx->nlev = L.nlev;
-    ctx->nchunk = (int)(L.chunk.size() / 2);
-    // the sweeps' thin tail: the thin levels that end the flat order (a
-    // level's chunks are contiguous there and share the flag)
-    ctx->tail_u = ctx->nchunk;
-    while (ctx->tail_u > 0 && (L.crun[4 * (size_t)(ctx->tail_u - 1) + 1] & kThinChunkFlag)) --ctx->tail_u;
-    if (ctx->tail_u == 0 || ctx->nchunk - ctx->tail_u < dev::kMinTailChunks) ctx->tail_u = ctx->nchunk;
-    ctx->tail_cells = 0;
-    for (int u = ctx->tail_u; u < ctx->nchunk; ++u) ctx->tail_cells += L.crun[4 * (size_t)u + 1] & 0xff;
-    ctx->tail_grid = (tail_grid > 0 && !sweep_by_tiles && ctx->tail_u < ctx->nchunk) ? tail_grid : 0;
-    ctx->ntiles = (int)L.tile_chunk.size() - 1;
+    for (int d = 0; d < 2; ++d) {
+        ctx->sweep[d].nchunk = L.sweep[d].nchunk;
+        ctx->sweep[d].tail = L.sweep[d].tail;
+    }
+    ctx->all_thin = L.all_thin;
+    ctx->tail_chunks = L.tail_chunks;
+    ctx->tail_cells = L.tail_cells;
+    ctx->tail_grid = (tail_grid > 0 && !sweep_by_tiles && ctx->tail_chunks > 0) ? tail_grid : 0;
+    ctx->ntiles = (int)L.sweep[0].tile_chunk.size() - 1;
     ctx->lpc = L.lpc;
     ctx->nblk_cell = (int)nblk_xcd(L.nC);
     ctx->node_of_dev.assign(L.node_of_dev.begin(), L.node_of_dev.end());
@@ -1082,12 +1116,21 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     ctx->nsym = (int)L.sym_node.size();
     ok = ok && dalloc(ctx, ctx->sym_node, L.sym_node.size(), "sym_node") &&
          dalloc(ctx, ctx->sym_n, L.sym_n.size(), "sym_n");
-    ok = ok && dalloc(ctx, ctx->crun, (size_t)ctx->nchunk, "chunk records") &&
-         dalloc(ctx, ctx->pos, (size_t)ctx->nchunk, "chunk positions") &&
-         dalloc(ctx, ctx->tile_chunk, L.tile_chunk.size(), "tile_chunk") &&
+    const bool mixed = precision == MFS_MIXED;
+    for (int d = 0; d < 2; ++d) {
+        mfs_ctx::Sweep& S = ctx->sweep[d];
+        const SweepLayout& H = L.sweep[d];
+        const size_t nd = H.ndep + 1;  // a last chunk without dependencies points one past them
+        ok = ok && dalloc(ctx, S.crec, (size_t)S.nchunk, "chunk records") &&
+             dalloc(ctx, S.pos, H.pos.size(), "chunk positions") &&
+             dalloc(ctx, S.tile_chunk, H.tile_chunk.size(), "tile_chunk") &&
+             dalloc(ctx, S.dnb, nd, "dependency neighbours") &&
+             (mixed ? dalloc(ctx, S.dgeo32, nd, "dependency geometry (FP32)")
+                    : dalloc(ctx, S.dgeo, nd, "dependency geometry"));
+    }
+    ok = ok && dalloc(ctx, ctx->cdep, L.cdep.size(), "cell dependencies") &&
          dalloc(ctx, ctx->snb, L.cfs.size(), "slot neighbours") &&
          dalloc(ctx, ctx->sgeo, L.cfs.size(), "slot geometry") && dalloc(ctx, ctx->depmask, L.nC, "depmask");
-    const bool mixed = precision == MFS_MIXED;
     if (mixed) {
         ok = ok && dalloc(ctx, ctx->q32, 5 * n, "q32") && dalloc(ctx, ctx->diag32, L.nC, "diag32") &&
              dalloc(ctx, ctx->dqf32, 5 * (size_t)L.nC, "dq_forward32") && dalloc(ctx, ctx->dq32, 5 * n, "dq32") &&
@@ -1111,9 +1154,9 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
         int per_cu = 0, cus = 0;
         const bool mixed = ctx->precision == MFS_MIXED;
         const int blk = 64 * ctx->sweep_waves;
-        const int occ = ctx->lpc == 4
+        const int occ = ctx->maxf == 4
                             ? (mixed ? sweep_occupancy<4, float>(&per_cu, blk) : sweep_occupancy<4, double>(&per_cu, blk))
-                            : (mixed ? sweep_occupancy<8, float>(&per_cu, blk) : sweep_occupancy<8, double>(&per_cu, blk));
+                            : (mixed ? sweep_occupancy<6, float>(&per_cu, blk) : sweep_occupancy<6, double>(&per_cu, blk));
         ok = occ == 0 &&
              hip_ok(ctx, hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx->device), "CU count");
         if (!ok) set_error("mfs_ctx_create: occupancy query failed");
@@ -1147,11 +1190,17 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
              upload(ctx, ctx->nden, L.nden.data(), L.nN, "upload nden") &&
              upload(ctx, ctx->sym_node, L.sym_node.data(), L.sym_node.size(), "upload sym") &&
              upload(ctx, ctx->sym_n, L.sym_n.data(), L.sym_n.size(), "upload sym_n") &&
-             upload(ctx, ctx->crun, reinterpret_cast<const int4*>(L.crun.data()), (size_t)ctx->nchunk, "upload crun") &&
-             upload(ctx, ctx->pos, L.pos.data(), L.pos.size(), "upload pos") &&
-             upload(ctx, ctx->tile_chunk, L.tile_chunk.data(), L.tile_chunk.size(), "upload tile_chunk") &&
              upload(ctx, ctx->depmask, L.depmask.data(), L.nC, "upload depmask") &&
-             upload(ctx, ctx->gface, gf.data(), (size_t)L.nB, "upload gface");
+             upload(ctx, ctx->gface, gf.data(), (size_t)L.nB, "upload gface") &&
+             upload(ctx, ctx->cdep, L.cdep.data(), L.cdep.size(), "upload cell dependencies");
+        for (int d = 0; d < 2; ++d) {
+            const mfs_ctx::Sweep& S = ctx->sweep[d];
+            const SweepLayout& H = L.sweep[d];
+            ok = ok &&
+                 upload(ctx, S.crec, reinterpret_cast<const int4*>(H.crec.data()), (size_t)S.nchunk, "upload chunks") &&
+                 upload(ctx, S.pos, H.pos.data(), H.pos.size(), "upload pos") &&
+                 upload(ctx, S.tile_chunk, H.tile_chunk.data(), H.tile_chunk.size(), "upload tile_chunk");
+        }
         // the slot tables, built on the device from the slot face ids
         int* dcfs = nullptr;
         ok = ok && hip_ok(ctx, hipMalloc((void**)&dcfs, L.cfs.size() * sizeof(int)), "hipMalloc(slot faces)");
@@ -1163,8 +1212,16 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                 hipLaunchKernelGGL(kern, dim3(gC), dim3(kBlock), 0, ctx->stream, L.nC, dcfs, ctx->cfo, ctx->fcell,
                                    ctx->fgeo, ctx->fdn, ctx->fno, ctx->fn, ctx->snb, ctx->sgeo,
                                    mixed ? ctx->sgeo32 : nullptr, ctx->sdn, ctx->sflip, ctx->snode);
-                ok = check_launch(ctx, "k_slot_tables") &&
-                     hip_ok(ctx, hipStreamSynchronize(ctx->stream), "slot tables");
+                ok = check_launch(ctx, "k_slot_tables");
+                auto dep = L.lpc == 4 ? dev::k_dep_tables<4> : dev::k_dep_tables<8>;
+                for (int d = 0; d < 2 && ok; ++d) {
+                    const mfs_ctx::Sweep& S = ctx->sweep[d];
+                    hipLaunchKernelGGL(dep, dim3(nblk((size_t)S.nchunk, kBlock / 64)), dim3(kBlock), 0, ctx->stream,
+                                       S.nchunk, S.crec, ctx->cdep, d, ctx->depmask, ctx->snb, ctx->sgeo, S.dnb,
+                                       S.dgeo, S.dgeo32);
+                    ok = check_launch(ctx, "k_dep_tables");
+                }
+                ok = ok && hip_ok(ctx, hipStreamSynchronize(ctx->stream), "slot tables");
             }
             (void)hipFree(dcfs);
         }
@@ -1657,12 +1714,12 @@ extern "C" int mfs_ctx_get_info(mfs_ctx* ctx, mfs_ctx_info* info) {
     info->tile_cells = ctx->tile_cells;
     info->sweep_waves = ctx->sweep_waves;
     info->sweep_tiles = ctx->ntiles;
-    info->sweep_workgroups = ctx->sweep_by_tiles ? std::min(ctx->sweep_grid, ctx->ntiles)
-                                                 : std::min(ctx->sweep_grid, (ctx->nchunk + ctx->sweep_waves - 1) /
-                                                                                 ctx->sweep_waves);
+    const int chunks = std::max(ctx->sweep[0].nchunk, ctx->sweep[1].nchunk);
+    info->sweep_workgroups =
+        std::min(ctx->sweep_grid, ctx->sweep_by_tiles ? ctx->ntiles : (chunks + ctx->sweep_waves - 1) / ctx->sweep_waves);
     info->sweep_by_tiles = ctx->sweep_by_tiles;
     info->compute_units = ctx->compute_units;
-    info->sweep_tail_chunks = ctx->tail_grid > 0 ? ctx->nchunk - ctx->tail_u : 0;
+    info->sweep_tail_chunks = ctx->tail_grid > 0 ? ctx->tail_chunks : 0;
     info->sweep_tail_cells = ctx->tail_grid > 0 ? ctx->tail_cells : 0;
     info->sweep_tail_workgroups = ctx->tail_grid > 0 ? tail_workgroups(ctx) : 0;
     return MFS_OK;
@@ -1703,7 +1760,8 @@ struct mfs_batch {
     bool dirty = true;            // block maps and sweep items need a rebuild
     // device-side maps for the current set of solves (position = index in `active`)
     std::vector<int> active;      // slot of each position
-    int ncell_blk = 0, nnode_blk = 0, nitems = 0;
+    int ncell_blk = 0, nnode_blk = 0;
+    int nitems[2] = {0, 0};       // chunks of the forward and the backward sweep
     int* cell_solve = nullptr;
     int* node_solve = nullptr;
     int2* items_f = nullptr;
@@ -1766,19 +1824,22 @@ bool batch_rebuild_maps(mfs_batch* b) {
     // last in the forward sweep and first in the backward sweep, so the
     // forward list aligns the solves at their last chunk (solve a starts at
     // step maxch - nchunk_a) and the backward list at their first.
-    int maxch = 0;
-    for (size_t a = 0; a < b->active.size(); ++a) maxch = std::max(maxch, b->slots[b->active[a]]->nchunk);
-    for (int k = 0; k < maxch; ++k)
-        for (size_t a = 0; a < b->active.size(); ++a) {
-            const int nch = b->slots[b->active[a]]->nchunk;
-            if (k < nch) itb.push_back(make_int2((int)a, k));
-            if (k >= maxch - nch) itf.push_back(make_int2((int)a, k - (maxch - nch)));
-        }
+    for (int dir = 0; dir < 2; ++dir) {
+        int maxch = 0;
+        for (int a : b->active) maxch = std::max(maxch, b->slots[a]->sweep[dir].nchunk);
+        for (int k = 0; k < maxch; ++k)
+            for (size_t a = 0; a < b->active.size(); ++a) {
+                const int nch = b->slots[b->active[a]]->sweep[dir].nchunk;
+                const int u = dir == 0 ? k - (maxch - nch) : k;
+                if (u >= 0 && u < nch) (dir == 0 ? itf : itb).push_back(make_int2((int)a, u));
+            }
+    }
     b->ncell_blk = (int)cs.size();
     b->nnode_blk = (int)ns.size();
-    b->nitems = (int)itf.size();
+    b->nitems[0] = (int)itf.size();
+    b->nitems[1] = (int)itb.size();
     if (!batch_ok(b, hipStreamSynchronize(b->stream), "batch sync")) return false;
-    const size_t need = std::max({cs.size(), ns.size(), itf.size(), (size_t)1});
+    const size_t need = std::max({cs.size(), ns.size(), itf.size(), itb.size(), (size_t)1});
     if (need > b->maps_cap) {
         (void)hipFree(b->cell_solve);
         (void)hipFree(b->node_solve);
@@ -1809,7 +1870,6 @@ bool batch_rebuild_maps(mfs_batch* b) {
 template <typename R>
 void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int blk0_node, int iter_done, int slot) {
     std::memset(&E, 0, sizeof(E));
-    const bool f64 = sizeof(R) == sizeof(double);
     E.nC = c->nC;
     E.nN = c->nN;
     E.n = c->nC + c->nB;
@@ -1849,27 +1909,9 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
     E.fno = c->fno;
     E.fn = c->fn;
     E.btype = c->btype;
-    auto& A = E.sw;
-    A.nC = c->nC;
-    A.nchunks = c->nchunk;
-    A.nq = c->nC + c->nB;
-    A.ntiles = c->ntiles;
-    A.tile_chunk = c->tile_chunk;
-    A.pos = c->pos;
-    A.flat = 1;
-    A.crun = c->crun;
-    A.snb = c->snb;
-    A.q64 = c->q[cur];
-    A.res = c->res;
-    A.qout = c->q[1 - cur];
-    A.depmask = c->depmask;
-    A.cell0 = c->cell0;
-    A.err = c->err;
-    A.tickets = A.tickets_next = nullptr;  // the batch sweeps assign (solve, position) items instead
-    A.ngroups = 0;
-    A.ubeg = 0;
-    A.uend = c->nchunk;
-    A.run_shift = 0;
+    E.snb = c->snb;
+    E.depmask = c->depmask;
+    sweep_args(E.sw, c, cur);  // the batch sweeps assign (solve, position) items instead of tickets
     if constexpr (sizeof(R) == sizeof(double)) {
         E.ell_w = c->ell_w;
         E.qn = c->qn;
@@ -1877,11 +1919,7 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
         E.gx = c->gx;
         E.gy = c->gy;
         E.gz = c->gz;
-        A.sgeo = c->sgeo;
-        A.q = c->q[cur];
-        A.diag = c->diag;
-        A.dqf = c->dqf;
-        A.dqb = c->dq;
+        E.sgeo = c->sgeo;
     } else {
         E.ell_w = c->ell_w32;
         E.qn = c->qn32;
@@ -1889,13 +1927,8 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
         E.gx = c->gx32;
         E.gy = c->gy32;
         E.gz = c->gz32;
-        A.sgeo = c->sgeo32;
-        A.q = c->q32;
-        A.diag = c->diag32;
-        A.dqf = c->dqf32;
-        A.dqb = c->dq32;
+        E.sgeo = c->sgeo32;
     }
-    (void)f64;
 }
 
 // Node values (with the symmetry projection) and the gradient of the
@@ -1926,7 +1959,7 @@ bool batch_gradient(mfs_batch* b, const dev::BatchSolve<R>* T, hipStream_t st) {
     return batch_ok(b, hipGetLastError(), "batch gradient");
 }
 
-template <int MAXF, int LPC, typename R>
+template <int MAXF, typename R>
 int batch_step_t(mfs_batch* b, int nsteps) {
     constexpr bool MIXED = sizeof(R) == sizeof(float);
     const int ns = (int)b->active.size();
@@ -1975,7 +2008,8 @@ int batch_step_t(mfs_batch* b, int nsteps) {
         return MFS_ERR_HIP;
     b->table_pending = true;
     auto* D = static_cast<dev::BatchSolve<R>*>(b->table_dev);
-    const dim3 sweep_grid((unsigned)std::max(1, std::min(b->sweep_grid, (b->nitems + kBatchSweepWaves - 1) /
+    const int most = std::max(b->nitems[0], b->nitems[1]);
+    const dim3 sweep_grid((unsigned)std::max(1, std::min(b->sweep_grid, (most + kBatchSweepWaves - 1) /
                                                                          kBatchSweepWaves)));
     // The gradient feeds nothing in an iteration, so with a second stream it
     // runs beside the next iteration (see step_iterations).
@@ -2013,21 +2047,23 @@ int batch_step_t(mfs_batch* b, int nsteps) {
         {
             SweepTurn turn(b->device, b->stream);
             if (turn.error()) return sweep_turn_failed(nullptr, turn.error()) ? MFS_OK : MFS_ERR_HIP;
-            int n_it = b->nitems;
+            int n_f = b->nitems[0], n_b = b->nitems[1];
             int ng = std::min(kTicketGroups, (int)sweep_grid.x);
             int* tk_f = b->tickets;
             int* tk_b = b->tickets + kTicketGroups * kTicketStride;
-            void* args[] = {(void*)&Tf, (void*)&b->items_f, (void*)&n_it, (void*)&tk_f, (void*)&tk_b, (void*)&ng};
+            void* args[] = {(void*)&Tf, (void*)&b->items_f, (void*)&n_f, (void*)&tk_f, (void*)&tk_b, (void*)&ng};
             if (!batch_ok(b,
-                          hipLaunchKernel((const void*)dev::k_b_sweep<true, LPC, R>, sweep_grid,
-                                                     dim3(64 * kBatchSweepWaves), args, 0, b->stream),
+                          hipLaunchKernel((const void*)dev::k_b_sweep<true, MAXF, R>, sweep_grid,
+                                                     dim3(64 * kBatchSweepWaves), args, dev::stage_bytes(kBatchSweepWaves),
+                                          b->stream),
                           "batch forward sweep"))
                 return MFS_ERR_HIP;
             if (side && mode == 4 && !side_gradient()) return MFS_ERR_HIP;
-            void* argsb[] = {(void*)&Tf, (void*)&b->items_b, (void*)&n_it, (void*)&tk_b, (void*)&tk_f, (void*)&ng};
+            void* argsb[] = {(void*)&Tf, (void*)&b->items_b, (void*)&n_b, (void*)&tk_b, (void*)&tk_f, (void*)&ng};
             if (!batch_ok(b,
-                          hipLaunchKernel((const void*)dev::k_b_sweep<false, LPC, R>, sweep_grid,
-                                                     dim3(64 * kBatchSweepWaves), argsb, 0, b->stream),
+                          hipLaunchKernel((const void*)dev::k_b_sweep<false, MAXF, R>, sweep_grid,
+                                                     dim3(64 * kBatchSweepWaves), argsb, dev::stage_bytes(kBatchSweepWaves),
+                                          b->stream),
                           "batch backward sweep"))
                 return MFS_ERR_HIP;
             if (!turn.done()) return sweep_turn_failed(nullptr, turn.error()) ? MFS_OK : MFS_ERR_HIP;
@@ -2082,12 +2118,14 @@ int batch_step_t(mfs_batch* b, int nsteps) {
     return MFS_OK;
 }
 
-template <int LPC, typename R>
+template <int MAXF, typename R>
 int batch_sweep_occupancy(int* per_cu) {
     int a = 0, c = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, dev::k_b_sweep<true, LPC, R>, 64 * kBatchSweepWaves, 0) !=
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&a, dev::k_b_sweep<true, MAXF, R>, 64 * kBatchSweepWaves,
+                                                     dev::stage_bytes(kBatchSweepWaves)) !=
             hipSuccess ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, dev::k_b_sweep<false, LPC, R>, 64 * kBatchSweepWaves, 0) !=
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&c, dev::k_b_sweep<false, MAXF, R>, 64 * kBatchSweepWaves,
+                                                     dev::stage_bytes(kBatchSweepWaves)) !=
             hipSuccess)
         return -1;
     *per_cu = std::min(a, c);
@@ -2172,10 +2210,10 @@ extern "C" int mfs_batch_attach(mfs_batch* b, mfs_ctx* c, int* slot) {
     if (first) {
         int per_cu = 0, cus = 0;
         const bool mixed = b->precision == MFS_MIXED;
-        const int occ = c->lpc == 4 ? (mixed ? batch_sweep_occupancy<4, float>(&per_cu)
+        const int occ = c->maxf == 4 ? (mixed ? batch_sweep_occupancy<4, float>(&per_cu)
                                              : batch_sweep_occupancy<4, double>(&per_cu))
-                                    : (mixed ? batch_sweep_occupancy<8, float>(&per_cu)
-                                             : batch_sweep_occupancy<8, double>(&per_cu));
+                                    : (mixed ? batch_sweep_occupancy<6, float>(&per_cu)
+                                             : batch_sweep_occupancy<6, double>(&per_cu));
         if (occ != 0 || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, b->device) != hipSuccess) {
             set_error("mfs_batch_attach: occupancy query failed");
             return MFS_ERR_HIP;
@@ -2248,8 +2286,8 @@ extern "C" int mfs_batch_step(mfs_batch* b, int nsteps) {
     }
     if (b->dirty && !batch_rebuild_maps(b)) return MFS_ERR_HIP;
     if (b->precision == MFS_MIXED)
-        return b->lpc == 4 ? batch_step_t<4, 4, float>(b, nsteps) : batch_step_t<6, 8, float>(b, nsteps);
-    return b->lpc == 4 ? batch_step_t<4, 4, double>(b, nsteps) : batch_step_t<6, 8, double>(b, nsteps);
+        return b->lpc == 4 ? batch_step_t<4, float>(b, nsteps) : batch_step_t<6, float>(b, nsteps);
+    return b->lpc == 4 ? batch_step_t<4, double>(b, nsteps) : batch_step_t<6, double>(b, nsteps);
 }
 
 extern "C" int mfs_batch_sync(mfs_batch* b) {

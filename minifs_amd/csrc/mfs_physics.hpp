@@ -112,14 +112,14 @@ MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R g
 template <typename R>
 struct FluxPre {
     R Q[5];          // conservative state of the neighbour
-    R rho, v_n, eig;  // density, normal velocity, lhs_omga * spectral radius
+    R m_n, eig;      // normal velocity * density, lhs_omga * spectral radius
     R peff, gam1;
     R f[5];          // -F(Q) (components 1-4)
 };
 
 template <typename R>
 MFS_HD void flux_lusgs_pre(FluxPre<R>& P, const R q[5], R nx, R ny, R nz, R gam, R p_bar, R lhs_omga) {
-    R rv2, p, c2;
+    R rv2, p, c2, v_n;
     P.gam1 = gam - R(1.);
     P.Q[0] = q[0];
     P.Q[1] = q[0] * q[1];
@@ -129,17 +129,17 @@ MFS_HD void flux_lusgs_pre(FluxPre<R>& P, const R q[5], R nx, R ny, R nz, R gam,
     p = q[4];
     P.Q[4] = p / P.gam1 + rv2;
 
-    P.v_n = q[1] * nx + q[2] * ny + q[3] * nz;
+    v_n = q[1] * nx + q[2] * ny + q[3] * nz;
     c2 = gam * (p + p_bar) / q[0];
-    P.eig = fabs(P.v_n) + sqrt(c2);
+    P.eig = fabs(v_n) + sqrt(c2);
     P.eig *= lhs_omga;
 
     P.peff = gam * p_bar / P.gam1;
-    P.f[1] = -P.Q[1] * P.v_n - p * nx;
-    P.f[2] = -P.Q[2] * P.v_n - p * ny;
-    P.f[3] = -P.Q[3] * P.v_n - p * nz;
-    P.f[4] = -(P.Q[4] + p + P.peff) * P.v_n;
-    P.rho = q[0];
+    P.f[1] = -P.Q[1] * v_n - p * nx;
+    P.f[2] = -P.Q[2] * v_n - p * ny;
+    P.f[3] = -P.Q[3] * v_n - p * nz;
+    P.f[4] = -(P.Q[4] + p + P.peff) * v_n;
+    P.m_n = v_n * q[0];
 }
 
 template <typename R>
@@ -150,8 +150,7 @@ MFS_HD void flux_lusgs_post(const FluxPre<R>& P, const R DQ[5], R nx, R ny, R nz
     p = P.gam1 * (Q[4] - rv2);
 
     flux[0] = DQ[1] * nx + DQ[2] * ny + DQ[3] * nz;
-    v_n = P.v_n * P.rho;
-    v_n += flux[0];
+    v_n = P.m_n + flux[0];
     v_n /= Q[0];
     flux[1] = P.f[1] + (Q[1] * v_n + p * nx);
     flux[2] = P.f[2] + (Q[2] * v_n + p * ny);
@@ -226,22 +225,16 @@ MFS_HD void flux_lusgs_delta(const R q[5], const R DQ[5], R nx, R ny, R nz, R ga
     flux_lusgs_delta_post(P, DQ, nx, ny, nz, flux);
 }
 
-// The three-stage DQ positivity limiter (DQ_limit == 2) of both sweeps
-// (forward_lusgs.cpp:939-973 and 1184-1218).  q is the swept cell's state.
+// The DQ positivity limiter (DQ_limit == 2) of both sweeps
+// (forward_lusgs.cpp:939-973 and 1184-1218) runs three stages: a DQ that
+// takes the swept cell's state q outside the limits is scaled by 0.1, by 0.1
+// again, then set to zero.  This is a stage's test (vv = |u|^2 of q).
 template <typename R>
-MFS_HD void dq_limit(const R q[5], R DQ[5], R gamm1, R rho_min, R rho_max, R p_min, R p_max) {
-    R vv = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
-    for (int stage = 0; stage < 3; ++stage) {
-        R dp = DQ[4] + R(0.5) * DQ[0] * vv - (DQ[1] * q[1] + DQ[2] * q[2] + DQ[3] * q[3]);
-        dp *= gamm1;
-        if ((q[0] + DQ[0]) < rho_min || (q[0] + DQ[0]) > rho_max || (q[4] + dp) < p_min || (q[4] + dp) > p_max) {
-            if (stage < 2) {
-                for (int i = 0; i < 5; ++i) DQ[i] *= R(0.1);
-            } else {
-                for (int i = 0; i < 5; ++i) DQ[i] = R(0.0);
-            }
-        }
-    }
+MFS_HD bool dq_outside(const R q[5], const R DQ[5], R vv, R gamm1, R rho_min, R rho_max, R p_min, R p_max) {
+    R dp = DQ[4] + R(0.5) * DQ[0] * vv - (DQ[1] * q[1] + DQ[2] * q[2] + DQ[3] * q[3]);
+    dp *= gamm1;
+    // no short circuit: four compares cost less than the branches between them
+    return ((q[0] + DQ[0]) < rho_min) | ((q[0] + DQ[0]) > rho_max) | ((q[4] + dp) < p_min) | ((q[4] + dp) > p_max);
 }
 
 // UpdateFlowField3D_CFL3d cell body (forward_lusgs.cpp:1386-1428); q holds

@@ -426,112 +426,161 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         }
     }
 
-    // ---- sweep chunks.  A chunk is up to `cpc` consecutive device cells of
-    // one tile and one forward level, so its cells never depend on one
-    // another.  Chunks are numbered in device order (tile, then level), and
-    // tile k owns chunks tile_chunk[k] .. tile_chunk[k+1]-1.  A lower
-    // neighbour has a smaller mesh id (same or earlier tile) and a lower
-    // level, so every forward dependency lies in an earlier chunk and every
-    // backward dependency in a later one.  rep_f/rep_b name, per chunk, the
-    // dependency expected to be published last: the one with the highest
-    // (forward) or lowest (backward) level, another tile's first.
+    // ---- sweep chunks, per direction (mfs_prep.hpp).  A lower neighbour has
+    // a smaller mesh id (same or earlier tile) and a lower level, so every
+    // forward dependency lies in an earlier level and tile order and every
+    // backward dependency in a later one.
     L.lpc = L.max_faces <= 4 ? 4 : 8;
-    L.cpc = 64 / L.lpc;
     {
-        std::vector<int> chunk_of(nC);
-        L.chunk.clear();
-        L.tile_chunk.clear();
-        int cur_tile = -1;
-        for (int d = 0; d < nC;) {
-            const int c0 = L.cell_of_dev[d];
-            const int l = L.flevel[c0], tile = c0 / kTileCells;
-            while (cur_tile < tile) {
-                L.tile_chunk.push_back((int)(L.chunk.size() / 2));
-                ++cur_tile;
-            }
-            int e = d;
-            while (e < nC && e - d < L.cpc && L.flevel[L.cell_of_dev[e]] == l &&
-                   L.cell_of_dev[e] / kTileCells == tile)
-                ++e;
-            const int t = (int)(L.chunk.size() / 2);
-            for (int x = d; x < e; ++x) chunk_of[x] = t;
-            L.chunk.push_back(d);
-            L.chunk.push_back(e - d);
-            d = e;
+        // (tile, level) groups of consecutive device cells, and the levels'
+        // widths in 64/lpc-cell units
+        const int unit = 64 / L.lpc;
+        std::vector<int> gfirst, glevel, width(L.nlev, 0);
+        for (int d = 0, tile = -1, lev = -1; d < nC; ++d) {
+            const int c = L.cell_of_dev[d];
+            if (c / kTileCells == tile && L.flevel[c] == lev) continue;
+            tile = c / kTileCells;
+            lev = L.flevel[c];
+            gfirst.push_back(d);
+            glevel.push_back(lev);
         }
-        const int nchunk = (int)(L.chunk.size() / 2);
-        L.tile_chunk.push_back(nchunk);
-        // flat schedule: every chunk of level l before any of level l+1,
-        // chunks of one level in chunk order (a stable counting sort)
-        L.run.resize(nchunk);
-        {
-            std::vector<int> at(L.nlev + 1, 0);
-            for (int t = 0; t < nchunk; ++t) at[L.flevel[L.cell_of_dev[L.chunk[2 * t]]] + 1]++;
-            for (int l = 0; l < L.nlev; ++l) at[l + 1] += at[l];
-            for (int t = 0; t < nchunk; ++t) L.run[at[L.flevel[L.cell_of_dev[L.chunk[2 * t]]]]++] = t;
+        const int ng = (int)gfirst.size();
+        gfirst.push_back(nC);
+        for (int g = 0; g < ng; ++g) width[glevel[g]] += (gfirst[g + 1] - gfirst[g] + unit - 1) / unit;
+        std::vector<char> thin(L.nlev);
+        for (int l = 0; l < L.nlev; ++l) thin[l] = width[l] <= kThinLevelChunks;
+        int tail_level = L.nlev;  // first level of the thin tail
+        while (tail_level > 0 && thin[tail_level - 1]) L.tail_chunks += width[--tail_level];
+        L.all_thin = tail_level == 0;
+        if (tail_level == 0 || L.tail_chunks < kMinTailChunks) {
+            tail_level = L.nlev;
+            L.tail_chunks = 0;
         }
-        L.rep_f.assign(nchunk, -1);
-        L.rep_b.assign(nchunk, -1);
-        // rank of a dependency: level first, then "in another tile"; the
-        // first of equal rank in the chunk's cell and slot order
-        std::vector<char> bad(nchunk, 0);
-        parallel_for(nchunk, [&](size_t tt) {
-            const int t = (int)tt;
-            long long bestF = -1, bestB = -1;
-            for (int d = L.chunk[2 * t]; d < L.chunk[2 * t] + L.chunk[2 * t + 1]; ++d) {
-                const int c = L.cell_of_dev[d];
-                for (int k = mcfo[c]; k < mcfo[c + 1]; ++k) {
-                    const int f = mcf[k];
-                    if (f < nB) continue;
-                    const int nb = other(c, f);
-                    const int dn = dcell[nb];
-                    const int tn = chunk_of[dn];
-                    const int foreign = (nb / kTileCells != c / kTileCells) ? 1 : 0;
-                    if (nb < c) {
-                        if (tn >= t) bad[t] = 1;
-                        const long long r = 2LL * L.flevel[nb] + foreign;
-                        if (r > bestF) {
-                            bestF = r;
-                            L.rep_f[t] = dn;
-                        }
-                    } else {
-                        if (tn <= t) bad[t] = 2;
-                        const long long r = 2LL * (L.nlev - L.flevel[nb]) + foreign;
-                        if (r > bestB) {
-                            bestB = r;
-                            L.rep_b[t] = dn;
-                        }
+        L.tail_cells = 0;
+        for (int g = 0; g < ng; ++g)
+            if (glevel[g] >= tail_level) L.tail_cells += gfirst[g + 1] - gfirst[g];
+        L.cdep.resize(2 * (size_t)nC);
+        std::string err[2];
+        auto build = [&](int dir) {
+            SweepLayout& S = L.sweep[dir];
+            auto deps = [&](int d) {
+                const unsigned m = (unsigned)L.depmask[d];
+                return __builtin_popcount(dir == 0 ? (m & 0xffu) : ((m >> 8) & 0xffu));
+            };
+            // chunks in device order: first cell, cells, dependencies, level
+            struct Chunk {
+                int first, cells, deps, level;
+            };
+            std::vector<Chunk> ch;
+            ch.reserve((size_t)nC / 24 + ng);
+            S.tile_chunk.clear();
+            int cur_tile = -1;
+            for (int g = 0; g < ng; ++g) {
+                const int tile = L.cell_of_dev[gfirst[g]] / kTileCells;
+                while (cur_tile < tile) {
+                    S.tile_chunk.push_back((int)ch.size());
+                    ++cur_tile;
+                }
+                const int most = thin[glevel[g]] ? kThinCells : 64;
+                for (int d = gfirst[g]; d < gfirst[g + 1];) {
+                    Chunk k{d, 0, 0, glevel[g]};
+                    while (d < gfirst[g + 1] && k.cells < most) {
+                        const int n = deps(d);
+                        if (k.deps + n > 64) break;
+                        k.deps += n;
+                        ++k.cells;
+                        ++d;
                     }
+                    ch.push_back(k);
                 }
             }
-        });
-        for (int t = 0; t < nchunk; ++t)
-            if (bad[t])
-                return std::string(bad[t] == 1 ? "forward" : "backward") + " sweep chunks are not topological";
+            const int nchunk = (int)ch.size();
+            S.nchunk = nchunk;
+            S.tile_chunk.push_back(nchunk);
+            // flat order: forward by level, then device order (a stable
+            // counting sort); backward exactly from the end
+            std::vector<int> at(L.nlev + 1, 0);
+            for (const Chunk& k : ch) at[k.level + 1]++;
+            for (int l = 0; l < L.nlev; ++l) at[l + 1] += at[l];
+            S.tail = nchunk - at[tail_level];
+            S.pos.resize(nchunk);
+            std::vector<int> chunk_at(nchunk);
+            for (int t = 0; t < nchunk; ++t) {
+                const int u = at[ch[t].level]++;
+                S.pos[t] = dir == 0 ? u : nchunk - 1 - u;
+                chunk_at[S.pos[t]] = t;
+            }
+            S.crec.resize(4 * (size_t)nchunk);
+            size_t nd = 0;
+            for (int u = 0; u < nchunk; ++u) {
+                const Chunk& k = ch[chunk_at[u]];
+                S.crec[4 * (size_t)u] = k.first;
+                S.crec[4 * (size_t)u + 1] = k.cells | (k.deps << 8) | (thin[k.level] ? kThinChunkFlag : 0);
+                S.crec[4 * (size_t)u + 2] = (int)nd;
+                nd += k.deps;
+            }
+            S.ndep = nd;
+            if (nd > 0x7fffffffu - 64) {
+                err[dir] = "mesh too large for the sweep tables";
+                return;
+            }
+            // the tile schedule walks a tile's chunks in the sweep's order
+            if (dir == 1)
+                for (size_t t = 0; t + 1 < S.tile_chunk.size(); ++t)
+                    std::reverse(S.pos.begin() + S.tile_chunk[t], S.pos.begin() + S.tile_chunk[t + 1]);
+            // per cell its place among the chunk's dependencies; per chunk
+            // the dependency of the latest level, another tile's first, the
+            // first of equal rank in the chunk's cell and face order (thin:
+            // that dependency's own latest)
+            parallel_for(nchunk, [&](size_t uu) {
+                const int u = (int)uu;
+                const int d0 = S.crec[4 * uu], cells = S.crec[4 * uu + 1] & 0xff;
+                long long best = -1;
+                int rep = -1, start = 0;
+                // the dependency of cell c that ranks above `best`, if any
+                auto latest = [&](int c, long long& best, int& rep) {
+                    for (int k = mcfo[c]; k < mcfo[c + 1]; ++k) {
+                        const int f = mcf[k];
+                        if (f < nB) continue;
+                        const int nb = other(c, f);
+                        if (dir == 0 ? nb > c : nb < c) continue;
+                        const int foreign = (nb / kTileCells != c / kTileCells) ? 1 : 0;
+                        const int l = L.flevel[nb];
+                        const long long r = 2LL * (dir == 0 ? l : L.nlev - l) + foreign;
+                        if (r > best) {
+                            best = r;
+                            rep = dcell[nb];
+                        }
+                    }
+                };
+                for (int d = d0; d < d0 + cells; ++d) {
+                    const int c = L.cell_of_dev[d];
+                    const int n = deps(d);
+                    L.cdep[2 * (size_t)d + dir] = (unsigned short)(start | (n << 8));
+                    start += n;
+                    latest(c, best, rep);
+                }
+                if (rep >= 0 && (S.crec[4 * uu + 1] & kThinChunkFlag)) {
+                    const int c = L.cell_of_dev[rep];
+                    best = -1;
+                    rep = -1;
+                    latest(c, best, rep);
+                }
+                S.crec[4 * (size_t)u + 3] = rep;
+            });
+        };
+        {
+            std::thread fwd([&] { build(0); });
+            build(1);
+            fwd.join();
+        }
+        for (const std::string& e : err)
+            if (!e.empty()) return e;
         // face slots per device cell (device face ids, ascending mesh face id, -1 = none)
         L.cfs.assign((size_t)nC * L.lpc, -1);
-        for (int d = 0; d < nC; ++d)
-            for (int k = L.cfo[d]; k < L.cfo[d + 1]; ++k) L.cfs[(size_t)d * L.lpc + (k - L.cfo[d])] = L.cf[k];
-        // the sweeps' tables: chunk records by position, slot neighbours and
-        // oriented geometry (the normal is negated where the cell is the
-        // face's second cell, exactly as the sweep would negate it)
-        // A chunk of a thin level (at most kThinLevelChunks chunks) has its
-        // lanes poll their own dependencies at once instead of one lane
-        // polling the latest first: few waves poll there, and the second
-        // round trip is a level's latency.  Flag: bit 8 of the cell count.
-        std::vector<int> lw(L.nlev, 0);
-        for (int t = 0; t < nchunk; ++t) ++lw[L.flevel[L.cell_of_dev[L.chunk[2 * t]]]];
-        L.crun.resize(4 * (size_t)nchunk);
-        L.pos.resize(nchunk);
-        for (int u = 0; u < nchunk; ++u) {
-            const int t = L.run[u];
-            const bool thin = lw[L.flevel[L.cell_of_dev[L.chunk[2 * t]]]] <= kThinLevelChunks;
-            L.pos[t] = u;
-            L.crun[4 * (size_t)u] = L.chunk[2 * t];
-            L.crun[4 * (size_t)u + 1] = L.chunk[2 * t + 1] | (thin ? kThinChunkFlag : 0);
-            L.crun[4 * (size_t)u + 2] = L.rep_f[t];
-            L.crun[4 * (size_t)u + 3] = L.rep_b[t];
-        }
+        parallel_for(nC, [&](size_t d) {
+            for (int k = L.cfo[d]; k < L.cfo[d + 1]; ++k) L.cfs[d * L.lpc + (k - L.cfo[d])] = L.cf[k];
+        });
         // tetrahedral meshes whose slots are all triangles take the
         // gradient's slot-node path (the device builds the slot tables from
         // cfs and the face arrays)

@@ -50,6 +50,29 @@ struct NoFillAlloc : std::allocator<T> {
 template <typename T>
 using lvec = std::vector<T, NoFillAlloc<T>>;
 
+// One direction's sweep schedule.  A chunk is the cells one wave takes at a
+// time: consecutive device cells of one (tile, level) group with at most 64
+// dependencies among them, at most 64 cells (kThinCells on a thin level).
+// A dependency is a face whose neighbour this direction reads: forward the
+// interior neighbours with a smaller mesh id, backward those with a larger
+// one and the ghosts.  The dependencies of a chunk are stored together,
+// cell by cell in the cell's ascending face order, so each lane of the wave
+// takes one; 64/2 cells per wave on average, where one lane per face slot
+// held 16 cells and left half the lanes idle (8 and two thirds on meshes
+// with up to 6 faces per cell).
+struct SweepLayout {
+    int nchunk = 0;
+    size_t ndep = 0;
+    int tail = 0;                       // chunks of the thin tail (forward: the last, backward: the first)
+    // per position of the sweep's order {first device cell, cells |
+    // dependencies << 8 | kThinChunkFlag, first dependency, the dependency
+    // expected to be published last (device cell, -1: none; on a thin level
+    // the one that this dependency itself waits for last)}
+    lvec<int> crec;
+    lvec<int> tile_chunk;               // ntile+1: first entry of each tile in pos
+    lvec<int> pos;                      // positions by tile, in the sweep's level order within the tile
+};
+
 struct HostLayout {
     int nC = 0, nF = 0, nB = 0, nN = 0;
     // cells in device order; cell_of_dev[d] = mesh cell id (ghost k stays at nC+k)
@@ -84,24 +107,19 @@ struct HostLayout {
     lvec<int> sym_node;                 // device nodes with nodesymm == 1
     lvec<double> sym_n;                 // 3 per symmetry node (xfn_n_symm, ...)
     // LU-SGS sweeps: forward DAG level of each mesh cell, the number of
-    // levels, and the chunks (device cell ranges of one level, `cpc` cells,
-    // `lpc` lanes per cell) with their latest dependencies
+    // levels, and each direction's chunks
     lvec<int> flevel;                   // nC, by mesh id
     int nlev = 0;
-    int lpc = 4, cpc = 16;
-    lvec<int> chunk;                    // 2 per chunk (device order): first device cell, cell count
-    lvec<int> tile_chunk;               // ntile+1: first chunk of each storage tile
-    lvec<int> run;                      // chunks by forward level (then tile): the flat schedule
-    lvec<int> rep_f, rep_b;             // per chunk: dependency expected to be published last (-1: none)
+    int lpc = 4;                        // slots per cell of the slot tables (4 for tetrahedra, otherwise 8)
     lvec<int> cfs;                      // lpc slots per device cell: device face id or -1
-    // what the sweeps read, laid out so that a chunk needs no chain of
-    // lookups: per position u of `run`, {first device cell, cell count
-    // (| kThinChunkFlag on a thin level), rep_f, rep_b} of chunk run[u]; per
-    // chunk, its position.  The per-slot tables (neighbour, oriented normal
-    // and area, side distance, sides, tetrahedra's face nodes) are built on
-    // the device from cfs and the face arrays (k_slot_tables).
-    lvec<int> crun;                     // 4 per position
-    lvec<int> pos;                      // per chunk
+    SweepLayout sweep[2];               // forward, backward
+    // per device cell, forward then backward: its first dependency within its
+    // chunk's (bits 0-7) and its dependency count (bits 8-15)
+    lvec<unsigned short> cdep;          // 2*nC
+    // the thin tail of the sweep order: the run of thin levels that ends it,
+    // counted in the level-width unit below, and its cells
+    int tail_chunks = 0, tail_cells = 0;
+    bool all_thin = false;              // every level is thin
     bool tri_slots = false;                    // tetrahedra with triangular slots only
     // initial state, 5 blocks of nC+nB, device cell order
     lvec<double> q;
@@ -109,10 +127,14 @@ struct HostLayout {
 
 // Cells per storage tile of the device order (the sweeps' workgroup unit).
 constexpr int kDefaultTileCells = 4096;
-// Sweep levels of at most this many chunks are thin: their chunks are
-// flagged in the count word of their record (crun[4u+1] bit 8).
+// Thin levels.  A level's width is counted in groups of 64/lpc cells per
+// tile; levels of at most kThinLevelChunks groups are thin.  A thin chunk
+// holds at most kThinCells cells, so that each of its 5-value results has a
+// lane of its own.
 constexpr int kThinLevelChunks = 64;
-constexpr int kThinChunkFlag = 0x100;
+constexpr int kThinCells = 12;
+constexpr int kMinTailChunks = 256;  // shorter tails stay with the wide levels
+constexpr int kThinChunkFlag = 0x10000;
 
 // Returns "" on success.
 std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int tile_cells = kDefaultTileCells);

@@ -368,3 +368,31 @@ __global__ __launch_bounds__(kBlock) void k_slot_tables(int nC, const int* __res
     }
     sflip[d] = flips;
 }
+
+// One direction's dependency tables of the sweeps (SweepLayout): the
+// neighbour and the oriented geometry of every dependency, chunk by chunk,
+// from the slot tables.  One wave per chunk, one lane per cell; mask_shift
+// selects the direction's slots in depmask (0 forward, 8 backward).
+template <int LPC>
+__global__ __launch_bounds__(kBlock) void k_dep_tables(int nchunk, const int4* __restrict__ crec,
+                                                      const unsigned short* __restrict__ cdep, int dir,
+                                                      const int* __restrict__ depmask, const int* __restrict__ snb,
+                                                      const double4* __restrict__ sgeo, int* __restrict__ dnb,
+                                                      double4* __restrict__ dgeo, float4* __restrict__ dgeo32) {
+    const int u = (int)(blockIdx.x * (kBlock / 64) + threadIdx.x / 64), lane = (int)threadIdx.x & 63;
+    if (u >= nchunk) return;
+    const int4 rec = crec[u];
+    if (lane >= (rec.y & 0xff)) return;
+    const int c = rec.x + lane;
+    const unsigned m = ((unsigned)depmask[c] >> (8 * dir)) & 0xffu;
+    size_t k = (size_t)rec.z + (cdep[2 * (size_t)c + dir] & 0xffu);
+    for (int s = 0; s < LPC; ++s) {
+        if (!((m >> s) & 1u)) continue;
+        const size_t i = (size_t)c * LPC + s;
+        const double4 g = sgeo[i];
+        dnb[k] = snb[i];
+        if (dgeo) dgeo[k] = g;
+        if (dgeo32) dgeo32[k] = make_float4((float)g.x, (float)g.y, (float)g.z, (float)g.w);
+        ++k;
+    }
+}

@@ -6,13 +6,22 @@
 // neighbours and the backward sweep that of its higher-numbered neighbours
 // and of its ghost cells (DQ = 0).
 //
-// Work decomposition: a wave handles one chunk of 64/LPC cells of the same
-// forward DAG level (contiguous in device order), LPC lanes per cell, one
-// lane per face slot.  Each lane evaluates FluxLUSGS3D for its own face;
-// the lanes of a cell then exchange the products and every lane of the cell
-// adds them in the cell's face order, so the sum is formed exactly as in
-// the serial sweep.  The limiter and the update run redundantly on the
-// lanes of a cell; each lane stores a share of the 5 results.
+// Work decomposition: a wave handles one chunk of cells of the same forward
+// DAG level (contiguous in device order) with at most 64 dependencies, one
+// lane per dependency: a face whose neighbour this sweep reads.  Each lane
+// evaluates FluxLUSGS3D for its own face and leaves the product in LDS; then
+// each cell has one lane, which adds its cell's products in the cell's face
+// order, exactly as the serial sweep forms the sum, and runs the limiter and
+// the update.  A cell has two dependencies per sweep on average, so a chunk
+// holds about 30 cells.
+// Bound: the wide levels by the latency of a chunk's rounds of loads and by
+// the memory system's gathers, so what counts is cells per round.  With one
+// lane per face slot (16 cells per wave, 8 on meshes with up to 6 faces per
+// cell) half the lanes had no dependency and every cell's lanes ran the
+// limiter and the update.  Wide-level launches, forward / backward, before
+// and after: 6.0M tetrahedra FP64 808 / 938 -> 690 / 770 us, 262k hexahedra
+// FP64 190 / 203 -> 146 / 148 us, a mixed batch of 2.3M cells 603 / 686 ->
+// 433 / 452 us.
 //
 // Schedule: cells are stored by tile (4096 consecutive mesh ids, a compact
 // region in TDTree numbering), then forward level; a chunk is up to 64/LPC
@@ -44,9 +53,10 @@
 // device-coherent loads and retries while any is the sentinel (each store
 // is single-copy atomic, so a non-sentinel value is final).  One lane per
 // wave first waits on the chunk's latest dependency (rep), which keeps the
-// polling traffic to one load per wave; on thin levels (few chunks, few
-// waves polling) every lane polls its own dependency at once, which saves
-// the second round trip on the level's critical path.  The forward sweep re-arms the
+// polling traffic to one load per wave; on thin levels it waits on that
+// dependency's own latest one, so that the wave's lanes are polling when
+// their dependencies come, which saves a round trip on the level's critical
+// path.  The forward sweep re-arms the
 // backward array and the backward sweep the forward one.
 //
 // Precision: R is the type of the implicit operator (state snapshot,
@@ -70,28 +80,31 @@ __device__ __forceinline__ void st_dev(R* p, R v) {
     using B = typename Real<R>::bits;
     __hip_atomic_store(reinterpret_cast<B*>(p), __builtin_bit_cast(B, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-
-// Value of lane S of this lane's group of LPC lanes (a quad for LPC = 4,
-// by DPP; otherwise by a cross-lane permute).  Called with all lanes active.
-template <int LPC, int S>
-__device__ __forceinline__ double cell_bcast(double v) {
-    if constexpr (LPC == 4) {
-        const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-        const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)b, S * 0x55, 0xf, 0xf, false);
-        const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(b >> 32), S * 0x55, 0xf, 0xf, false);
-        return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
-    } else {
-        return __shfl(v, (int)(threadIdx.x & ~(unsigned)(LPC - 1)) + S, 64);
-    }
+// The same for readers on this XCD only: the store stops at the XCD's L2,
+// where the device-scope loads of its other CUs find it.
+template <typename R>
+__device__ __forceinline__ void st_xcd(R* p, R v) {
+    using B = typename Real<R>::bits;
+    __hip_atomic_store(reinterpret_cast<B*>(p), __builtin_bit_cast(B, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-template <int LPC, int S>
-__device__ __forceinline__ float cell_bcast(float v) {
-    if constexpr (LPC == 4) {
-        const int r = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), S * 0x55, 0xf, 0xf, false);
-        return __builtin_bit_cast(float, r);
-    } else {
-        return __shfl(v, (int)(threadIdx.x & ~(unsigned)(LPC - 1)) + S, 64);
-    }
+__device__ __forceinline__ int xcd_id() {  // HW_REG_XCC_ID, bits 0-3
+    return (int)__builtin_amdgcn_s_getreg(20 | (0 << 6) | ((4 - 1) << 11));
+}
+
+// The next ticket of a counter, taken by lane 0 (0 in the others).  The
+// address is kept in vector registers: for an address that the compiler
+// knows to be uniform it combines the wave's atomics and broadcasts the
+// result at once, which waits for the atomic's round trip.  A wave's loads
+// and atomics return in the order of issue, so a chunk takes its wave's next
+// ticket after its last load of the first rounds: nothing that it waits for
+// then queues behind the atomic except a late dependency.
+__device__ __forceinline__ int take_ticket(int* ctr) {
+    auto p = (__attribute__((address_space(1))) int*)ctr;
+    asm volatile("" : "+v"(p));
+    int t = 0;
+    if ((threadIdx.x & 63) == 0) t = __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return t;
 }
 
 // 5-value records read with 128-bit buffer loads: 3 loads for a 40-byte
@@ -129,9 +142,10 @@ __device__ __forceinline__ void ld5w(const T* base, int nrec, int i, T (&v)[5]) 
         for (int j = 0; j < 5; ++j) v[j] = __builtin_bit_cast(T, w[j]);
     }
 }
-// Record i of `base` (nrec records) as published by another wave, read
-// once.  The wide path is not an atomic: single reads only, never in a
-// wait loop (the compiler could keep its value across the loop's turns).
+// Record i of `base` (nrec records) as published by another wave.  Each of
+// its values is read whole (8 or 4 aligned bytes), so a value other than the
+// sentinel is final.  The wide path is not an atomic to the compiler: a wait
+// loop puts a memory barrier for the compiler between its turns.
 template <typename T>
 __device__ __forceinline__ void read_published(bool wide, const T* base, int nrec, int i, T (&v)[5]) {
     if (wide) {
@@ -149,17 +163,24 @@ __device__ __forceinline__ bool wait_failed(int* err, unsigned spins) {
     return __shfl(__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), 0, 64) != 0;
 }
 
+// One direction's schedule and tables (SweepLayout in mfs_prep.hpp).
+template <typename R>
+struct SweepDir {
+    int nchunks;
+    const int4* crec;                       // per position: first cell, cells | deps << 8 | flag, first dep, rep
+    const int* dnb;                         // per dependency: the neighbour
+    const typename Real<R>::vec4* dgeo;     // per dependency: normal away from the cell + area
+    const int* tile_chunk;                  // tiles schedule: first entry of each tile in pos
+    const int* pos;                         // tiles schedule: positions, tile by tile
+};
+
 template <typename R>
 struct SweepArgs {
-    int nC, nchunks;
+    int nC;
     int nq;                                 // records of the state arrays: interior and ghost cells
     int ntiles;
-    const int* tile_chunk;                  // ntiles+1: first chunk of each tile (device order)
-    const int* pos;                         // per chunk: its position in the flat order
-    int flat;                               // 1: flat schedule, 0: tiles
-    const int4* crun;                       // per position: first device cell, cell count, rep fwd, rep bwd
-    const int* snb;                         // LPC per device cell: neighbour across the slot's face
-    const typename Real<R>::vec4* sgeo;     // LPC per device cell: normal away from the cell + area
+    SweepDir<R> dir[2];                     // forward, backward
+    const unsigned short* cdep;             // per cell and direction: first dependency in the chunk, count
     const R* q;                             // operator state (cell-major, 5 per cell)
     const double* q64;                      // FP64 state the backward sweep updates
     const double* res;                      // forward: initial DQ (FP64 residual)
@@ -167,49 +188,19 @@ struct SweepArgs {
     R* dqf;                                 // forward DQ, 5 per cell
     R* dqb;                                 // backward (final) DQ, 5 per cell incl. ghosts (0)
     double* qout;                           // backward: updated state
-    const int* depmask;                     // per cell: forward / backward dependency face slots
     int cell0;                              // cell with mesh id 0 (forward: divide only)
     int* err;
     int* tickets;                           // this sweep's ticket counters (flat schedule)
     int* tickets_next;                      // the other direction's, zeroed here for its next sweep
     int ngroups;                            // ticket groups in use (<= kTicketGroups and <= workgroups)
-    // flat schedule: this launch walks sweep steps [ubeg, uend) of the
-    // sweep's order (step u is position u forward, nchunks-1-u backward);
-    // a sweep split in two launches runs its wide levels and its thin tail
-    // apart, each launch ending when all its steps are done
+    // flat schedule: this launch walks positions [ubeg, uend) of the sweep's
+    // order; a sweep split in two launches runs its wide levels and its thin
+    // tail apart, each launch ending when all its chunks are done
     int ubeg, uend;
-    // flat schedule: the steps go to the ticket groups in runs of
-    // 2^run_shift consecutive steps (run k to group k mod ngroups)
+    // flat schedule: the positions go to the ticket groups in runs of
+    // 2^run_shift consecutive ones (run k to group k mod ngroups)
     int run_shift;
 };
-
-// Adds the LPC per-face products of this lane's cell in slot order (the
-// cell's ascending face order), taking only the slots in `use`.
-template <bool FWD, int LPC, typename R>
-__device__ __forceinline__ void add_cell_terms(const R (&p)[5], unsigned use, R (&D)[5], R (&acc)[5]) {
-#define MFS_ADD_SLOT(S)                                                                      \
-    if constexpr ((S) < LPC) {                                                               \
-        R ps[5];                                                                             \
-        _Pragma("unroll") for (int j = 0; j < 5; ++j) ps[j] = cell_bcast<LPC, (S)>(p[j]);    \
-        if (use & (1u << (S))) {                                                             \
-            _Pragma("unroll") for (int j = 0; j < 5; ++j) {                                  \
-                if (FWD)                                                                     \
-                    D[j] -= ps[j];                                                           \
-                else                                                                         \
-                    acc[j] += ps[j];                                                         \
-            }                                                                                \
-        }                                                                                    \
-    }
-    MFS_ADD_SLOT(0)
-    MFS_ADD_SLOT(1)
-    MFS_ADD_SLOT(2)
-    MFS_ADD_SLOT(3)
-    MFS_ADD_SLOT(4)
-    MFS_ADD_SLOT(5)
-    MFS_ADD_SLOT(6)
-    MFS_ADD_SLOT(7)
-#undef MFS_ADD_SLOT
-}
 
 template <typename R>
 __device__ __forceinline__ void load5r(const R* __restrict__ p, R v[5]) {
@@ -217,14 +208,19 @@ __device__ __forceinline__ void load5r(const R* __restrict__ p, R v[5]) {
     for (int j = 0; j < 5; ++j) v[j] = p[j];
 }
 
-// This wave's staging area for a chunk's records (at most 80 words: 16
-// cells of 5 values), in LDS.  Its lanes write their cells' values, then
-// read back consecutive words; the wave barriers keep the compiler from
-// moving the accesses across each other (a wave's LDS accesses complete in
-// order).
+// This wave's words of LDS: the dependencies' products (5 x 64 values), then
+// the chunk's records (64 cells of 5 values).  A wave's LDS accesses complete
+// in order; lds_order keeps the compiler from moving them across each other.
+// A launch gives every wave of a workgroup kStageWords doubles.
+constexpr int kStageWords = 5 * 64;
+inline size_t stage_bytes(int waves) { return (size_t)waves * kStageWords * sizeof(double); }
 __device__ __forceinline__ double* stage_words() {
-    __shared__ double stage[kSweepBlock / 64][80];
-    return stage[threadIdx.x / 64];
+    extern __shared__ double mfs_stage[];
+    return mfs_stage + (threadIdx.x / 64) * kStageWords;
+}
+__device__ __forceinline__ void lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
 }
 
 // The part of the face term that does not depend on the neighbour's DQ:
@@ -233,47 +229,96 @@ __device__ __forceinline__ double* stage_words() {
 template <typename R>
 using FacePre = std::conditional_t<sizeof(R) == sizeof(double), FluxPre<R>, FluxDeltaPre<R>>;
 
-// The chunk at position u of a sweep's order (the forward sweep walks the
-// positions up, the backward sweep down).  Returns false when a wait
-// expired (the error word is set).
+// v[j] by selects (an array indexed at run time would go to scratch memory).
+template <typename R>
+__device__ __forceinline__ R pick5(R v0, R v1, R v2, R v3, R v4, int j) {
+    const R a = j == 1 ? v1 : v0, b = j == 3 ? v3 : v2;
+    const R x = j < 2 ? a : b;
+    return j == 4 ? v4 : x;
+}
+
+// The limiter's three stages for the wave's cells; `x` is scaled with DQ.  A
+// cell outside the limits is rare, and where the first stage scales no cell
+// of the wave the others see the same values again, so they are left out.
+template <typename R>
+__device__ __forceinline__ void limit_dq(bool skip, const R (&q)[5], R (&DQ)[5], R& x, R gamm1, R rho_min, R rho_max,
+                                         R p_min, R p_max) {
+    const R vv = q[1] * q[1] + q[2] * q[2] + q[3] * q[3];
+#pragma unroll 1
+    for (int stage = 0; stage < 3; ++stage) {
+        const bool bad = !skip & dq_outside(q, DQ, vv, gamm1, rho_min, rho_max, p_min, p_max);
+        if (__builtin_amdgcn_ballot_w64(bad) == 0) return;
+        if (bad) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) DQ[j] = stage < 2 ? DQ[j] * R(0.1) : R(0.0);
+            x = stage < 2 ? x * R(0.1) : R(0.0);
+        }
+    }
+}
+
+// What a launch's chunks are: all treated as wide, all thin (the thin tail),
+// or each by its flag.
+constexpr int kWideChunks = 0, kThinChunks = 1, kAnyChunks = 2;
+
+// A record that no kernel writes, at an index that every lane shares: read
+// through the scalar cache.
+__device__ __forceinline__ int4 load_record(const int4* p, int u) {
+    typedef int v4i __attribute__((ext_vector_type(4)));
+    const v4i r = ((const __attribute__((address_space(4))) v4i*)p)[u];
+    return make_int4(r[0], r[1], r[2], r[3]);
+}
+
+// The chunk at position u (the same in every lane) of a sweep's order.
+// Returns false when a wait expired (the error word is set).
 //
 // Latency: a chunk's operands come in three rounds of loads: its record;
 // then the latest dependency's first value (lane 0, requested first), the
-// cell's mask, slot neighbours and geometry, state, Diag and right-hand
-// side; then the neighbours' states together with their DQ when the latest
-// dependency was already published.  The DQ-independent half of every face
-// term is evaluated before waiting, so only the DQ-dependent half, the
-// sum, the limiter and the stores follow the dependency's arrival.
-template <bool FWD, int LPC, typename R, bool THIN = true>
-__device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowConst& K, int u) {
+// dependencies' neighbours and geometry, the cells' state, Diag and
+// right-hand side; then the neighbours' states together with their DQ when
+// the latest dependency was already published.  The DQ-independent half of
+// every face term is evaluated before waiting, so only the DQ-dependent
+// half, the sum, the limiter and the stores follow the dependency's arrival.
+// With a ticket counter, `next` receives the wave's next ticket.
+//
+// On a thin level the chunk has at most 12 cells and its 5-value
+// results one lane each: lane 5k + j sums, divides and stores value j of
+// cell k, so that one subtraction chain, one division and one store stand
+// where a lane per cell would run five of each on the level's critical path.
+template <bool FWD, int MAXD, typename R, int KIND>
+__device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowConst& K, int u, int* ctr, int& next) {
     using B = typename Real<R>::bits;
     constexpr B kSent = Real<R>::kSent;
+    const SweepDir<R>& S = A.dir[FWD ? 0 : 1];
     const int lane = (int)threadIdx.x & 63;
-    const int k = lane / LPC;  // cell of the chunk
-    const int s = lane % LPC;  // face slot
     R* const poll = FWD ? A.dqf : A.dqb;
-    const int4 rec = A.crun[u];
-    const int rep = FWD ? rec.z : rec.w;
+    const int4 rec = load_record(S.crec, u);
+    const int c0 = rec.x, nc = rec.y & 0xff, nd = (rec.y >> 8) & 0xff, rep = rec.w;
+    // a thin level: every lane polls its own dependency (a batch interleaves
+    // many solves, so no level of one solve is thin there)
+    const bool thin = KIND == kThinChunks || (KIND == kAnyChunks && (rec.y & kThinChunkFlag) != 0);
     B rv = 0;
     if (lane == 0 && rep >= 0) rv = ld_dev<R>(poll + (size_t)rep * 5);
-    const bool active = k < (rec.y & 0xff);
-    // a thin level: every lane polls its own dependency (a batch interleaves
-    // many solves, so no level of one solve is thin there: THIN = false)
-    const bool thin = THIN && (rec.y & 0x100) != 0;
-    const int c = rec.x + (active ? k : 0);  // idle lanes read the first cell and store nothing
-    const unsigned m = (unsigned)A.depmask[c];
-    unsigned kind = FWD ? (m & 0xffu) : ((m >> 8) & 0xffu);  // slots that take part
-    const unsigned pendm = FWD ? kind : ((m >> 16) & 0xffu);  // slots with a DQ to wait for
-    if (FWD && c == A.cell0) kind = 0;  // forward_lusgs.cpp:803-804: the first cell only divides
-    const bool mine = active && ((kind >> s) & 1u);
-    bool pend = mine && ((pendm >> s) & 1u);
-    const size_t sl = (size_t)c * LPC + s;
-    const int nb = A.snb[sl];
-    const typename Real<R>::vec4 g = A.sgeo[sl];
+    // this lane's dependency
+    const bool mine = lane < nd;
+    const size_t kd = (size_t)rec.z + (mine ? lane : 0);
+    const int nb = S.dnb[kd];
+    const typename Real<R>::vec4 g = S.dgeo[kd];
+    bool pend = mine && (FWD || nb < A.nC);  // ghosts have DQ = 0
+    // this lane's cell (thin: and value); lanes past the chunk's cells read
+    // the first cell and store nothing
+    const int k5 = thin ? lane / 5 : lane;
+    const int j5 = lane - 5 * (lane / 5);
+    const bool active = k5 < nc;
+    const int c = c0 + (active ? k5 : 0);
+    const unsigned cd = A.cdep[2 * (size_t)c + (FWD ? 0 : 1)];
+    const int dep0 = (int)(cd & 0xffu), ndep = (int)(cd >> 8);
     R qc[5], D[5];
     load5r(A.q + (size_t)c * 5, qc);
     const R dg = A.diag[c];
-    if (FWD) {
+    if (thin) {
+        const size_t w = (size_t)c * 5 + j5;
+        D[0] = FWD ? (R)A.res[w] : A.dqf[w];
+    } else if (FWD) {
 #pragma unroll
         for (int j = 0; j < 5; ++j) D[j] = (R)A.res[(size_t)c * 5 + j];
     } else {
@@ -290,9 +335,8 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     const bool wide = wide_records(A.nq);  // the same for every wave
     // one read of every pending dependency (they are interior cells); a
     // value still the sentinel leaves the lane pending
-    auto read_deps = [&] {
-        R b[5];
-        read_published(wide, static_cast<const R*>(poll), A.nC, nb, b);
+    R b[5];
+    auto settle = [&] {
         bool ok = true;
 #pragma unroll
         for (int j = 0; j < 5; ++j) ok = ok && (__builtin_bit_cast(B, b[j]) != kSent);
@@ -302,7 +346,11 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
             pend = false;
         }
     };
-    if (rep_seen && pend) read_deps();  // the dependencies are most likely out: read them now
+    // where the latest dependency is out, the others most likely are too:
+    // their reads go out with the neighbours' states
+    const bool early = rep_seen && pend;
+    if (early) read_published(wide, static_cast<const R*>(poll), A.nC, nb, b);
+    if (ctr) next = take_ticket(ctr);
     FacePre<R> pre;
     if (mine) {
         if constexpr (sizeof(R) == sizeof(double))
@@ -311,8 +359,9 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
             flux_lusgs_delta_pre<R>(pre, qnb, g.x, g.y, g.z, (R)K.gam, (R)K.p_bar, (R)K.lhs_omga);
     }
 
+    if (early) settle();
     unsigned spins = 0;
-    if (!rep_seen && !thin) {  // one lane waits for the chunk's latest dependency
+    if (!rep_seen) {  // one lane waits for the chunk's latest dependency (thin: for that one's own)
         while (true) {
             B v = 0;
             if (lane == 0) v = ld_dev<R>(poll + (size_t)rep * 5);
@@ -325,34 +374,22 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
             __builtin_amdgcn_s_sleep(2);
         }
     }
-    // wide levels: the chunk's latest dependency is out, so the others most
-    // likely are too; one read of each before the retry loop
-    if (!thin && pend) read_deps();
-    // every lane reads its face's dependency, retrying the rare unpublished one
+    // every lane reads its face's dependency and retries an unpublished one
     while (__ballot(pend) != 0) {
         if (pend) {
-            B b[5];
-            bool ok = true;
-#pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                b[j] = ld_dev<R>(poll + (size_t)nb * 5 + j);
-                ok = ok && (b[j] != kSent);
-            }
-            if (ok) {
-#pragma unroll
-                for (int j = 0; j < 5; ++j) dv[j] = __builtin_bit_cast(R, b[j]);
-                pend = false;
-            }
+            asm volatile("" ::: "memory");  // the reads of this turn are not those of the last
+            read_published(wide, static_cast<const R*>(poll), A.nC, nb, b);
+            settle();
         }
         if (__ballot(pend) == 0) break;
         if (++spins > kSpinLimit || wait_failed(A.err, spins)) {
             if (lane == 0) atomicExch(A.err, 1);
             return false;
         }
-        __builtin_amdgcn_s_sleep(1);
+        if (KIND != kThinChunks) __builtin_amdgcn_s_sleep(1);
     }
     // this lane's face term: forward 0.5*A*F (DQ -= term), backward A*F (summed)
-    R p[5] = {R(0), R(0), R(0), R(0), R(0)};
+    R* const st = reinterpret_cast<R*>(stage_words());
     if (mine) {
         R fl[5];
         if constexpr (sizeof(R) == sizeof(double))  // the reference's expression, bit for bit
@@ -361,119 +398,201 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
             flux_lusgs_delta_post<R>(pre, dv, g.x, g.y, g.z, fl);
         const R tmp = FWD ? R(0.5) * g.w : g.w;
 #pragma unroll
-        for (int j = 0; j < 5; ++j) p[j] = tmp * fl[j];
+        for (int j = 0; j < 5; ++j) st[j * 64 + lane] = tmp * fl[j];
     }
-    R acc[5] = {R(0), R(0), R(0), R(0), R(0)};
-    add_cell_terms<FWD, LPC, R>(p, kind, D, acc);
-    if (FWD) {
+    lds_order();
+    R* const own = FWD ? A.dqf : A.dqb;    // published
+    R* const other = FWD ? A.dqb : A.dqf;  // re-armed for the next sweep
+    const R sent = __builtin_bit_cast(R, kSent);
+    const int nw = 5 * nc;  // words of the chunk's records
+    const size_t w0 = (size_t)c0 * 5;
+    if (thin) {
+        R t[MAXD];
 #pragma unroll
-        for (int j = 0; j < 5; ++j) D[j] /= dg;
-        if (c != A.cell0)
-            dq_limit<R>(qc, D, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min, (R)K.p_max);
-    } else {
-        const R tmp = R(2.0) * dg;
+        for (int m = 0; m < MAXD; ++m) t[m] = st[j5 * 64 + ((dep0 + m) & 63)];
+        R x = D[0], acc = R(0);
 #pragma unroll
-        for (int j = 0; j < 5; ++j) D[j] -= acc[j] / tmp;
-        dq_limit<R>(qc, D, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min, (R)K.p_max);
-    }
-    // Stores.  The chunk's cells are contiguous, so its 5-value records
-    // form one run of words: lane w stores word w (and w + 64), and every
-    // store instruction writes whole, consecutive words.  Stored value by
-    // value from the cell's lanes, a record's words went out as 8- and
-    // 32-byte pieces of lines: a quarter of the sweeps' write requests were
-    // 32-byte partial writes, and the wide levels are bound by memory
-    // traffic.  On thin levels the values are published straight from the
-    // cell's lanes: there the staging round trip would lengthen the
-    // level's dependent chain.
-    const int nw = 5 * (rec.y & 0xff);  // words of the chunk's records
-    {
-        R* const own = FWD ? A.dqf : A.dqb;    // published
-        R* const other = FWD ? A.dqb : A.dqf;  // re-armed for the next sweep
-        if (thin) {
-            if (active) {
-#pragma unroll
-                for (int j = 0; j < 5; ++j)
-                    if (j % LPC == s) st_dev<R>(own + (size_t)c * 5 + j, D[j]);
+        for (int m = 0; m < MAXD; ++m)
+            if (m < ndep) {
+                if (FWD)
+                    x -= t[m];
+                else
+                    acc += t[m];
             }
+        if (FWD) {
+            x /= dg;
         } else {
-            double* const st = stage_words();
-            if (active) {
-#pragma unroll
-                for (int j = 0; j < 5; ++j)
-                    if (j % LPC == s) st[k * 5 + j] = (double)D[j];  // exact for R = float too
-            }
-            __builtin_amdgcn_wave_barrier();
-            for (int w = lane; w < nw; w += 64) st_dev<R>(own + (size_t)rec.x * 5 + w, (R)st[w]);
-            __builtin_amdgcn_wave_barrier();
+            const R tmp = R(2.0) * dg;
+            x -= acc / tmp;
         }
-        const R sent = __builtin_bit_cast(R, kSent);
-        for (int w = lane; w < nw; w += 64) other[(size_t)rec.x * 5 + w] = sent;
+        lds_order();
+        st[lane] = x;
+        lds_order();
+#pragma unroll
+        for (int j = 0; j < 5; ++j) D[j] = st[5 * (lane / 5) + j];
+        lds_order();
+        limit_dq<R>(FWD && c == A.cell0, qc, D, x, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min, (R)K.p_max);
+        if (lane < nw) {
+            if (KIND == kThinChunks)
+                st_xcd<R>(own + w0 + lane, x);
+            else
+                st_dev<R>(own + w0 + lane, x);
+            other[w0 + lane] = sent;
+        }
+    } else {
+        R acc[5] = {R(0), R(0), R(0), R(0), R(0)};
+#pragma unroll
+        for (int m = 0; m < MAXD; ++m) {
+            R t[5];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) t[j] = st[j * 64 + ((dep0 + m) & 63)];
+            if (m < ndep) {
+#pragma unroll
+                for (int j = 0; j < 5; ++j) {
+                    if (FWD)
+                        D[j] -= t[j];
+                    else
+                        acc[j] += t[j];
+                }
+            }
+        }
+        if (FWD) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) D[j] /= dg;
+        } else {
+            const R tmp = R(2.0) * dg;
+#pragma unroll
+            for (int j = 0; j < 5; ++j) D[j] -= acc[j] / tmp;
+        }
+        R none = R(0);
+        limit_dq<R>(FWD && c == A.cell0, qc, D, none, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min, (R)K.p_max);
+        // Stores.  The chunk's cells are contiguous, so its 5-value records
+        // form one run of words: lane w stores words w, w + 64, ..., and
+        // every store instruction writes whole, consecutive words.  Stored
+        // value by value from the cell's lane, a record's words would go out
+        // as pieces of lines, and the wide levels are bound by memory traffic.
+        lds_order();
+        if (active) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) st[lane * 5 + j] = D[j];
+        }
+        lds_order();
+        for (int w = lane; w < nw; w += 64) st_dev<R>(own + w0 + w, st[w]);
+        for (int w = lane; w < nw; w += 64) other[w0 + w] = sent;
+        lds_order();
     }
     if (!FWD) {
         double qnew[5], dd[5];
-        if constexpr (sizeof(R) == sizeof(double)) {
 #pragma unroll
-            for (int j = 0; j < 5; ++j) qnew[j] = qc[j];
-        } else {
-#pragma unroll
-            for (int j = 0; j < 5; ++j) qnew[j] = q64c[j];
+        for (int j = 0; j < 5; ++j) {
+            if constexpr (sizeof(R) == sizeof(double))
+                qnew[j] = qc[j];
+            else
+                qnew[j] = q64c[j];
+            dd[j] = (double)D[j];
         }
-#pragma unroll
-        for (int j = 0; j < 5; ++j) dd[j] = (double)D[j];
         update_cell(qnew, dd, K);
         if (thin) {
-            if (active) {
-#pragma unroll
-                for (int j = 0; j < 5; ++j)
-                    if (j % LPC == s) A.qout[(size_t)c * 5 + j] = qnew[j];
-            }
+            if (lane < nw) A.qout[w0 + lane] = pick5(qnew[0], qnew[1], qnew[2], qnew[3], qnew[4], j5);
         } else {
-            double* const st = stage_words();
+            double* const sd = stage_words();
             if (active) {
 #pragma unroll
-                for (int j = 0; j < 5; ++j)
-                    if (j % LPC == s) st[k * 5 + j] = qnew[j];
+                for (int j = 0; j < 5; ++j) sd[lane * 5 + j] = qnew[j];
             }
-            __builtin_amdgcn_wave_barrier();
-            for (int w = lane; w < nw; w += 64) A.qout[(size_t)rec.x * 5 + w] = st[w];
-            __builtin_amdgcn_wave_barrier();
+            lds_order();
+            for (int w = lane; w < nw; w += 64) A.qout[w0 + w] = sd[w];
+            lds_order();
         }
     }
     return true;
 }
 
-template <bool FWD, int LPC, typename R>
+// Ticket counters of a launch: one int per group, kTicketStride apart; the
+// ints after the first counter are the words of an XCD-local launch: the
+// XCD it runs on plus one, and the workgroups that joined it.
+constexpr int kElectWord = 1, kJoinWord = 2;
+__device__ __forceinline__ void clear_tickets(int* tickets) {
+    if (blockIdx.x != 0) return;
+    if (threadIdx.x < kTicketGroups) tickets[threadIdx.x * kTicketStride] = 0;
+    if (threadIdx.x >= 64 && threadIdx.x < 66) tickets[kElectWord + (threadIdx.x - 64)] = 0;
+}
+
+// A launch of wide levels, or of a whole sweep, on the resident grid.
+template <bool FWD, int MAXD, typename R, int KIND>
 __global__ __launch_bounds__(kSweepBlock) void k_sweep(SweepArgs<R> A, FlowConst K) {
     // a sweep that follows a failed one in the same stream does not start
     if (__hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+    clear_tickets(A.tickets_next);  // the other set of counters is idle during this launch
+    const int ng = A.ngroups;
+    const int grp = (int)blockIdx.x % ng;
+    int* const ctr = A.tickets + grp * kTicketStride;
+    int tk = __builtin_amdgcn_readfirstlane(take_ticket(ctr));
+    while (true) {
+        const int sh = A.run_shift;
+        const int u = A.ubeg + ((((tk >> sh) * ng + grp) << sh) | (tk & ((1 << sh) - 1)));
+        if (u >= A.uend) return;
+        int next = 0;
+        if (!sweep_chunk<FWD, MAXD, R, KIND>(A, K, u, ctr, next)) return;
+        tk = __builtin_amdgcn_readfirstlane(next);
+    }
+}
+
+// A launch of thin levels on one XCD.  The first workgroup to start elects
+// its XCD, and up to `join` workgroups of that XCD take the chunks from one
+// counter; the others leave at once (the grid is 8 times `join`, and
+// workgroups are dealt to the XCDs in turn).  Whichever XCD it is, the
+// workgroup that elected it runs, and a chunk is only ever held by a running
+// wave, so the launch ends however its workgroups are placed.
+//
+// A level of the tail is one hop from a wave's store to the next wave's poll.
+// Measured between two waves, an 8-byte word takes 0.39 us to another XCD,
+// 0.36 us to this one with a device-scope store, and 0.22 us with a store
+// that stops in this XCD's L2: a device-scope load is served from the L2 of
+// its own XCD as long as no other XCD has written the line.  With the chunk's
+// results one lane each and the next ticket taken behind the first loads, a
+// level of the 6.0M-cell mesh's tail (234 levels, FP64) took 1.88 us before
+// and 1.29 us now (tails alone, forward and backward, 438 / 442 -> 303 / 305
+// us; 262k hexahedra 252 -> 160 us; all 27 levels of a 1,296-cell mesh 53 ->
+// 34 us).  Of it the store and the polls take 0.6 us, the face terms 0.23,
+// the sum, the division and the limiter 0.3.  One wave per SIMD of the XCD is
+// fastest (64 workgroups of 2 waves; 64 of 4: 2% slower iterations, 128 of 4:
+// 7%): more waves only add polls.
+template <bool FWD, int MAXD, typename R>
+__global__ __launch_bounds__(kSweepBlock) void k_sweep_xcd(SweepArgs<R> A, FlowConst K, int join) {
+    __shared__ int in;
+    if (threadIdx.x == 0) {
+        const int me = xcd_id() + 1;
+        int* const elect = A.tickets + kElectWord;
+        const int won = atomicCAS(elect, 0, me);
+        in = (won == 0 || won == me) && atomicAdd(A.tickets + kJoinWord, 1) < join;
+    }
+    clear_tickets(A.tickets_next);
+    __syncthreads();
+    if (!in || __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+    int tk = __builtin_amdgcn_readfirstlane(take_ticket(A.tickets));
+    while (true) {
+        const int u = A.ubeg + tk;
+        if (u >= A.uend) return;
+        int next = 0;
+        if (!sweep_chunk<FWD, MAXD, R, kThinChunks>(A, K, u, A.tickets, next)) return;
+        tk = __builtin_amdgcn_readfirstlane(next);
+    }
+}
+
+// The tile schedule: one workgroup per tile.
+template <bool FWD, int MAXD, typename R>
+__global__ __launch_bounds__(kSweepBlock) void k_sweep_tiles(SweepArgs<R> A, FlowConst K) {
+    if (__hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
+    const SweepDir<R>& S = A.dir[FWD ? 0 : 1];
     const int W = (int)blockDim.x / 64;
     const int w = (int)threadIdx.x / 64;
-    if (A.flat) {
-        // the other direction's counters are idle during this sweep
-        if (blockIdx.x == 0 && threadIdx.x < kTicketGroups) A.tickets_next[threadIdx.x * kTicketStride] = 0;
-        const int ng = A.ngroups;
-        const int grp = (int)blockIdx.x % ng;
-        int* const ctr = A.tickets + grp * kTicketStride;
-        const int lane = (int)threadIdx.x & 63;
-        int tk = 0;
-        if (lane == 0) tk = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        tk = __shfl(tk, 0, 64);
-        while (true) {
-            const int sh = A.run_shift;
-            const int u = A.ubeg + ((((tk >> sh) * ng + grp) << sh) | (tk & ((1 << sh) - 1)));
-            if (u >= A.uend) return;
-            int next = 0;  // taken now, used after this chunk: its latency overlaps the chunk
-            if (lane == 0) next = __hip_atomic_fetch_add(ctr, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (!sweep_chunk<FWD, LPC, R>(A, K, FWD ? u : A.nchunks - 1 - u)) return;
-            tk = __shfl(next, 0, 64);
-        }
-    }
+    int none = 0;
     for (int kk = blockIdx.x; kk < A.ntiles; kk += gridDim.x) {
         const int k = FWD ? kk : A.ntiles - 1 - kk;
-        const int c0 = A.tile_chunk[k], c1 = A.tile_chunk[k + 1];
-        for (int j = w; j < c1 - c0; j += W) {
-            const int t = FWD ? c0 + j : c1 - 1 - j;
-            if (!sweep_chunk<FWD, LPC, R>(A, K, A.pos[t])) return;
-        }
+        const int t0 = S.tile_chunk[k], t1 = S.tile_chunk[k + 1];
+        for (int t = t0 + w; t < t1; t += W)
+            if (!sweep_chunk<FWD, MAXD, R, kAnyChunks>(A, K, __builtin_amdgcn_readfirstlane(S.pos[t]), nullptr, none))
+                return;
     }
 }
