@@ -42,8 +42,9 @@ struct BatchSolve {
     const int *fno, *fn, *btype;
     const typename Real<R>::vec4* fgeo_r;
     R *gx, *gy, *gz;
-    const int* snode;             // tetrahedral meshes: slot nodes (nullptr otherwise)
-    const int *snb, *depmask;     // slot neighbours; boundary slots of the gradient
+    const int4* cnode;            // tetrahedral meshes: the cells' nodes (nullptr otherwise) and choices
+    const unsigned short* gsel;
+    const int* snb;               // slot neighbours
     const typename Real<R>::vec4* sgeo;  // slot geometry (gradient)
     const double4* sgeo64;        // FP64 slot geometry, distances and sides (residual kernel)
     const double* sdn;
@@ -123,8 +124,8 @@ __global__ __launch_bounds__(kBlock) void k_b_grad(const BatchSolve<R>* __restri
     const BatchSolve<R>& S = T[cell_solve[blockIdx.x]];
     const int lb = (int)blockIdx.x - S.blk0_cell;
     const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
-    if (MAXF == 4 && S.snode)
-        grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask,
+    if (MAXF == 4 && S.cnode)
+        grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.cnode, S.gsel,
                          S.qnew, S.qn, S.vol, S.gx, S.gy, S.gz);
     else
         grad_body<MAXF, R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn,
@@ -184,8 +185,8 @@ __global__ __launch_bounds__(kBlock) void k_b_grad_claim(const BatchSolve<R>* __
         const BatchSolve<R>& S = T[cell_solve[gb]];
         const int lb = gb - S.blk0_cell;
         const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
-        if (MAXF == 4 && S.snode)
-            grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask,
+        if (MAXF == 4 && S.cnode)
+            grad_tet_body<R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.snb, S.sgeo, S.cnode, S.gsel,
                              S.qnew, S.qn, S.vol, S.gx, S.gy, S.gz);
         else
             grad_body<MAXF, R>(lg * kBlock + (int)threadIdx.x, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn,
@@ -210,8 +211,8 @@ __global__ __launch_bounds__(kBlock) void k_b_grad_flux_ts(const BatchSolve<R>* 
     const int lb = (int)blockIdx.x - S.blk0_cell;
     const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
     const int c = lg * kBlock + (int)threadIdx.x;
-    if (MAXF == 4 && S.snode)
-        grad_tet_body<R>(c, S.nC, S.n, S.snb, S.sgeo, S.snode, S.depmask, S.qnew, S.qn, S.vol, S.gx, S.gy,
+    if (MAXF == 4 && S.cnode)
+        grad_tet_body<R>(c, S.nC, S.n, S.snb, S.sgeo, S.cnode, S.gsel, S.qnew, S.qn, S.vol, S.gx, S.gy,
                          S.gz);
     else
         grad_body<MAXF, R>(c, S.nC, S.n, S.cfo, S.cf, S.fcell, S.fgeo_r, S.fno, S.fn, S.btype, S.qnew, S.qn, S.vol,

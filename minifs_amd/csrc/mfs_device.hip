@@ -843,7 +843,7 @@ bool launch_gradient_t(mfs_ctx* ctx, bool next = false, double next_cfl = 0.0, h
             if (!check_launch(ctx, "k_node_symm")) return false;
         }
     }
-    if (MAXF == 4 && ctx->snode && next) {
+    if (MAXF == 4 && ctx->cnode && next) {
         Timed t(ctx, "grad_flux_ts", st);
         const typename dev::Real<R>::vec4* sgeo_r;
         if constexpr (F64)
@@ -852,14 +852,14 @@ bool launch_gradient_t(mfs_ctx* ctx, bool next = false, double next_cfl = 0.0, h
             sgeo_r = ctx->sgeo32;
         constexpr bool MIXED = !F64;
         hipLaunchKernelGGL((dev::k_grad_flux_ts<MIXED, R>), dim3(ctx->nblk_cell), dim3(kBlock), 0, st,
-                           ctx->nC, n, ctx->snb, sgeo_r, ctx->snode, ctx->depmask, q, qn, ctx->vol, gx, gy, gz,
+                           ctx->nC, n, ctx->snb, sgeo_r, ctx->cnode, ctx->gsel, q, qn, ctx->vol, gx, gy, gz,
                            ctx->sgeo, ctx->sdn, ctx->sflip, ctx->res, ctx->dt, ctx->diag, ctx->part, ctx->K, next_cfl,
                            0.5 * next_cfl, MIXED ? ctx->q32 : nullptr, MIXED ? ctx->diag32 : nullptr);
         return check_launch(ctx, "k_grad_flux_ts");
     }
     {
         Timed t(ctx, "gradient", st);
-        if (MAXF == 4 && ctx->snode) {
+        if (MAXF == 4 && ctx->cnode) {
             const typename dev::Real<R>::vec4* sgeo;
             if constexpr (F64)
                 sgeo = ctx->sgeo;
@@ -871,11 +871,11 @@ bool launch_gradient_t(mfs_ctx* ctx, bool next = false, double next_cfl = 0.0, h
             const int gg = ((ctx->compute_units + dev::kXcd - 1) / dev::kXcd) * dev::kXcd;
             if (st != ctx->stream && gg > 0 && gg < ctx->nblk_cell)
                 hipLaunchKernelGGL(dev::k_grad_tet_claim<R>, dim3(gg), dim3(kBlock), 0, st, ctx->nblk_cell, ctx->nC,
-                                   n, ctx->snb, sgeo, ctx->snode, ctx->depmask, q, qn, ctx->vol, gx, gy, gz,
+                                   n, ctx->snb, sgeo, ctx->cnode, ctx->gsel, q, qn, ctx->vol, gx, gy, gz,
                                    ctx->tickets + kGradClaimOffset);
             else
                 hipLaunchKernelGGL(dev::k_grad_tet<R>, dim3(ctx->nblk_cell), dim3(kBlock), 0, st, ctx->nC, n,
-                                   ctx->snb, sgeo, ctx->snode, ctx->depmask, q, qn, ctx->vol, gx, gy, gz);
+                                   ctx->snb, sgeo, ctx->cnode, ctx->gsel, q, qn, ctx->vol, gx, gy, gz);
             if (!check_launch(ctx, "k_grad_tet")) return false;
         } else {
             hipLaunchKernelGGL((dev::k_grad<MAXF, R>), dim3(ctx->nblk_cell), dim3(kBlock), 0, st, ctx->nC,
@@ -908,7 +908,7 @@ bool launch_gradient(mfs_ctx* ctx, bool next = false, double next_cfl = 0.0, hip
                           : launch_gradient_t<6, double>(ctx, next, next_cfl, st, qs);
 }
 // whether launch_gradient(ctx, true, ...) also runs the next residual pass
-bool gradient_fuses_next(const mfs_ctx* ctx) { return ctx->maxf == 4 && ctx->snode; }
+bool gradient_fuses_next(const mfs_ctx* ctx) { return ctx->maxf == 4 && ctx->cnode; }
 
 bool usable(mfs_ctx* ctx) {
     if (!ctx) {
@@ -1143,7 +1143,9 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
          dalloc(ctx, ctx->err, 4, "err") &&
          dalloc(ctx, ctx->tickets, kTicketInts, "sweep tickets") &&
          dalloc(ctx, ctx->gface, (size_t)L.nB, "ghost faces");
-    if (L.tri_slots) ok = ok && dalloc(ctx, ctx->snode, 12 * (size_t)L.nC, "slot nodes");
+    if (L.tri_slots)
+        ok = ok && dalloc(ctx, ctx->cnode, (size_t)L.nC, "cell nodes") &&
+             dalloc(ctx, ctx->gsel, (size_t)L.nC, "gradient choices");
     ok = ok && dalloc(ctx, ctx->sdn, L.cfs.size(), "slot distances") && dalloc(ctx, ctx->sflip, L.nC, "slot sides");
     ok = ok && ensure_hist(ctx, 64);
     // per-device set-up: the sweep order's event and the address of the
@@ -1210,8 +1212,8 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                 const unsigned gC = (unsigned)((L.nC + kBlock - 1) / kBlock);
                 auto kern = L.lpc == 4 ? dev::k_slot_tables<4> : dev::k_slot_tables<8>;
                 hipLaunchKernelGGL(kern, dim3(gC), dim3(kBlock), 0, ctx->stream, L.nC, dcfs, ctx->cfo, ctx->fcell,
-                                   ctx->fgeo, ctx->fdn, ctx->fno, ctx->fn, ctx->snb, ctx->sgeo,
-                                   mixed ? ctx->sgeo32 : nullptr, ctx->sdn, ctx->sflip, ctx->snode);
+                                   ctx->fgeo, ctx->fdn, ctx->snb, ctx->sgeo, mixed ? ctx->sgeo32 : nullptr, ctx->sdn,
+                                   ctx->sflip);
                 ok = check_launch(ctx, "k_slot_tables");
                 auto dep = L.lpc == 4 ? dev::k_dep_tables<4> : dev::k_dep_tables<8>;
                 for (int d = 0; d < 2 && ok; ++d) {
@@ -1221,7 +1223,17 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                                        S.dgeo, S.dgeo32);
                     ok = check_launch(ctx, "k_dep_tables");
                 }
+                int bad = 0;  // err[3] is free until the first sweep
+                if (ok && ctx->cnode) {
+                    ok = hip_ok(ctx, hipMemsetAsync(ctx->err, 0, sizeof(int) * 4, ctx->stream), "memset err");
+                    hipLaunchKernelGGL(dev::k_tet_tables, dim3(gC), dim3(kBlock), 0, ctx->stream, L.nC, dcfs, ctx->fn,
+                                       ctx->depmask, ctx->cnode, ctx->gsel, ctx->err + 3);
+                    ok = ok && check_launch(ctx, "k_tet_tables") &&
+                         hip_ok(ctx, hipMemcpyAsync(&bad, ctx->err + 3, sizeof(int), hipMemcpyDeviceToHost, ctx->stream),
+                                "tetrahedra check");
+                }
                 ok = ok && hip_ok(ctx, hipStreamSynchronize(ctx->stream), "slot tables");
+                if (bad) ctx->cnode = nullptr;  // its memory stays with the context
             }
             (void)hipFree(dcfs);
         }
@@ -1898,7 +1910,8 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
     E.q32 = c->q32;
     E.diag32 = c->diag32;
     E.K = c->K;
-    E.snode = c->snode;
+    E.cnode = c->cnode;
+    E.gsel = c->gsel;
     E.sgeo64 = c->sgeo;
     E.sdn = c->sdn;
     E.sflip = c->sflip;
@@ -1910,7 +1923,6 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
     E.fn = c->fn;
     E.btype = c->btype;
     E.snb = c->snb;
-    E.depmask = c->depmask;
     sweep_args(E.sw, c, cur);  // the batch sweeps assign (solve, position) items instead of tickets
     if constexpr (sizeof(R) == sizeof(double)) {
         E.ell_w = c->ell_w;

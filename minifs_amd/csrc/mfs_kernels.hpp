@@ -92,6 +92,11 @@ __device__ __forceinline__ void load5(const double* __restrict__ p, double v[5])
 #pragma unroll
     for (int j = 0; j < 5; ++j) v[j] = p[j];
 }
+template <typename R>
+__device__ __forceinline__ void load5r(const R* __restrict__ p, R v[5]) {
+#pragma unroll
+    for (int j = 0; j < 5; ++j) v[j] = p[j];
+}
 
 __global__ void k_fill(double* p, size_t n, double v) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -953,58 +958,59 @@ __device__ __forceinline__ void grad_body(int c, int nC, int n, const int* __res
     }
 }
 
-// The same gradient for tetrahedral cells, from per-slot tables laid out
-// by cell: the neighbour across each face (snb), the face's unit normal
-// pointing away from the cell with its area (sgeo), the face's three nodes
-// in the face's own order (snode), and in bits 24-27 of depmask the
-// boundary slots that take the cell/ghost average.  A cell reads 4 + 16 +
-// 12 contiguous values and then gathers its node values, instead of
-// walking face list -> face -> nodes.  Subtracting q_f*A*n for a face whose
-// second cell this is equals adding q_f*A*(-n) exactly, so the sums are
-// the same bits as grad_body's.
+// The same gradient for tetrahedral cells, from tables laid out by cell: the
+// unit normals pointing away from the cell with their areas (sgeo), the four
+// nodes (cnode; node s is the one off the face of slot s) and a word of
+// choices (gsel, k_tet_tables).  Subtracting q_f*A*n for a face whose second
+// cell this is equals adding q_f*A*(-n) exactly, so the sums are the same
+// bits as grad_body's.
+//
+// Bound: the gathers.  Each node's 5 values are one scattered 40-byte record,
+// and a wave's load of 64 of them costs the CU's address and tag units a
+// cycle or more per lane, so the cell's four records are gathered once, where
+// gathering three per face took twelve.  A face's sum is (a + b) + c with c
+// the node its face list names last; which node that is, is the face's choice
+// of two bits, taken by selects (a + b commutes; a leading 0 + would only turn
+// a sum of negative zeros positive, which the accumulators do anyway).
+// Measured alone, before and after: 6.0M cells FP64 650 -> 440 us (1.8 GB of
+// compulsory reads and writes, 4.1 TB/s), 2.9M cells FP32 215 -> 134 us.
 template <typename R>
 __device__ __forceinline__ void grad_tet_body(int c, int nC, int n, const int* __restrict__ snb,
                                               const typename Real<R>::vec4* __restrict__ sgeo,
-                                              const int* __restrict__ snode, const int* __restrict__ depmask,
+                                              const int4* __restrict__ cnode, const unsigned short* __restrict__ gsel,
                                               const double* __restrict__ q, const R* __restrict__ qn,
                                               const double* __restrict__ vol, R* __restrict__ gx,
                                               R* __restrict__ gy, R* __restrict__ gz) {
     if (c >= nC) return;
-    const unsigned fca = (unsigned)depmask[c] >> 24;
-    const int4 nb4 = reinterpret_cast<const int4*>(snb)[c];
-    const int nbs[4] = {nb4.x, nb4.y, nb4.z, nb4.w};
+    const int4 nd = cnode[c];
+    const unsigned sel = gsel[c];
     typename Real<R>::vec4 g[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s) g[s] = sgeo[(size_t)c * 4 + s];
-    const int4* sn = reinterpret_cast<const int4*>(snode + (size_t)c * 12);
-    const int4 t0 = sn[0], t1 = sn[1], t2 = sn[2];
-    const int tn[12] = {t0.x, t0.y, t0.z, t0.w, t1.x, t1.y, t1.z, t1.w, t2.x, t2.y, t2.z, t2.w};
+    R v[4][5];
+    load5r(qn + (size_t)nd.x * 5, v[0]);
+    load5r(qn + (size_t)nd.y * 5, v[1]);
+    load5r(qn + (size_t)nd.z * 5, v[2]);
+    load5r(qn + (size_t)nd.w * 5, v[3]);
+    const R vc = (R)vol[c];
     R ax[5] = {R(0), R(0), R(0), R(0), R(0)}, ay[5] = {R(0), R(0), R(0), R(0), R(0)},
       az[5] = {R(0), R(0), R(0), R(0), R(0)};
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
+        constexpr int I[4] = {1, 0, 0, 0}, J[4] = {2, 2, 1, 1}, L[4] = {3, 3, 3, 2};  // the face's nodes
+        const R(&vi)[5] = v[I[s]], (&vj)[5] = v[J[s]], (&vk)[5] = v[L[s]];
+        const unsigned last = (sel >> (2 * s)) & 3u;
         R qs[5];
-        if ((fca >> s) & 1u) {
 #pragma unroll
-            for (int j = 0; j < 5; ++j)
-                qs[j] = R(0.5) * ((R)q[(size_t)c * 5 + j] + (R)q[(size_t)nbs[s] * 5 + j]);
-        } else {
-            R sum[5] = {R(0), R(0), R(0), R(0), R(0)};
-            R v0[5], v1[5], v2[5];
+        for (int j = 0; j < 5; ++j) {
+            const R a = last == 0 ? vj[j] : vi[j], b = last == 2 ? vj[j] : vk[j];
+            const R e = last == 1 ? vj[j] : vi[j], d = last == 2 ? vk[j] : e;
+            qs[j] = ((a + b) + d) / R(3.0);
+        }
+        if ((sel >> (8 + s)) & 1u) {
+            const size_t o = (size_t)snb[(size_t)c * 4 + s] * 5;
 #pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                v0[j] = qn[(size_t)tn[3 * s] * 5 + j];
-                v1[j] = qn[(size_t)tn[3 * s + 1] * 5 + j];
-                v2[j] = qn[(size_t)tn[3 * s + 2] * 5 + j];
-            }
-#pragma unroll
-            for (int j = 0; j < 5; ++j) {
-                sum[j] += v0[j];
-                sum[j] += v1[j];
-                sum[j] += v2[j];
-            }
-#pragma unroll
-            for (int j = 0; j < 5; ++j) qs[j] = sum[j] / R(3.0);
+            for (int j = 0; j < 5; ++j) qs[j] = R(0.5) * ((R)q[(size_t)c * 5 + j] + (R)q[o + j]);
         }
 #pragma unroll
         for (int j = 0; j < 5; ++j) {
@@ -1014,7 +1020,6 @@ __device__ __forceinline__ void grad_tet_body(int c, int nC, int n, const int* _
             az[j] += sa * g[s].z;
         }
     }
-    const R vc = (R)vol[c];
 #pragma unroll
     for (int j = 0; j < 5; ++j) {
         // nothing in the iteration reads the gradient: streaming stores keep
@@ -1029,11 +1034,11 @@ __device__ __forceinline__ void grad_tet_body(int c, int nC, int n, const int* _
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_grad_tet(int nC, int n, const int* __restrict__ snb,
                                                      const typename Real<R>::vec4* __restrict__ sgeo,
-                                                     const int* __restrict__ snode, const int* __restrict__ depmask,
+                                                     const int4* __restrict__ cnode, const unsigned short* __restrict__ gsel,
                                                      const double* __restrict__ q, const R* __restrict__ qn,
                                                      const double* __restrict__ vol, R* __restrict__ gx,
                                                      R* __restrict__ gy, R* __restrict__ gz) {
-    grad_tet_body<R>(xcd_block() * kBlock + (int)threadIdx.x, nC, n, snb, sgeo, snode, depmask, q, qn, vol, gx, gy,
+    grad_tet_body<R>(xcd_block() * kBlock + (int)threadIdx.x, nC, n, snb, sgeo, cnode, gsel, q, qn, vol, gx, gy,
                      gz);
 }
 
@@ -1059,8 +1064,8 @@ __global__ __launch_bounds__(kBlock) void k_grad_tet(int nC, int n, const int* _
 template <typename R>
 __global__ __launch_bounds__(kBlock) void k_grad_tet_claim(int nblk, int nC, int n, const int* __restrict__ snb,
                                                            const typename Real<R>::vec4* __restrict__ sgeo,
-                                                           const int* __restrict__ snode,
-                                                           const int* __restrict__ depmask,
+                                                           const int4* __restrict__ cnode,
+                                                           const unsigned short* __restrict__ gsel,
                                                            const double* __restrict__ q, const R* __restrict__ qn,
                                                            const double* __restrict__ vol, R* __restrict__ gx,
                                                            R* __restrict__ gy, R* __restrict__ gz, int* counters) {
@@ -1074,7 +1079,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_tet_claim(int nblk, int nC, int
         __syncthreads();  // every thread has read `claimed`
         int next = 0;
         if (threadIdx.x == 0) next = atomicAdd(ctr, 1);
-        grad_tet_body<R>((x * span + k) * kBlock + (int)threadIdx.x, nC, n, snb, sgeo, snode, depmask, q, qn, vol,
+        grad_tet_body<R>((x * span + k) * kBlock + (int)threadIdx.x, nC, n, snb, sgeo, cnode, gsel, q, qn, vol,
                          gx, gy, gz);
         if (threadIdx.x == 0) claimed = next;
         __syncthreads();
@@ -1093,7 +1098,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_tet_claim(int nblk, int nC, int
 template <bool MIXED, typename R>
 __global__ __launch_bounds__(kBlock) void k_grad_flux_ts(int nC, int n, const int* __restrict__ snb,
                                                         const typename Real<R>::vec4* __restrict__ sgeo_r,
-                                                        const int* __restrict__ snode, const int* __restrict__ depmask,
+                                                        const int4* __restrict__ cnode, const unsigned short* __restrict__ gsel,
                                                         const double* __restrict__ q, const R* __restrict__ qn,
                                                         const double* __restrict__ vol, R* __restrict__ gx,
                                                         R* __restrict__ gy, R* __restrict__ gz,
@@ -1104,7 +1109,7 @@ __global__ __launch_bounds__(kBlock) void k_grad_flux_ts(int nC, int n, const in
                                                         double cfl_min, float* __restrict__ q32,
                                                         float* __restrict__ diag32) {
     const int c = xcd_block() * kBlock + (int)threadIdx.x;
-    grad_tet_body<R>(c, nC, n, snb, sgeo_r, snode, depmask, q, qn, vol, gx, gy, gz);  // no-op past nC
+    grad_tet_body<R>(c, nC, n, snb, sgeo_r, cnode, gsel, q, qn, vol, gx, gy, gz);  // no-op past nC
     flux_ts_slot_body<4, MIXED>(c, nC, snb, sgeo, sdn, sflip, q, vol, res, dt, diag,
                                 part + blockIdx.x, (int)gridDim.x, K, cfl, cfl_min, q32, diag32);
 }

@@ -331,15 +331,13 @@ __global__ __launch_bounds__(kBlock) void k_cell_centroid_fix(MetricArgs A, doub
 // face's unit normal pointing away from the cell with its area (negated
 // exactly where the cell is the face's second cell; zeros for an empty
 // slot), the distance on this cell's side, per cell the slots where it is
-// the second cell (bits 0-7) and its face count (bits 8-11), and for
-// tetrahedra each slot's three face nodes in the face's order.
+// the second cell (bits 0-7) and its face count (bits 8-11).
 template <int LPC>
 __global__ __launch_bounds__(kBlock) void k_slot_tables(int nC, const int* __restrict__ cfs,
                                                        const int* __restrict__ cfo, const int2* __restrict__ fcell,
                                                        const double4* __restrict__ fgeo,
-                                                       const double2* __restrict__ fdn, const int* __restrict__ fno,
-                                                       const int* __restrict__ fn, int* snb, double4* sgeo,
-                                                       float4* sgeo32, double* sdn, int* sflip, int* snode) {
+                                                       const double2* __restrict__ fdn, int* snb, double4* sgeo,
+                                                       float4* sgeo32, double* sdn, int* sflip) {
     const int d = (int)(blockIdx.x * kBlock + threadIdx.x);
     if (d >= nC) return;
     int flips = (cfo[d + 1] - cfo[d]) << 8;
@@ -363,10 +361,54 @@ __global__ __launch_bounds__(kBlock) void k_slot_tables(int nC, const int* __res
         if (sgeo32) sgeo32[i] = make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w);
         const double2 dn = fdn[f];
         sdn[i] = flip ? dn.y : dn.x;
-        if (snode)
-            for (int k = 0; k < 3; ++k) snode[12 * (size_t)d + 3 * sl + k] = fn[fno[f] + k];
     }
     sflip[d] = flips;
+}
+
+// The gradient's tables of a tetrahedral cell: its four nodes, node s being
+// the one that is not on the face of slot s, and a word with, in bits 2s and
+// 2s+1, which of that face's nodes its face list names last (0-2, in the
+// order of the cell's nodes) and in bit 8+s whether the slot takes the
+// cell/ghost average (depmask bits 24-27).  `bad` is set where four triangles
+// do not close a tetrahedron; such a mesh takes the general gradient.
+__global__ __launch_bounds__(kBlock) void k_tet_tables(int nC, const int* __restrict__ cfs, const int* __restrict__ fn,
+                                                      const int* __restrict__ depmask, int4* cnode,
+                                                      unsigned short* gsel, int* bad) {
+    const int d = (int)(blockIdx.x * kBlock + threadIdx.x);
+    if (d >= nC) return;
+    int t[4][3], v[4];
+    for (int s = 0; s < 4; ++s)
+        for (int k = 0; k < 3; ++k) t[s][k] = fn[3 * (size_t)cfs[4 * (size_t)d + s] + k];
+    bool ok = true;
+    for (int s = 0; s < 4; ++s) {  // the one node of the next slot's face that this slot's face lacks
+        const int* o = t[(s + 1) & 3];
+        int found = 0;
+        for (int k = 0; k < 3; ++k)
+            if (o[k] != t[s][0] && o[k] != t[s][1] && o[k] != t[s][2]) {
+                v[s] = o[k];
+                ++found;
+            }
+        ok = ok && found == 1;
+    }
+    unsigned sel = (((unsigned)depmask[d] >> 24) & 15u) << 8;
+    for (int s = 0; s < 4 && ok; ++s) {
+        int last = -1, on = 0, m = 0;
+        for (int j = 0; j < 4; ++j) {
+            if (j == s) continue;
+            for (int k = 0; k < 3; ++k) on += t[s][k] == v[j];
+            if (t[s][2] == v[j]) last = m;
+            ++m;
+        }
+        ok = on == 3 && last >= 0 && v[0] != v[1] && v[0] != v[2] && v[0] != v[3] && v[1] != v[2] && v[1] != v[3] &&
+             v[2] != v[3];
+        sel |= (unsigned)last << (2 * s);
+    }
+    if (!ok) {
+        *bad = 1;
+        return;
+    }
+    cnode[d] = make_int4(v[0], v[1], v[2], v[3]);
+    gsel[d] = (unsigned short)sel;
 }
 
 // One direction's dependency tables of the sweeps (SweepLayout): the

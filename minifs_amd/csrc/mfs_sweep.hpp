@@ -202,12 +202,6 @@ struct SweepArgs {
     int run_shift;
 };
 
-template <typename R>
-__device__ __forceinline__ void load5r(const R* __restrict__ p, R v[5]) {
-#pragma unroll
-    for (int j = 0; j < 5; ++j) v[j] = p[j];
-}
-
 // This wave's words of LDS: the dependencies' products (5 x 64 values), then
 // the chunk's records (64 cells of 5 values).  A wave's LDS accesses complete
 // in order; lds_order keeps the compiler from moving them across each other.
