@@ -171,11 +171,14 @@ typedef struct mfs_ctx_options {
                           * residual pass; 2, 3, 4, 5 on a second stream of the context, started after the
                           * update, after the next iteration's residual pass, after its forward sweep, or
                           * after the wide levels of its forward sweep, when the thin tail begins
-                          * (nothing in an iteration reads the gradient).  Default 5 (the fastest on 6.0M
-                          * cells in both precisions). */
-    int sweep_tail_grid; /* workgroups of the sweeps' thin-tail launch: each sweep of the flat schedule runs
-                          * its wide levels and the run of thin levels that ends its order (at most 64
-                          * chunks each) as two launches.  0: default (64); -1: one launch per sweep. */
+                          * (nothing in an iteration reads the gradient).  With 5, and a tail long enough
+                          * to hide it, the gradient runs inside the tails' launches instead, on the CUs
+                          * they leave idle.  Default 5 (the fastest on 6.0M cells in both precisions). */
+    int sweep_tail_grid; /* workgroups (of 2 waves, on one XCD) of the sweeps' thin-tail launch: each sweep
+                          * of the flat schedule runs its wide levels and the run of thin levels that ends
+                          * its order as two launches.  A level is thin with at most 64 chunks, counted as
+                          * 16 cells of a tile (8 on meshes with more than 4 faces per cell).  0: default
+                          * (64); -1: one launch per sweep. */
 } mfs_ctx_options;
 int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p, int precision, const mfs_ctx_options* opt,
                       mfs_ctx** out);

@@ -123,6 +123,7 @@ struct mfs_ctx {
     // other work can fill the CUs the tail leaves idle.
     int tail_grid = 0;
     bool all_thin = false;  // every level is thin
+    int thin_levels = 0;    // levels of the thin tail, or all
     int tail_chunks = 0;  // its width in groups of 64/lpc cells per tile
     int tail_cells = 0;
     int compute_units = 0;  // CUs of the device

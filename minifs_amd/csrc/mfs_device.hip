@@ -36,7 +36,7 @@ void set_error(const std::string& msg);  // mfs_capi.cpp
 // side-stream gradient's block counters (2.03 MiB).
 constexpr int kNoAllocMaxCells = 1 << 23;
 constexpr size_t kNoAllocPartDoubles = (size_t)(((kNoAllocMaxCells + 255) / 256 + 7) / 8 * 8) * 8;
-constexpr size_t kNoAllocTicketInts = 2 * 64 * 64 + 2 * 8 * 64;
+constexpr size_t kNoAllocTicketInts = 2 * 64 * 64 + 4 * 8 * 64;
 constexpr size_t kNoAllocBytes = kNoAllocPartDoubles * sizeof(double) + kNoAllocTicketInts * sizeof(int);
 static __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
@@ -79,7 +79,9 @@ constexpr int kTicketStride = 64;  // ints between counters (256 bytes)
 // stream (a context's gradient; a batch's node values and gradient).
 constexpr size_t kGradClaimOffset = 2 * (size_t)kTicketGroups * kTicketStride;
 constexpr size_t kNodeClaimOffset = kGradClaimOffset + (size_t)dev::kXcd * kTicketStride;
-constexpr size_t kTicketInts = kNodeClaimOffset + (size_t)dev::kXcd * kTicketStride;
+// and the same for the side work of the two directions' thin launches
+constexpr size_t kSideOffset = kNodeClaimOffset + (size_t)dev::kXcd * kTicketStride;
+constexpr size_t kTicketInts = kSideOffset + 2 * (size_t)dev::kXcd * kTicketStride;
 // Wide launches hand out runs of 4 consecutive steps per ticket group: on
 // the 6.0M-cell mesh 1.2% faster per FP64 iteration than single steps
 // (1.0% mixed), and 8-step runs gained less.  The thin tail keeps single
@@ -108,7 +110,18 @@ constexpr int kDefaultBatchGradientStreamMixed = 4;
 // of kThinWaves waves, all on one XCD (k_sweep_xcd; a thin level has at most
 // 64 groups of cells), when it holds at least kMinTailChunks of them.
 constexpr int kDefaultTailGrid = 64;
-constexpr int kThinWaves = 2;  // waves per workgroup of an XCD-local launch of thin levels
+constexpr int kThinWaves = 2;  // waves that a workgroup of the tail grid stands for
+// Workgroups per CU of a thin launch with side work (4 waves each, the
+// registers' limit).
+constexpr int kSideGroups = 4;
+// The gradient runs inside the thin launches up to this many cells per thin
+// level, and on the second stream above, where the thin levels are too short
+// to hide it and the second stream spreads it over the wide levels too.
+// Measured, ms per iteration, second stream / inside: 6.0M cells FP64, 26k
+// cells per thin level, 3.12 / 2.91; 1.3M cells FP64, 10k, 1.04 / 0.97; 262k
+// hexahedra FP64, 2k, 0.675 / 0.667; 2.9M cells mixed in the shallow order,
+// 117k, 1.02 / 1.13; 2.1M cells FP64 in a 3/512 order, about 59k, 1.03 / 1.11.
+constexpr int kSideCellsPerLevel = 36000;
 
 #include "mfs_kernels.hpp"
 #include "mfs_sweep.hpp"
@@ -263,6 +276,7 @@ using dev::kTicketGroups;
 using dev::kTicketStride;
 using dev::kGradClaimOffset;
 using dev::kNodeClaimOffset;
+using dev::kSideOffset;
 using dev::kTicketInts;
 
 bool hip_ok(mfs_ctx* ctx, hipError_t e, const char* what) {
@@ -712,11 +726,79 @@ void sweep_args(dev::SweepArgs<R>& A, const mfs_ctx* ctx, int cur) {
     A.cell0 = ctx->cell0;
 }
 
+// Whether each sweep has a launch of thin levels, on one XCD.
+bool thin_launch(const mfs_ctx* ctx) { return sweep_split(ctx) || (!ctx->sweep_by_tiles && ctx->all_thin); }
+
+// Symmetry-plane projection of the node values.
+template <typename R>
+bool launch_node_symm(mfs_ctx* ctx, hipStream_t st) {
+    if (ctx->nsym == 0) return true;
+    R* qn;
+    if constexpr (sizeof(R) == sizeof(double))
+        qn = ctx->qn;
+    else
+        qn = ctx->qn32;
+    hipLaunchKernelGGL(dev::k_node_symm<R>, dim3(nblk(ctx->nsym)), dim3(kBlock), 0, st, ctx->nsym, ctx->sym_node,
+                       ctx->sym_n, qn);
+    return check_launch(ctx, "k_node_symm");
+}
+
+// The side work of one direction's thin launch: the node values or the
+// gradient of the state `q` (none for a null `q`).
+template <typename R>
+dev::SideWork<R> side_work(mfs_ctx* ctx, bool fwd, const double* q) {
+    dev::SideWork<R> W{};
+    int* const side = ctx->tickets + kSideOffset;
+    const size_t one = (size_t)dev::kXcd * kTicketStride;
+    W.counters = side + (fwd ? 0 : one);
+    W.clear = side + (fwd ? one : 0);
+    if (!q) return W;
+    W.nblk = fwd ? (int)nblk_xcd(ctx->nN) : ctx->nblk_cell;
+    W.nN = ctx->nN;
+    W.nlo = ctx->nlo;
+    W.ell_off = ctx->ell_off;
+    W.ell_ab = ctx->ell_ab;
+    W.nden = ctx->nden;
+    W.q = q;
+    W.nC = ctx->nC;
+    W.n = ctx->nC + ctx->nB;
+    W.snb = ctx->snb;
+    W.cnode = ctx->cnode;
+    W.gsel = ctx->gsel;
+    W.vol = ctx->vol;
+    W.cfo = ctx->cfo;
+    W.cf = ctx->cf;
+    W.fno = ctx->fno;
+    W.fn = ctx->fn;
+    W.btype = ctx->btype;
+    W.fcell = ctx->fcell;
+    if constexpr (sizeof(R) == sizeof(double)) {
+        W.ell_w = ctx->ell_w;
+        W.qn = ctx->qn;
+        W.sgeo = ctx->sgeo;
+        W.fgeo = ctx->fgeo;
+        W.gx = ctx->gx;
+        W.gy = ctx->gy;
+        W.gz = ctx->gz;
+    } else {
+        W.ell_w = ctx->ell_w32;
+        W.qn = ctx->qn32;
+        W.sgeo = ctx->sgeo32;
+        W.fgeo = ctx->fgeo32;
+        W.gx = ctx->gx32;
+        W.gy = ctx->gy32;
+        W.gz = ctx->gz32;
+    }
+    return W;
+}
+
 // The two sweeps and the update.  `after` is enqueued after the forward
 // sweep, or, with at_tail on a split sweep, after its wide levels, before
-// its thin tail.
+// its thin tail.  With grad_q (a context with thin launches) the gradient of
+// that state runs beside the thin levels: its node values with the forward
+// sweep's, its Green-Gauss pass with the backward sweep's.
 template <int MAXD, typename R>
-bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_tail) {
+bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_tail, const double* grad_q) {
     dev::SweepArgs<R> A;
     sweep_args(A, ctx, ctx->cur);
     const bool flat = !ctx->sweep_by_tiles;
@@ -739,7 +821,7 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     int* const tk[2] = {ctx->tickets, ctx->tickets + kTicketGroups * kTicketStride};
     int set = 0;
     // ev0 / ev1: the timing events that this launch's start / end set
-    auto launch = [&](const void* fn, bool thin, dim3 g, int ubeg, int uend, const char* what, hipEvent_t ev0,
+    auto launch = [&](const void* fn, bool fwd, bool thin, dim3 g, int ubeg, int uend, const char* what, hipEvent_t ev0,
                       hipEvent_t ev1) {
         A.ubeg = ubeg;
         A.uend = uend;
@@ -748,12 +830,24 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
         A.tickets = tk[set];
         A.tickets_next = tk[1 - set];
         set ^= 1;
-        int join = (int)g.x;
-        void* args[] = {&A, &ctx->K, &join};
-        if (thin) g.x *= dev::kXcd;  // one XCD's share of the grid takes part
-        const int waves = thin ? dev::kThinWaves : ctx->sweep_waves;
-        return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(64 * waves), args, dev::stage_bytes(waves), ctx->stream, ev0,
-                                             ev1, 0), what);
+        if (!thin) {
+            void* args[] = {&A, &ctx->K};
+            return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(64 * ctx->sweep_waves), args,
+                                                 dev::stage_bytes(ctx->sweep_waves), ctx->stream, ev0, ev1, 0), what);
+        }
+        // the tail grid's waves on one XCD; with side work, workgroups for
+        // every CU
+        constexpr int W = kBlock / 64;
+        const int join = std::max(1, ((int)g.x * dev::kThinWaves + W - 1) / W);
+        dev::XcdArgs<R> P{A, ctx->K, side_work<R>(ctx, fwd, grad_q), join};
+        g.x = (unsigned)(join * dev::kXcd);
+        if (P.W.nblk > 0) {
+            const int most = (int)g.x + P.W.nblk;
+            g.x = std::max<unsigned>(g.x, (unsigned)std::min(dev::kSideGroups * ctx->compute_units, most));
+        }
+        void* args[] = {&P};
+        return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(kBlock), args, dev::stage_bytes(W), ctx->stream, ev0, ev1, 0),
+                      what);
     };
     SweepTurn turn(ctx->device, ctx->stream);
     if (turn.error()) return sweep_turn_failed(ctx, turn.error());
@@ -763,16 +857,17 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
                           : flat ? (const void*)dev::k_sweep<true, MAXD, R, dev::kAnyChunks>
                                  : (const void*)dev::k_sweep_tiles<true, MAXD, R>;
         if (split) {
-            if (!launch((const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>, false, grid, 0, wf, "k_sweep<fwd>",
+            if (!launch((const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>, true, false, grid, 0, wf, "k_sweep<fwd>",
                         t.start(0), t.stop(0)))
                 return false;
             if (at_tail && after && !after()) return false;
-            if (!launch((const void*)dev::k_sweep_xcd<true, MAXD, R>, true, tgrid, wf, nf, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
+            if (!launch((const void*)dev::k_sweep_xcd<true, MAXD, R>, true, true, tgrid, wf, nf, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
                 return false;
-        } else if (!launch(fwd, local, local ? lgrid : grid, 0, nf, "k_sweep<fwd>", t.start(0), t.stop(0))) {
+        } else if (!launch(fwd, true, local, local ? lgrid : grid, 0, nf, "k_sweep<fwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("fwd_sweep", "fwd_sweep_wide", "fwd_sweep_tail");
+        if (grad_q && !launch_node_symm<R>(ctx, ctx->stream)) return false;
     }
     if ((!at_tail || !split) && after && !after()) return false;
     {
@@ -781,12 +876,12 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
                           : flat ? (const void*)dev::k_sweep<false, MAXD, R, dev::kAnyChunks>
                                  : (const void*)dev::k_sweep_tiles<false, MAXD, R>;
         if (split) {
-            if (!launch((const void*)dev::k_sweep_xcd<false, MAXD, R>, true, tgrid, 0, tb,
+            if (!launch((const void*)dev::k_sweep_xcd<false, MAXD, R>, false, true, tgrid, 0, tb,
                         "k_sweep<bwd> (thin tail)", t.start(0), t.stop(0)) ||
-                !launch((const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>, false, grid, tb, nb, "k_sweep<bwd>",
+                !launch((const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>, false, false, grid, tb, nb, "k_sweep<bwd>",
                         t.start(1), t.stop(1)))
                 return false;
-        } else if (!launch(bwd, local, local ? lgrid : grid, 0, nb, "k_sweep<bwd>", t.start(0), t.stop(0))) {
+        } else if (!launch(bwd, false, local, local ? lgrid : grid, 0, nb, "k_sweep<bwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("bwd_sweep", "bwd_sweep_tail", "bwd_sweep_wide");
@@ -795,12 +890,13 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     ctx->cur = 1 - ctx->cur;
     return true;
 }
-bool launch_sweeps(mfs_ctx* ctx, const std::function<bool()>& after = nullptr, bool at_tail = false) {
+bool launch_sweeps(mfs_ctx* ctx, const std::function<bool()>& after = nullptr, bool at_tail = false,
+                   const double* grad_q = nullptr) {
     if (ctx->precision == MFS_MIXED)
-        return ctx->maxf == 4 ? launch_sweeps_t<4, float>(ctx, after, at_tail)
-                              : launch_sweeps_t<6, float>(ctx, after, at_tail);
-    return ctx->maxf == 4 ? launch_sweeps_t<4, double>(ctx, after, at_tail)
-                          : launch_sweeps_t<6, double>(ctx, after, at_tail);
+        return ctx->maxf == 4 ? launch_sweeps_t<4, float>(ctx, after, at_tail, grad_q)
+                              : launch_sweeps_t<6, float>(ctx, after, at_tail, grad_q);
+    return ctx->maxf == 4 ? launch_sweeps_t<4, double>(ctx, after, at_tail, grad_q)
+                          : launch_sweeps_t<6, double>(ctx, after, at_tail, grad_q);
 }
 
 // CalculateGradient: node values, then the gradient.  With `next` set (the
@@ -837,11 +933,7 @@ bool launch_gradient_t(mfs_ctx* ctx, bool next = false, double next_cfl = 0.0, h
         hipLaunchKernelGGL(dev::k_node<R>, dim3(nblk_xcd(ctx->nN)), dim3(kBlock), 0, st, ctx->nN, ctx->nlo,
                            ctx->ell_off, ctx->ell_ab, ew, ctx->nden, q, qn);
         if (!check_launch(ctx, "k_node")) return false;
-        if (ctx->nsym > 0) {
-            hipLaunchKernelGGL(dev::k_node_symm<R>, dim3(nblk(ctx->nsym)), dim3(kBlock), 0, st, ctx->nsym,
-                               ctx->sym_node, ctx->sym_n, qn);
-            if (!check_launch(ctx, "k_node_symm")) return false;
-        }
+        if (!launch_node_symm<R>(ctx, st)) return false;
     }
     if (MAXF == 4 && ctx->cnode && next) {
         Timed t(ctx, "grad_flux_ts", st);
@@ -1056,6 +1148,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
         ctx->sweep[d].tail = L.sweep[d].tail;
     }
     ctx->all_thin = L.all_thin;
+    ctx->thin_levels = L.thin_levels;
     ctx->tail_chunks = L.tail_chunks;
     ctx->tail_cells = L.tail_cells;
     ctx->tail_grid = (tail_grid > 0 && !sweep_by_tiles && ctx->tail_chunks > 0) ? tail_grid : 0;
@@ -1383,6 +1476,11 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
     const int mode = ctx->gstream ? ctx->gradient_stream : 1;
     const bool side = mode >= 2;
     const bool fuse = !side && gradient_fuses_next(ctx);
+    // Mode 5 with thin launches: the pending gradient is their side work, on
+    // the solver stream.  (Timing every kernel group needs it in launches of
+    // its own.)
+    const bool inside = mode == 5 && thin_launch(ctx) && ctx->timing != 1 &&
+                        ctx->nC <= (long long)dev::kSideCellsPerLevel * ctx->thin_levels;
     const double* grad_q = nullptr;  // state of the gradient not yet launched
     int grad_par = 0;
     // records `ev` on the solver stream and starts the pending gradient
@@ -1422,12 +1520,15 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
         }
         // ForwardLUSGS: sweeps + update
         std::function<bool()> after_fwd;
-        if (side && mode >= 4 && grad_q) after_fwd = [&] { return side_gradient(ctx->sdone); };
-        if (!launch_sweeps(ctx, after_fwd, mode == 5)) return MFS_ERR_HIP;
+        if (side && !inside && mode >= 4 && grad_q) after_fwd = [&] { return side_gradient(ctx->sdone); };
+        if (!launch_sweeps(ctx, after_fwd, mode == 5, inside ? grad_q : nullptr)) return MFS_ERR_HIP;
         // SetGhostVariables, when enabled (main.cpp:283 has the call commented out)
         if (ctx->ghost_refresh && !launch_ghosts(ctx)) return MFS_ERR_HIP;
         // CalculateGradient (fused: with the next iteration's first pass)
-        if (side) {
+        if (inside) {
+            grad_q = ctx->q[ctx->cur];
+            if (s + 1 == nsteps && !launch_gradient(ctx)) return MFS_ERR_HIP;
+        } else if (side) {
             grad_q = ctx->q[ctx->cur];
             grad_par = par;
             if ((mode == 2 || s + 1 == nsteps) && !side_gradient(ctx->sdone)) return MFS_ERR_HIP;
@@ -1438,7 +1539,7 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
         ctx->hist_n++;
         ctx->iter_done++;
     }
-    if (side && nsteps > 0) {
+    if (side && !inside && nsteps > 0) {
         // join: everything later on the solver stream (entry points,
         // downloads, mfs_sync) comes after the last gradient
         const int last = (ctx->iter_done - 1) & 1;

@@ -452,6 +452,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         int tail_level = L.nlev;  // first level of the thin tail
         while (tail_level > 0 && thin[tail_level - 1]) L.tail_chunks += width[--tail_level];
         L.all_thin = tail_level == 0;
+        L.thin_levels = L.nlev - tail_level;
         if (tail_level == 0 || L.tail_chunks < kMinTailChunks) {
             tail_level = L.nlev;
             L.tail_chunks = 0;

@@ -118,7 +118,7 @@ struct HostLayout {
     lvec<unsigned short> cdep;          // 2*nC
     // the thin tail of the sweep order: the run of thin levels that ends it,
     // counted in the level-width unit below, and its cells
-    int tail_chunks = 0, tail_cells = 0;
+    int tail_chunks = 0, tail_cells = 0, thin_levels = 0;  // thin_levels: also where every level is thin
     bool all_thin = false;              // every level is thin
     bool tri_slots = false;                    // tetrahedra with triangular slots only
     // initial state, 5 blocks of nC+nB, device cell order

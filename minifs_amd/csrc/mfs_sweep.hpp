@@ -532,14 +532,94 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(SweepArgs<R> A, FlowConst
     }
 }
 
-// A launch of thin levels on one XCD.  The first workgroup to start elects
-// its XCD, and up to `join` workgroups of that XCD take the chunks from one
-// counter; the others leave at once (the grid is 8 times `join`, and
-// workgroups are dealt to the XCDs in turn).  Whichever XCD it is, the
-// workgroup that elected it runs, and a chunk is only ever held by a running
-// wave, so the launch ends however its workgroups are placed.
+// The gradient of the previous iteration beside a sweep's thin levels: its
+// node values (a forward launch) or its Green-Gauss pass (a backward one), in
+// blocks of kBlock nodes or cells.
+template <typename R>
+struct SideWork {
+    int nblk;             // blocks, a multiple of 8 (0: none)
+    int* counters;        // one per XCD's span of blocks, kTicketStride apart, zero at the launch
+    int* clear;           // the counters of the other direction's launch, zeroed here
+    // node values
+    int nN;
+    const int *nlo, *ell_off;
+    const int2* ell_ab;
+    const R* ell_w;
+    const double *nden, *q;
+    R* qn;
+    // gradient: tetrahedra by cnode, other cells by their face lists
+    int nC, n;
+    const int* snb;
+    const typename Real<R>::vec4 *sgeo, *fgeo;
+    const int4* cnode;
+    const unsigned short* gsel;
+    const double* vol;
+    const int *cfo, *cf, *fno, *fn, *btype;
+    const int2* fcell;
+    R *gx, *gy, *gz;
+};
+
+template <bool FWD, int MAXF, typename R>
+__device__ __forceinline__ void side_block(const SideWork<R>& W, int b) {
+    const int i = b * kBlock + (int)threadIdx.x;
+    if constexpr (FWD)
+        node_body<R>(i, b * (kBlock / 64) + (int)threadIdx.x / 64, W.nN, W.nlo, W.ell_off, W.ell_ab, W.ell_w, W.nden,
+                     W.q, W.qn);
+    else if (MAXF == 4 && W.cnode)
+        grad_tet_body<R>(i, W.nC, W.n, W.snb, W.sgeo, W.cnode, W.gsel, W.q, W.qn, W.vol, W.gx, W.gy, W.gz);
+    else
+        grad_body<MAXF, R>(i, W.nC, W.n, W.cfo, W.cf, W.fcell, W.fgeo, W.fno, W.fn, W.btype, W.q, W.qn, W.vol, W.gx,
+                           W.gy, W.gz);
+}
+
+// Claims and works blocks until none are left: those of this XCD's span
+// first (blocks x*span .. (x+1)*span-1, whose gathers then share one L2),
+// then the other XCDs'.  The next block is claimed while the current one is
+// worked on.
+template <bool FWD, int MAXF, typename R>
+__device__ __forceinline__ void side_blocks(const SideWork<R>& W, int home) {
+    __shared__ int claimed;
+    const int span = W.nblk / kXcd;
+    for (int t = 0; t < kXcd; ++t) {
+        const int x = (home + t) % kXcd;
+        int* const ctr = W.counters + x * kTicketStride;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            claimed = t > 0 && __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= span
+                          ? span
+                          : atomicAdd(ctr, 1);
+        __syncthreads();
+        int k = claimed;
+        while (k < span) {
+            __syncthreads();  // every thread has read `claimed`
+            int next = 0;
+            if (threadIdx.x == 0) next = atomicAdd(ctr, 1);
+            side_block<FWD, MAXF, R>(W, x * span + k);
+            if (threadIdx.x == 0) claimed = next;
+            __syncthreads();
+            k = claimed;
+        }
+    }
+}
+
+template <typename R>
+struct XcdArgs {
+    SweepArgs<R> A;
+    FlowConst K;
+    SideWork<R> W;
+    int join;
+};
+
+// A launch of thin levels on one XCD, with the previous iteration's gradient
+// on the others.  The first workgroup to start elects its XCD, and up to
+// `join` workgroups of that XCD take the chunks from one counter; its other
+// workgroups leave at once (workgroups are dealt to the XCDs in turn, so the
+// grid holds at least 8 times `join`).  Whichever XCD it is, the workgroup
+// that elected it runs, and a chunk is only ever held by a running wave, so
+// the launch ends however its workgroups are placed.  The workgroups of the
+// other XCDs work the side blocks, and so do the sweeping ones once their
+// chunks are done.
 //
-// A level of the tail is one hop from a wave's store to the next wave's poll.
 // Measured between two waves, an 8-byte word takes 0.39 us to another XCD,
 // 0.36 us to this one with a device-scope store, and 0.22 us with a store
 // that stops in this XCD's L2: a device-scope load is served from the L2 of
@@ -550,28 +630,56 @@ __global__ __launch_bounds__(kSweepBlock) void k_sweep(SweepArgs<R> A, FlowConst
 // us; 262k hexahedra 252 -> 160 us; all 27 levels of a 1,296-cell mesh 53 ->
 // 34 us).  Of it the store and the polls take 0.6 us, the face terms 0.23,
 // the sum, the division and the limiter 0.3.  One wave per SIMD of the XCD is
-// fastest (64 workgroups of 2 waves; 64 of 4: 2% slower iterations, 128 of 4:
-// 7%): more waves only add polls.
-template <bool FWD, int MAXD, typename R>
-__global__ __launch_bounds__(kSweepBlock) void k_sweep_xcd(SweepArgs<R> A, FlowConst K, int join) {
-    __shared__ int in;
+// fastest (128 waves; 256: 2% slower iterations, 512: 7%): more waves only
+// add polls.
+//
+// The side blocks fill the CUs that the sweep leaves idle without sharing its
+// XCD's issue slots and L2: on a second stream their workgroups landed there
+// too, and a tail of 303 us took 605 us beside the node values and 436 beside
+// the gradient (6.0M cells, FP64); inside, the two launches take 373 us with
+// the node values (290 us alone) and 519 with the gradient (440 alone).
+template <bool FWD, int MAXF, typename R>
+__global__ __launch_bounds__(kBlock) void k_sweep_xcd(XcdArgs<R> P) {
+    const SweepArgs<R>& A = P.A;
+    __shared__ int role;  // 1: sweeps, 0: side blocks only, -1: leaves
+    const int me = xcd_id();
     if (threadIdx.x == 0) {
-        const int me = xcd_id() + 1;
         int* const elect = A.tickets + kElectWord;
-        const int won = atomicCAS(elect, 0, me);
-        in = (won == 0 || won == me) && atomicAdd(A.tickets + kJoinWord, 1) < join;
+        int won = __hip_atomic_load(elect, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (won == 0) {
+            won = atomicCAS(elect, 0, me + 1);
+            if (won == 0) won = me + 1;
+        }
+        role = won != me + 1 ? 0 : atomicAdd(A.tickets + kJoinWord, 1) < P.join ? 1 : -1;
     }
     clear_tickets(A.tickets_next);
+    if (blockIdx.x == 0 && threadIdx.x < kXcd) P.W.clear[threadIdx.x * kTicketStride] = 0;
     __syncthreads();
-    if (!in || __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return;
-    int tk = __builtin_amdgcn_readfirstlane(take_ticket(A.tickets));
-    while (true) {
-        const int u = A.ubeg + tk;
-        if (u >= A.uend) return;
-        int next = 0;
-        if (!sweep_chunk<FWD, MAXD, R, kThinChunks>(A, K, u, A.tickets, next)) return;
-        tk = __builtin_amdgcn_readfirstlane(next);
+    const int r = role;
+    if (r < 0) return;
+    if (r == 1 && __hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+        int tk = __builtin_amdgcn_readfirstlane(take_ticket(A.tickets));
+        while (true) {
+            const int u = A.ubeg + tk;
+            if (u >= A.uend) break;
+            int next = 0;
+            if (!sweep_chunk<FWD, MAXF, R, kThinChunks>(A, P.K, u, A.tickets, next)) break;
+            tk = __builtin_amdgcn_readfirstlane(next);
+        }
     }
+    // The side work's arguments are read from the kernel's argument memory
+    // from here on: read at the start they would take the scalar registers
+    // that the sweep's loop needs.
+    typedef const __attribute__((address_space(4))) unsigned* Words;
+    Words w = (Words)__builtin_amdgcn_kernarg_segment_ptr() + offsetof(XcdArgs<R>, W) / 4;
+    asm volatile("" : "+s"(w));
+    struct Copy {
+        unsigned v[sizeof(SideWork<R>) / 4];
+    } copy;
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(copy) / 4; ++i) copy.v[i] = w[i];
+    const SideWork<R> W = __builtin_bit_cast(SideWork<R>, copy);
+    if (W.nblk > 0) side_blocks<FWD, MAXF, R>(W, me % kXcd);
 }
 
 // The tile schedule: one workgroup per tile.
