@@ -23,12 +23,14 @@ struct Real<double> {
     using bits = unsigned long long;
     using vec4 = double4;
     static constexpr bits kSent = 0x7FF4D51F5EED0000ULL;
+    static constexpr double kMost = 1.7976931348623157e308;  // largest finite value
 };
 template <>
 struct Real<float> {
     using bits = unsigned int;
     using vec4 = float4;
     static constexpr bits kSent = 0x7FA5D51Fu;
+    static constexpr float kMost = 3.4028235e38f;
 };
 
 template <int NV, int NW = kBlock / 64>

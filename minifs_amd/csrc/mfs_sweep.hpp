@@ -231,6 +231,16 @@ __device__ __forceinline__ R pick5(R v0, R v1, R v2, R v3, R v4, int j) {
     return j == 4 ? v4 : x;
 }
 
+// The room that value v has inside (lo, hi), and zero where it has none
+// beyond the rounding of sums of its size.
+template <typename R>
+__device__ __forceinline__ R min_room(R v, R lo, R hi) {
+    const R a = v - lo, b = hi - v;
+    const R m = a < b ? a : b;
+    const R size = __builtin_fabs(v) + __builtin_fabs(lo) + __builtin_fabs(hi);
+    return m > size * (sizeof(R) == 8 ? R(1e-9) : R(1e-3)) ? m : R(0);
+}
+
 // The limiter's three stages for the wave's cells; `x` is scaled with DQ.  A
 // cell outside the limits is rare, and where the first stage scales no cell
 // of the wave the others see the same values again, so they are left out.
@@ -324,26 +334,21 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     if constexpr (!FWD && sizeof(R) != sizeof(double)) load5(A.q64 + (size_t)c * 5, q64c);
     bool rep_seen = (rep < 0) || (__shfl(rv, 0, 64) != kSent);
     R qnb[5] = {R(0), R(0), R(0), R(0), R(0)};
-    R dv[5] = {R(0), R(0), R(0), R(0), R(0)};
+    R dv[5] = {R(0), R(0), R(0), R(0), R(0)};  // the neighbour's DQ (a ghost's stays 0)
     if (mine) load5r(A.q + (size_t)nb * 5, qnb);
     const bool wide = wide_records(A.nq);  // the same for every wave
     // one read of every pending dependency (they are interior cells); a
     // value still the sentinel leaves the lane pending
-    R b[5];
     auto settle = [&] {
-        bool ok = true;
+        bool missing = false;
 #pragma unroll
-        for (int j = 0; j < 5; ++j) ok = ok && (__builtin_bit_cast(B, b[j]) != kSent);
-        if (ok) {
-#pragma unroll
-            for (int j = 0; j < 5; ++j) dv[j] = b[j];
-            pend = false;
-        }
+        for (int j = 0; j < 5; ++j) missing |= __builtin_bit_cast(B, dv[j]) == kSent;
+        pend = missing;
     };
     // where the latest dependency is out, the others most likely are too:
     // their reads go out with the neighbours' states
     const bool early = rep_seen && pend;
-    if (early) read_published(wide, static_cast<const R*>(poll), A.nC, nb, b);
+    if (early) read_published(wide, static_cast<const R*>(poll), A.nC, nb, dv);
     if (ctr) next = take_ticket(ctr);
     FacePre<R> pre;
     if (mine) {
@@ -354,6 +359,21 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     }
 
     if (early) settle();
+    // Thin levels: bounds under which this lane's value cannot take its cell
+    // near the limiter's limits.  With |DQ_0| at most half the room that rho
+    // has, and each of the five terms of dp at most a 16th of the room that p
+    // has, rho and p stay well inside; where there is no room beyond rounding
+    // (a clamped state) no value counts as safe.
+    R safe_r = R(-1), safe_p = R(-1), safe_w = R(0);
+    if (thin) {
+        const R mr = min_room(qc[0], (R)K.rho_min, (R)K.rho_max), mp = min_room(qc[4], (R)K.p_min, (R)K.p_max);
+        const R vv = qc[1] * qc[1] + qc[2] * qc[2] + qc[3] * qc[3];
+        const R w = pick5(R(0.5) * vv, qc[1], qc[2], qc[3], R(1), j5);
+        safe_w = (R)K.gamm1 * __builtin_fabs(w);
+        safe_r = j5 == 0 ? R(0.5) * mr : Real<R>::kMost;
+        safe_p = R(0.0625) * mp;
+        if (!((mr > R(0)) & (mp > R(0)))) safe_r = R(-1);
+    }
     unsigned spins = 0;
     if (!rep_seen) {  // one lane waits for the chunk's latest dependency (thin: for that one's own)
         while (true) {
@@ -372,7 +392,7 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     while (__ballot(pend) != 0) {
         if (pend) {
             asm volatile("" ::: "memory");  // the reads of this turn are not those of the last
-            read_published(wide, static_cast<const R*>(poll), A.nC, nb, b);
+            read_published(wide, static_cast<const R*>(poll), A.nC, nb, dv);
             settle();
         }
         if (__ballot(pend) == 0) break;
@@ -419,13 +439,27 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
             const R tmp = R(2.0) * dg;
             x -= acc / tmp;
         }
-        lds_order();
-        st[lane] = x;
-        lds_order();
+        // The limiter needs the cell's five values, an exchange through LDS on
+        // the level's critical path.  A value so small that no cell's limits
+        // can be reached is known by its own lane (safe_r, safe_p below), so
+        // the exchange is left to the rare chunk with a larger one; the
+        // backward sweep's update makes it after publishing.
+        const bool near = !((__builtin_fabs(x) <= safe_r) & (__builtin_fabs(x) * safe_w <= safe_p));
+        bool have = false;
+        auto exchange = [&] {
+            lds_order();
+            st[lane] = x;
+            lds_order();
 #pragma unroll
-        for (int j = 0; j < 5; ++j) D[j] = st[5 * (lane / 5) + j];
-        lds_order();
-        limit_dq<R>(FWD && c == A.cell0, qc, D, x, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min, (R)K.p_max);
+            for (int j = 0; j < 5; ++j) D[j] = st[5 * (lane / 5) + j];
+            lds_order();
+            have = true;
+        };
+        if (__builtin_amdgcn_ballot_w64(near) != 0) {
+            exchange();
+            limit_dq<R>(FWD && c == A.cell0, qc, D, x, (R)K.gamm1, (R)K.rho_min, (R)K.rho_max, (R)K.p_min,
+                        (R)K.p_max);
+        }
         if (lane < nw) {
             if (KIND == kThinChunks)
                 st_xcd<R>(own + w0 + lane, x);
@@ -433,6 +467,7 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
                 st_dev<R>(own + w0 + lane, x);
             other[w0 + lane] = sent;
         }
+        if (!FWD && !have) exchange();
     } else {
         R acc[5] = {R(0), R(0), R(0), R(0), R(0)};
 #pragma unroll
@@ -626,10 +661,10 @@ struct XcdArgs {
 // its own XCD as long as no other XCD has written the line.  With the chunk's
 // results one lane each and the next ticket taken behind the first loads, a
 // level of the 6.0M-cell mesh's tail (234 levels, FP64) took 1.88 us before
-// and 1.29 us now (tails alone, forward and backward, 438 / 442 -> 303 / 305
-// us; 262k hexahedra 252 -> 160 us; all 27 levels of a 1,296-cell mesh 53 ->
-// 34 us).  Of it the store and the polls take 0.6 us, the face terms 0.23,
-// the sum, the division and the limiter 0.3.  One wave per SIMD of the XCD is
+// and 1.20 us now (tails alone, forward and backward, 438 / 442 -> 279 / 288
+// us; 262k hexahedra 252 -> 131 us; all 27 levels of a 1,296-cell mesh 53 ->
+// 32 us).  Of it the store and the polls take 0.6 us, the face terms 0.23,
+// the sum and the division 0.1.  One wave per SIMD of the XCD is
 // fastest (128 waves; 256: 2% slower iterations, 512: 7%): more waves only
 // add polls.
 //

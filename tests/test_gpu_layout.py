@@ -68,3 +68,52 @@ def test_sweep_chunks_bitwise(tmp_path, cells, dims, tree, opts):
     s.close()
     o.close()
     g.close()
+
+
+@pytest.mark.parametrize("n,amp,opts", [(8, 0.5, {}), (8, 0.1, {}), (8, 0.5, {"sweep_by_tiles": 1}), (20, 0.5, {}),
+                                        (20, 0.02, {}), (20, 0.5, {"sweep_tail_grid": -1})])
+def test_limiter_paths_bitwise(tmp_path, n, amp, opts):
+    """The DQ limiter in every sweep path (all levels thin, wide levels with a
+    thin tail, one launch, tiles) on states far from and near the freestream
+    with tightened limits, where thin chunks decide by bounds on single
+    values whether the cells' five values are exchanged: bit for bit against
+    the oracle, whose counters show the limiter's stages (large amplitude);
+    and the FP32 operator gives the same bits in every path."""
+    from tests import guards
+
+    print(f"[layout] limiter n={n} amp={amp} {opts}", flush=True)
+    p = guards.params()
+    g0 = mfs.Grid.box_bump(n).decouple()
+    mesh, bc = str(tmp_path / "m.mfl"), str(tmp_path / "m.bc")
+    g0.save(mesh, bc)
+    i = g0.info
+    st = guards.perturbed_state(i["nTCell"] + i["nBFace"], p, amp=amp)
+    if amp < 0.5:
+        st["p"] *= amp
+    g = g0.preprocess(p)
+    o = Oracle(mesh, bc, guards.MACH, guards.ALPHA, guards.CFL, limits=guards.LIMITS)
+    s = mfs.Solver(g, p, **opts)
+    for k, a in st.items():
+        o.set(k, a)
+        s.upload(k, a)
+    for it in range(guards.ITERS):
+        o.run(1, 0)
+        s.step(1)
+        for nm in FIELDS:
+            np.testing.assert_array_equal(s.field(nm), o.get(nm), err_msg=f"iteration {it}: {nm}")
+    c = o.counts()
+    if amp == 0.5:
+        assert all(c[k] > 0 for k in ("fwd_limit1", "fwd_limit2", "fwd_limit3", "bwd_limit1", "bwd_limit3")), c
+    s.close()
+    m = [mfs.Solver(g, p, precision=mfs.MFS_MIXED, **kw) for kw in (opts, {"sweep_by_tiles": 1, "tile_cells": 512})]
+    for x in m:
+        for k, a in st.items():
+            x.upload(k, a)
+        x.step(guards.ITERS)
+    for nm in FIELDS:
+        np.testing.assert_array_equal(m[0].field(nm), m[1].field(nm), err_msg=f"mixed {nm}")
+        assert np.isfinite(m[0].field(nm)).all()
+    for x in m:
+        x.close()
+    o.close()
+    g.close()
