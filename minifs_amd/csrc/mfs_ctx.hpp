@@ -74,8 +74,8 @@ struct mfs_ctx {
     int nsym = 0;
     int* sym_node = nullptr;
     double* sym_n = nullptr;
-    std::vector<int> node_of_dev;  // host: device node -> mesh node
-    std::vector<int> cell_of_dev;  // host: device cell -> mesh cell
+    int *dev_of_cell = nullptr, *dev_of_node = nullptr;  // mesh cell / node -> device cell / node
+    bool io_member = false;  // counted among the users of its device's staging slots
     // sweeps
     // per direction (forward, backward): the schedule and the dependency
     // tables (SweepLayout in mfs_prep.hpp)

@@ -113,6 +113,43 @@ __global__ void k_fill_i(int* p, size_t n, int v) {
     if (i < n) p[i] = v;
 }
 
+// A field between its device array and the reference layout.  Value t of the
+// layout is row t % rows of block t / rows; a row below nmap is stored at
+// device row map[row], and the value of block j at row d at
+// [d * row_stride + j * block_stride + offset].
+struct FieldMap {
+    size_t rows, nmap;
+    const int* map;
+    size_t row_stride, block_stride, offset;
+};
+__device__ __forceinline__ size_t field_index(const FieldMap& M, size_t t) {
+    const size_t j = t / M.rows, row = t - j * M.rows;
+    const size_t d = row < M.nmap ? (size_t)M.map[row] : row;
+    return d * M.row_stride + j * M.block_stride + M.offset;
+}
+// Values [t0, t0 + cnt) of the layout to out, as doubles (src32: an FP32 field).
+__global__ __launch_bounds__(kBlock) void k_field_out(FieldMap M, size_t t0, size_t cnt, const double* __restrict__ src,
+                                                      const float* __restrict__ src32, double* __restrict__ out) {
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= cnt) return;
+    const size_t k = field_index(M, t0 + i);
+    out[i] = src32 ? (double)src32[k] : src[k];
+}
+// The other way, into one array or two.
+__global__ __launch_bounds__(kBlock) void k_field_in(FieldMap M, size_t t0, size_t cnt, const double* __restrict__ in,
+                                                     double* __restrict__ dst, double* __restrict__ dst2) {
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i >= cnt) return;
+    const size_t k = field_index(M, t0 + i);
+    const double v = in[i];
+    dst[k] = v;
+    if (dst2) dst2[k] = v;
+}
+__global__ __launch_bounds__(kBlock) void k_narrow(size_t n, const double* __restrict__ src, float* __restrict__ dst) {
+    const size_t i = (size_t)blockIdx.x * kBlock + threadIdx.x;
+    if (i < n) dst[i] = (float)src[i];
+}
+
 // SetGhostVariables (src/Kernels/load_grid.cpp:953-1212), inviscid branch:
 // the ghost state behind each boundary face from the state of the cell in
 // front of it.  One thread per boundary face k; the ghost is cell nC+k and

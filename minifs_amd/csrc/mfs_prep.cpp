@@ -604,6 +604,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
     });
     for (int j = 0; j < 5; ++j)
         for (int k = nC; k < n; ++k) L.q[(size_t)j * n + k] = src[j][k];
+    L.dev_of_cell = std::move(dcell);
+    L.dev_of_node = std::move(dnode);
     return "";
 }
 

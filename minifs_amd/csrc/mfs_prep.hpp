@@ -77,6 +77,7 @@ struct HostLayout {
     int nC = 0, nF = 0, nB = 0, nN = 0;
     // cells in device order; cell_of_dev[d] = mesh cell id (ghost k stays at nC+k)
     lvec<int> cell_of_dev;
+    std::vector<int> dev_of_cell, dev_of_node;  // the inverse maps
     int dev_cell0 = 0;                         // device id of mesh cell 0
     // per device cell: bits 0-7 forward dependency slots (interior neighbour
     // with a smaller mesh id), bits 8-15 backward slots (neighbour with a

@@ -663,8 +663,8 @@ struct XcdArgs {
 // level of the 6.0M-cell mesh's tail (234 levels, FP64) took 1.88 us before
 // and 1.20 us now (tails alone, forward and backward, 438 / 442 -> 279 / 288
 // us; 262k hexahedra 252 -> 131 us; all 27 levels of a 1,296-cell mesh 53 ->
-// 32 us).  Of it the store and the polls take 0.6 us, the face terms 0.23,
-// the sum and the division 0.1.  One wave per SIMD of the XCD is
+// 32 us).  Of it the store and the polls take 0.5 to 0.65 us, the face terms 0.2,
+// the sum and the division 0.25.  One wave per SIMD of the XCD is
 // fastest (128 waves; 256: 2% slower iterations, 512: 7%): more waves only
 // add polls.
 //
