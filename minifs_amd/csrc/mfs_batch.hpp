@@ -103,7 +103,7 @@ __global__ __launch_bounds__(kSweepBlock) void k_b_sweep(const BatchSolve<R>* __
         if (__hip_atomic_load(A.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
             next = take_ticket(ctr);  // the solve has failed: its chunks are passed over
         else
-            (void)sweep_chunk<FWD, MAXD, R, kWideChunks>(A, T[su.x].K, su.y, ctr, next);
+            (void)sweep_chunk<FWD, MAXD, R, kBatchChunks>(A, T[su.x].K, su.y, ctr, next);
         tk = __builtin_amdgcn_readfirstlane(next);
     }
 }

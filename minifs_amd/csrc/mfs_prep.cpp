@@ -512,6 +512,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                 chunk_at[S.pos[t]] = t;
             }
             S.crec.resize(4 * (size_t)nchunk);
+            S.rep.resize(nchunk);
             size_t nd = 0;
             for (int u = 0; u < nchunk; ++u) {
                 const Chunk& k = ch[chunk_at[u]];
@@ -531,8 +532,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                     std::reverse(S.pos.begin() + S.tile_chunk[t], S.pos.begin() + S.tile_chunk[t + 1]);
             // per cell its place among the chunk's dependencies; per chunk
             // the dependency of the latest level, another tile's first, the
-            // first of equal rank in the chunk's cell and face order (thin:
-            // that dependency's own latest)
+            // first of equal rank in the chunk's cell and face order (narrow
+            // levels: that dependency's own latest)
             parallel_for(nchunk, [&](size_t uu) {
                 const int u = (int)uu;
                 const int d0 = S.crec[4 * uu], cells = S.crec[4 * uu + 1] & 0xff;
@@ -561,7 +562,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                     start += n;
                     latest(c, best, rep);
                 }
-                if (rep >= 0 && (S.crec[4 * uu + 1] & kThinChunkFlag)) {
+                S.rep[u] = rep;
+                if (rep >= 0 && width[L.flevel[L.cell_of_dev[d0]]] <= kDirectLevelChunks) {
                     const int c = L.cell_of_dev[rep];
                     best = -1;
                     rep = -1;

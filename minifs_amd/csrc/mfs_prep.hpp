@@ -66,9 +66,11 @@ struct SweepLayout {
     int tail = 0;                       // chunks of the thin tail (forward: the last, backward: the first)
     // per position of the sweep's order {first device cell, cells |
     // dependencies << 8 | kThinChunkFlag, first dependency, the dependency
-    // expected to be published last (device cell, -1: none; on a thin level
-    // the one that this dependency itself waits for last)}
+    // expected to be published last (device cell, -1: none; on levels of at
+    // most kDirectLevelChunks the one that this dependency itself waits for
+    // last)}
     lvec<int> crec;
+    lvec<int> rep;                      // per position: the dependency expected to be published last
     lvec<int> tile_chunk;               // ntile+1: first entry of each tile in pos
     lvec<int> pos;                      // positions by tile, in the sweep's level order within the tile
 };
@@ -134,6 +136,16 @@ constexpr int kDefaultTileCells = 4096;
 // lane of its own.
 constexpr int kThinLevelChunks = 64;
 constexpr int kThinCells = 12;
+// On levels of at most this many groups a wave waits on a dependency one
+// level further back and then polls its own at once (SweepLayout::crec); on
+// wider ones it waits on its latest dependency with one load, since there the
+// waves that poll are many.  Measured, ms per iteration for 64 / 256 / 1024 /
+// 2048: 262k hexahedra FP64 0.653 / 0.640 / 0.630 / 0.630, 195k prisms mixed
+// 0.456 / 0.445 / 0.440 / 0.437, 1.3M tetrahedra FP64 0.963 / 0.955 / 0.947 /
+// 0.951, 6.0M 2.90 / 2.88 / 2.86 / 2.87.  A batch interleaves its solves'
+// levels and waits on the latest dependency on all (12 mixed solves of 2.3M
+// cells: 1.167 / 1.175 / 1.190 / 1.198).
+constexpr int kDirectLevelChunks = 1024;
 constexpr int kMinTailChunks = 256;  // shorter tails stay with the wide levels
 constexpr int kThinChunkFlag = 0x10000;
 

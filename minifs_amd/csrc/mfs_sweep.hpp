@@ -53,7 +53,7 @@
 // device-coherent loads and retries while any is the sentinel (each store
 // is single-copy atomic, so a non-sentinel value is final).  One lane per
 // wave first waits on the chunk's latest dependency (rep), which keeps the
-// polling traffic to one load per wave; on thin levels it waits on that
+// polling traffic to one load per wave; on narrow levels it waits on that
 // dependency's own latest one, so that the wave's lanes are polling when
 // their dependencies come, which saves a round trip on the level's critical
 // path.  The forward sweep re-arms the
@@ -167,7 +167,8 @@ __device__ __forceinline__ bool wait_failed(int* err, unsigned spins) {
 template <typename R>
 struct SweepDir {
     int nchunks;
-    const int4* crec;                       // per position: first cell, cells | deps << 8 | flag, first dep, rep
+    const int4* crec;                       // per position: first cell, cells | deps << 8 | flag, first dep, wait
+    const int* rep;                         // per position: the latest dependency (a batch waits on it)
     const int* dnb;                         // per dependency: the neighbour
     const typename Real<R>::vec4* dgeo;     // per dependency: normal away from the cell + area
     const int* tile_chunk;                  // tiles schedule: first entry of each tile in pos
@@ -261,11 +262,14 @@ __device__ __forceinline__ void limit_dq(bool skip, const R (&q)[5], R (&DQ)[5],
 }
 
 // What a launch's chunks are: all treated as wide, all thin (the thin tail),
-// or each by its flag.
-constexpr int kWideChunks = 0, kThinChunks = 1, kAnyChunks = 2;
+// each by its flag, or a batch's (wide, waiting on the latest dependency).
+constexpr int kWideChunks = 0, kThinChunks = 1, kAnyChunks = 2, kBatchChunks = 3;
 
 // A record that no kernel writes, at an index that every lane shares: read
 // through the scalar cache.
+__device__ __forceinline__ int load_record(const int* p, int u) {
+    return ((const __attribute__((address_space(4))) int*)p)[u];
+}
 __device__ __forceinline__ int4 load_record(const int4* p, int u) {
     typedef int v4i __attribute__((ext_vector_type(4)));
     const v4i r = ((const __attribute__((address_space(4))) v4i*)p)[u];
@@ -296,7 +300,8 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     const int lane = (int)threadIdx.x & 63;
     R* const poll = FWD ? A.dqf : A.dqb;
     const int4 rec = load_record(S.crec, u);
-    const int c0 = rec.x, nc = rec.y & 0xff, nd = (rec.y >> 8) & 0xff, rep = rec.w;
+    const int c0 = rec.x, nc = rec.y & 0xff, nd = (rec.y >> 8) & 0xff;
+    const int rep = KIND == kBatchChunks ? load_record(S.rep, u) : rec.w;
     // a thin level: every lane polls its own dependency (a batch interleaves
     // many solves, so no level of one solve is thin there)
     const bool thin = KIND == kThinChunks || (KIND == kAnyChunks && (rec.y & kThinChunkFlag) != 0);
@@ -375,7 +380,7 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
         if (!((mr > R(0)) & (mp > R(0)))) safe_r = R(-1);
     }
     unsigned spins = 0;
-    if (!rep_seen) {  // one lane waits for the chunk's latest dependency (thin: for that one's own)
+    if (!rep_seen) {  // one lane waits for the chunk's latest dependency (narrow levels: for that one's own)
         while (true) {
             B v = 0;
             if (lane == 0) v = ld_dev<R>(poll + (size_t)rep * 5);
