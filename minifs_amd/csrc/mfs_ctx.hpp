@@ -83,7 +83,7 @@ struct mfs_ctx {
         int nchunk = 0;
         int tail = 0;               // chunks of the thin tail
         int4* crec = nullptr;
-        int* rep = nullptr;
+        int* batch_wait = nullptr;
         int* dnb = nullptr;
         double4* dgeo = nullptr;    // FP64 operator
         float4* dgeo32 = nullptr;   // FP32 operator (mixed precision)

@@ -795,7 +795,7 @@ void sweep_args(dev::SweepArgs<R>& A, const mfs_ctx* ctx, int cur) {
         const mfs_ctx::Sweep& S = ctx->sweep[d];
         A.dir[d].nchunks = S.nchunk;
         A.dir[d].crec = S.crec;
-        A.dir[d].rep = S.rep;
+        A.dir[d].batch_wait = S.batch_wait;
         A.dir[d].dnb = S.dnb;
         A.dir[d].tile_chunk = S.tile_chunk;
         A.dir[d].pos = S.pos;
@@ -1311,7 +1311,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
         const SweepLayout& H = L.sweep[d];
         const size_t nd = H.ndep + 1;  // a last chunk without dependencies points one past them
         ok = ok && dalloc(ctx, S.crec, (size_t)S.nchunk, "chunk records") &&
-             dalloc(ctx, S.rep, H.rep.size(), "latest dependencies") &&
+             dalloc(ctx, S.batch_wait, H.batch_wait.size(), "batch waits") &&
              dalloc(ctx, S.pos, H.pos.size(), "chunk positions") &&
              dalloc(ctx, S.tile_chunk, H.tile_chunk.size(), "tile_chunk") &&
              dalloc(ctx, S.dnb, nd, "dependency neighbours") &&
@@ -1395,7 +1395,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
             const SweepLayout& H = L.sweep[d];
             ok = ok &&
                  upload(ctx, S.crec, reinterpret_cast<const int4*>(H.crec.data()), (size_t)S.nchunk, "upload chunks") &&
-                 upload(ctx, S.rep, H.rep.data(), H.rep.size(), "upload rep") &&
+                 upload(ctx, S.batch_wait, H.batch_wait.data(), H.batch_wait.size(), "upload waits") &&
                  upload(ctx, S.pos, H.pos.data(), H.pos.size(), "upload pos") &&
                  upload(ctx, S.tile_chunk, H.tile_chunk.data(), H.tile_chunk.size(), "upload tile_chunk");
         }

@@ -512,7 +512,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                 chunk_at[S.pos[t]] = t;
             }
             S.crec.resize(4 * (size_t)nchunk);
-            S.rep.resize(nchunk);
+            S.batch_wait.resize(nchunk);
             size_t nd = 0;
             for (int u = 0; u < nchunk; ++u) {
                 const Chunk& k = ch[chunk_at[u]];
@@ -562,14 +562,15 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                     start += n;
                     latest(c, best, rep);
                 }
-                S.rep[u] = rep;
-                if (rep >= 0 && width[L.flevel[L.cell_of_dev[d0]]] <= kDirectLevelChunks) {
-                    const int c = L.cell_of_dev[rep];
+                // narrow levels wait on that dependency's own latest instead
+                int further = -1;
+                if (rep >= 0) {
                     best = -1;
-                    rep = -1;
-                    latest(c, best, rep);
+                    latest(L.cell_of_dev[rep], best, further);
                 }
-                S.crec[4 * (size_t)u + 3] = rep;
+                const int groups = width[L.flevel[L.cell_of_dev[d0]]];
+                S.batch_wait[u] = groups <= kBatchDirectLevelChunks ? further : rep;
+                S.crec[4 * (size_t)u + 3] = groups <= kDirectLevelChunks ? further : rep;
             });
         };
         {

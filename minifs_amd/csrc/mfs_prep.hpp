@@ -70,7 +70,7 @@ struct SweepLayout {
     // most kDirectLevelChunks the one that this dependency itself waits for
     // last)}
     lvec<int> crec;
-    lvec<int> rep;                      // per position: the dependency expected to be published last
+    lvec<int> batch_wait;               // the last of these for a batch (kBatchDirectLevelChunks)
     lvec<int> tile_chunk;               // ntile+1: first entry of each tile in pos
     lvec<int> pos;                      // positions by tile, in the sweep's level order within the tile
 };
@@ -143,9 +143,9 @@ constexpr int kThinCells = 12;
 // 2048: 262k hexahedra FP64 0.653 / 0.640 / 0.630 / 0.630, 195k prisms mixed
 // 0.456 / 0.445 / 0.440 / 0.437, 1.3M tetrahedra FP64 0.963 / 0.955 / 0.947 /
 // 0.951, 6.0M 2.90 / 2.88 / 2.86 / 2.87.  A batch interleaves its solves'
-// levels and waits on the latest dependency on all (12 mixed solves of 2.3M
-// cells: 1.167 / 1.175 / 1.190 / 1.198).
-constexpr int kDirectLevelChunks = 1024;
+// levels, so more waves poll at once there and the line lies lower (12 mixed
+// solves of 2.3M cells: 1.236 with 0, then 1.167 / 1.175 / 1.190 / 1.198).
+constexpr int kDirectLevelChunks = 1024, kBatchDirectLevelChunks = 64;
 constexpr int kMinTailChunks = 256;  // shorter tails stay with the wide levels
 constexpr int kThinChunkFlag = 0x10000;
 

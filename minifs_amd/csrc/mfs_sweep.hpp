@@ -168,7 +168,7 @@ template <typename R>
 struct SweepDir {
     int nchunks;
     const int4* crec;                       // per position: first cell, cells | deps << 8 | flag, first dep, wait
-    const int* rep;                         // per position: the latest dependency (a batch waits on it)
+    const int* batch_wait;                  // per position: the dependency a batch waits on
     const int* dnb;                         // per dependency: the neighbour
     const typename Real<R>::vec4* dgeo;     // per dependency: normal away from the cell + area
     const int* tile_chunk;                  // tiles schedule: first entry of each tile in pos
@@ -262,7 +262,7 @@ __device__ __forceinline__ void limit_dq(bool skip, const R (&q)[5], R (&DQ)[5],
 }
 
 // What a launch's chunks are: all treated as wide, all thin (the thin tail),
-// each by its flag, or a batch's (wide, waiting on the latest dependency).
+// each by its flag, or a batch's (wide, with waits of their own).
 constexpr int kWideChunks = 0, kThinChunks = 1, kAnyChunks = 2, kBatchChunks = 3;
 
 // A record that no kernel writes, at an index that every lane shares: read
@@ -301,7 +301,7 @@ __device__ __forceinline__ bool sweep_chunk(const SweepArgs<R>& A, const FlowCon
     R* const poll = FWD ? A.dqf : A.dqb;
     const int4 rec = load_record(S.crec, u);
     const int c0 = rec.x, nc = rec.y & 0xff, nd = (rec.y >> 8) & 0xff;
-    const int rep = KIND == kBatchChunks ? load_record(S.rep, u) : rec.w;
+    const int rep = KIND == kBatchChunks ? load_record(S.batch_wait, u) : rec.w;
     // a thin level: every lane polls its own dependency (a batch interleaves
     // many solves, so no level of one solve is thin there)
     const bool thin = KIND == kThinChunks || (KIND == kAnyChunks && (rec.y & kThinChunkFlag) != 0);
