@@ -465,54 +465,7 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
     }
 }
 
-// Residual, local time step and LU-SGS diagonal in one pass over a cell's
-// faces, for the fused iteration: the arithmetic of k_flux<false> and
-// k_timestep<true>, which both read the state at the start of the
-// iteration.  The cell's own state is loaded once and only the neighbour's
-// is gathered per face.  With MIXED the FP32 inputs of the implicit
-// operator (state snapshot, Diag) are written as well.
-template <int MAXF, bool MIXED>
-__device__ __forceinline__ void flux_ts_body(int c, int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                             const int2* __restrict__ fcell, const double4* __restrict__ fgeo,
-                                             const double2* __restrict__ fdn, const double* __restrict__ q,
-                                             const double* __restrict__ vol, double* __restrict__ res,
-                                             double* __restrict__ dt, double* __restrict__ diag,
-                                             double* __restrict__ pblk, int pstride, const FlowConst& K, double cfl,
-                                             double cfl_min, float* __restrict__ q32, float* __restrict__ diag32) {
-    double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    double vmin = kBIGd, vmax = 0.0;
-    if (c < nC) {
-        double qc[5];
-        load5(q + (size_t)c * 5, qc);
-        int fs[MAXF];
-        const int nf = cell_faces<MAXF>(cfo, cf, c, fs);
-        int oth[MAXF];
-        double4 g[MAXF];
-        double dnv[MAXF];
-        bool first[MAXF];
-#pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            const int2 cc = fcell[fs[s]];
-            const double2 d = fdn[fs[s]];
-            g[s] = fgeo[fs[s]];
-            first[s] = (cc.x == c);  // c is the face's c1
-            oth[s] = first[s] ? cc.y : cc.x;
-            dnv[s] = first[s] ? d.x : d.y;
-        }
-        double dtc;
-        flux_ts_cell<MAXF, MIXED>(c, qc, nf, oth, g, dnv, first, q, vol, res, dt, diag, K, cfl, cfl_min, q32, diag32,
-                                  r, dtc);
-        vmin = dtc;
-        vmax = dtc;
-    }
-    double s2[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) s2[j] = r[j] * r[j];
-    block_sum<5>(s2, pblk, pstride);
-    block_minmax(vmin, vmax, pblk + (size_t)5 * pstride, pblk + (size_t)6 * pstride);
-}
-
-// The same from the per-slot tables laid out by cell (neighbour, normal
+// The pass from the per-slot tables laid out by cell (neighbour, normal
 // pointing away from the cell with its area, this side's distance, and the
 // slots whose face has this cell second): contiguous reads, then the
 // neighbours' states.  The stored normal is the slot normal negated back
@@ -570,19 +523,6 @@ __global__ __launch_bounds__(kBlock) void k_flux_ts_slot(int nC, const int* __re
                                                          float* __restrict__ q32, float* __restrict__ diag32) {
     flux_ts_slot_body<LPC, MIXED>(xcd_block() * kBlock + (int)threadIdx.x, nC, snb, sgeo, sdn, sflip, q, vol, res,
                                   dt, diag, part + blockIdx.x, (int)gridDim.x, K, cfl, cfl_min, q32, diag32);
-}
-
-template <int MAXF, bool MIXED>
-__global__ __launch_bounds__(kBlock) void k_flux_ts(int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                                    const int2* __restrict__ fcell, const double4* __restrict__ fgeo,
-                                                    const double2* __restrict__ fdn, const double* __restrict__ q,
-                                                    const double* __restrict__ vol, double* __restrict__ res,
-                                                    double* __restrict__ dt, double* __restrict__ diag,
-                                                    double* __restrict__ part, FlowConst K, double cfl,
-                                                    double cfl_min, float* __restrict__ q32,
-                                                    float* __restrict__ diag32) {
-    flux_ts_body<MAXF, MIXED>(xcd_block() * kBlock + (int)threadIdx.x, nC, cfo, cf, fcell, fgeo, fdn, q, vol, res, dt,
-                              diag, part + blockIdx.x, (int)gridDim.x, K, cfl, cfl_min, q32, diag32);
 }
 
 // Diag alone (forward_lusgs.cpp:94-99 + CalDiagLUSGS :554-595), from dt.
