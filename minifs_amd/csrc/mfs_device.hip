@@ -703,18 +703,25 @@ bool launch_timestep(mfs_ctx* ctx, bool with_diag, double cfl, double cfl_min) {
                           : launch_timestep_t<6>(ctx, with_diag, cfl, cfl_min);
 }
 
+// Whether mfs_step's residual pass ends with its reduction (timing every
+// kernel group keeps them apart, and so does the pass that the previous
+// gradient launch carries).
+bool inline_reduce(const mfs_ctx* ctx) { return ctx->nblk_cell <= dev::kInlineReduceBlocks && ctx->timing != 1; }
+
 template <int MAXF>
 bool launch_flux_ts_t(mfs_ctx* ctx, double cfl, double cfl_min) {
     Timed t(ctx, "flux_ts");
     constexpr int LPC = MAXF == 4 ? 4 : 8;  // slots per cell of the slot tables
+    const dev::InlineReduce I{inline_reduce(ctx) ? ctx->err + 1 : nullptr, ctx->run, ctx->hist, ctx->hist_n,
+                              ctx->P.ratio_dtmax};
     if (ctx->precision == MFS_MIXED)
         hipLaunchKernelGGL((dev::k_flux_ts_slot<LPC, true>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream,
                            ctx->nC, ctx->snb, ctx->sgeo, ctx->sdn, ctx->sflip, ctx->q[ctx->cur], ctx->vol, ctx->res,
-                           ctx->dt, ctx->diag, ctx->part, ctx->K, cfl, cfl_min, ctx->q32, ctx->diag32);
+                           ctx->dt, ctx->diag, ctx->part, ctx->K, cfl, cfl_min, ctx->q32, ctx->diag32, I);
     else
         hipLaunchKernelGGL((dev::k_flux_ts_slot<LPC, false>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream,
                            ctx->nC, ctx->snb, ctx->sgeo, ctx->sdn, ctx->sflip, ctx->q[ctx->cur], ctx->vol, ctx->res,
-                           ctx->dt, ctx->diag, ctx->part, ctx->K, cfl, cfl_min, nullptr, nullptr);
+                           ctx->dt, ctx->diag, ctx->part, ctx->K, cfl, cfl_min, nullptr, nullptr, I);
     return check_launch(ctx, "k_flux_ts_slot");
 }
 bool launch_flux_ts(mfs_ctx* ctx, double cfl, double cfl_min) {
@@ -1607,9 +1614,10 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
         // diagonal, in one pass over the faces (res written from zero);
         // after the first iteration the previous gradient launch did it
         // when fused.
-        if ((s == 0 || !fuse) && !launch_flux_ts(ctx, cfl, cfl_min)) return MFS_ERR_HIP;
+        const bool own_pass = s == 0 || !fuse;
+        if (own_pass && !launch_flux_ts(ctx, cfl, cfl_min)) return MFS_ERR_HIP;
         if (side && mode == 3 && !side_gradient(ctx->sdone)) return MFS_ERR_HIP;
-        if (!launch_reduce(ctx, 1 | 2 | 4, ctx->hist_n)) return MFS_ERR_HIP;
+        if (!(own_pass && inline_reduce(ctx)) && !launch_reduce(ctx, 1 | 2 | 4, ctx->hist_n)) return MFS_ERR_HIP;
         if (!launch_diag(ctx, true)) return MFS_ERR_HIP;  // acts only when the ratio_dtmax clamp triggers
         // The backward sweep writes the state buffer that the gradient of
         // two iterations back reads.  (Waiting between the forward sweep's

@@ -33,6 +33,13 @@ struct Real<float> {
     static constexpr float kMost = 3.4028235e38f;
 };
 
+// A value that the last block of the same launch reads (write-through, where
+// a plain store may stay in the XCD's L2).
+__device__ __forceinline__ void st_part(double* p, double v) {
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(p), __builtin_bit_cast(unsigned long long, v),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <int NV, int NW = kBlock / 64>
 __device__ __forceinline__ void block_sum(double (&v)[NV], double* out, int stride = 1) {
     __shared__ double s[NW][NV];
@@ -508,21 +515,13 @@ __device__ __forceinline__ void flux_ts_slot_body(int c, int nC, const int* __re
     double s2[5];
 #pragma unroll
     for (int j = 0; j < 5; ++j) s2[j] = r[j] * r[j];
-    block_sum<5>(s2, pblk, pstride);
-    block_minmax(vmin, vmax, pblk + (size_t)5 * pstride, pblk + (size_t)6 * pstride);
-}
-
-template <int LPC, bool MIXED>
-__global__ __launch_bounds__(kBlock) void k_flux_ts_slot(int nC, const int* __restrict__ snb,
-                                                         const double4* __restrict__ sgeo,
-                                                         const double* __restrict__ sdn, const int* __restrict__ sflip,
-                                                         const double* __restrict__ q, const double* __restrict__ vol,
-                                                         double* __restrict__ res, double* __restrict__ dt,
-                                                         double* __restrict__ diag, double* __restrict__ part,
-                                                         FlowConst K, double cfl, double cfl_min,
-                                                         float* __restrict__ q32, float* __restrict__ diag32) {
-    flux_ts_slot_body<LPC, MIXED>(xcd_block() * kBlock + (int)threadIdx.x, nC, snb, sgeo, sdn, sflip, q, vol, res,
-                                  dt, diag, part + blockIdx.x, (int)gridDim.x, K, cfl, cfl_min, q32, diag32);
+    __shared__ double tot[7];
+    block_sum<5>(s2, tot);
+    block_minmax(vmin, vmax, tot + 5, tot + 6);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int j = 0; j < 7; ++j) st_part(pblk + (size_t)j * pstride, tot[j]);
+    }
 }
 
 // Diag alone (forward_lusgs.cpp:94-99 + CalDiagLUSGS :554-595), from dt.
@@ -679,6 +678,100 @@ __device__ __forceinline__ void reduce_body(int nblk, const double* __restrict__
 __global__ __launch_bounds__(kReduceBlock) void k_reduce(int nblk, const double* __restrict__ part, double* __restrict__ run,
                                                    double* __restrict__ hist, int slot, int mode, double ratio_dtmax) {
     reduce_body(nblk, part, run, hist, slot, mode, ratio_dtmax);
+}
+
+// The same reduction by the last block of the pass that writes the partials,
+// for up to kInlineReduceBlocks of them: no launch of its own (k_reduce takes
+// 8 us on a mesh of a few blocks, most of it start and a serial tree of 16
+// waves' sums).  Thread t stands for threads t, t + 256, ... of k_reduce, so
+// the sums are k_reduce's.  Each block counts itself in `counter` after its
+// partials are written through; the last one sets it back to zero.
+// ms per iteration, launch of its own -> here: 1k cells 0.0885 -> 0.083, 20k
+// 0.198 -> 0.192, 94k (368 blocks) 0.309 -> 0.306; with 768 and 1024 blocks,
+// whose partials the one block of 256 threads reads in eight round trips,
+// both take the same (0.443 | 0.442 and 0.634 | 0.632), hence the line.
+constexpr int kInlineReduceBlocks = 512;
+struct InlineReduce {
+    int* counter;  // null: no reduction here
+    double *run, *hist;
+    int slot;
+    double ratio_dtmax;
+};
+__device__ __forceinline__ double ld_part(const double* p) {
+    return __builtin_bit_cast(double, __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p),
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+__device__ __forceinline__ void reduce_last_block(int nblk, const double* part, const InlineReduce& I) {
+    __shared__ int last;
+    if (threadIdx.x == 0) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this thread's partials are written
+        last = __hip_atomic_fetch_add(I.counter, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == nblk - 1;
+    }
+    __syncthreads();
+    if (!last) return;
+    constexpr int NW = kReduceBlock / 64, P = kReduceBlock / kBlock;
+    __shared__ double wave[NW][7];
+    const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x / 64;
+    if (threadIdx.x == 0) __hip_atomic_store(I.counter, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int groups = min(P, (nblk + kBlock - 1) / kBlock);  // of 256 threads of k_reduce with records
+    for (int g = 0; g < groups; ++g) {
+        double v[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        double a = kBIGd, b = 0.0;
+        for (int k = g * kBlock + (int)threadIdx.x; k < nblk; k += kReduceBlock) {
+            double r[7];
+#pragma unroll
+            for (int j = 0; j < 7; ++j) r[j] = ld_part(part + (size_t)j * nblk + k);
+#pragma unroll
+            for (int j = 0; j < 5; ++j) v[j] += r[j];
+            a = smin(a, r[5]);
+            b = smax(b, r[6]);
+        }
+#pragma unroll
+        for (int off = 32; off >= 1; off >>= 1) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) v[j] += __shfl_down(v[j], off, 64);
+            a = smin(a, __shfl_down(a, off, 64));
+            b = smax(b, __shfl_down(b, off, 64));
+        }
+        if (lane == 0) {
+            double* const o = wave[g * (kBlock / 64) + w];
+#pragma unroll
+            for (int j = 0; j < 5; ++j) o[j] = v[j];
+            o[5] = a;
+            o[6] = b;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 7) {  // one value each, over the waves that had records
+        const int j = (int)threadIdx.x, waves = groups * (kBlock / 64);
+        double x = wave[0][j];
+        for (int k = 1; k < waves; ++k) {
+            const double y = wave[k][j];
+            x = j < 5 ? x + y : j == 5 ? smin(x, y) : smax(x, y);
+        }
+        double out = x;
+        if (j < 5) out = I.run[3 + j] = sqrt(x);
+        if (j == 5) out = I.run[1] = smin(I.run[1], x);
+        if (j == 6) out = I.run[0] = smax(I.run[0], x);
+        wave[0][j] = out;  // the wave's lanes run together: every read of this word is done
+        I.hist[(size_t)I.slot * 7 + (j < 5 ? j : j == 5 ? 6 : 5)] = out;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) I.run[2] = (wave[0][6] / wave[0][5] > I.ratio_dtmax) ? 1.0 : 0.0;
+}
+
+template <int LPC, bool MIXED>
+__global__ __launch_bounds__(kBlock) void k_flux_ts_slot(int nC, const int* __restrict__ snb,
+                                                         const double4* __restrict__ sgeo,
+                                                         const double* __restrict__ sdn, const int* __restrict__ sflip,
+                                                         const double* __restrict__ q, const double* __restrict__ vol,
+                                                         double* __restrict__ res, double* __restrict__ dt,
+                                                         double* __restrict__ diag, double* part, FlowConst K,
+                                                         double cfl, double cfl_min, float* __restrict__ q32,
+                                                         float* __restrict__ diag32, InlineReduce I) {
+    flux_ts_slot_body<LPC, MIXED>(xcd_block() * kBlock + (int)threadIdx.x, nC, snb, sgeo, sdn, sflip, q, vol, res,
+                                  dt, diag, part + blockIdx.x, (int)gridDim.x, K, cfl, cfl_min, q32, diag32);
+    if (I.counter) reduce_last_block((int)gridDim.x, part, I);
 }
 
 // The same reduction in two launches, for many blocks.  One workgroup

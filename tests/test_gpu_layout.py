@@ -117,3 +117,30 @@ def test_limiter_paths_bitwise(tmp_path, n, amp, opts):
         x.close()
     o.close()
     g.close()
+
+
+@pytest.mark.parametrize("cells,dims", [("tet", (1, 1, 1)), ("hex", (3, 2, 4)), ("hex", (8, 8, 33)),
+                                        ("tet", (22, 23, 22)), ("hex", (63, 65, 32)), ("hex", (64, 65, 32))])
+@pytest.mark.parametrize("mixed", [False, True])
+def test_history_of_the_residual_pass_and_of_its_own_launch(cells, dims, mixed):
+    """Up to 512 blocks of 256 cells, the residual pass's last block sums the
+    norms and the time step range; above, and with each kernel group timed, a
+    launch of its own does.  Both give the same history, bit for bit: meshes
+    of one block, with an odd last block, more than 256 blocks, 512 blocks
+    and more."""
+    print(f"[layout] history {cells} {dims} mixed={mixed}", flush=True)
+    out = []
+    for level in (0, 1):
+        g = mfs.Grid.box_bump(*dims, seed=3, cells=cells).decouple(2, 512)
+        p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0, ratio_dtmax=1.5)
+        g.preprocess(p)
+        s = mfs.Solver(g, p, precision=mfs.MFS_MIXED if mixed else mfs.MFS_FP64)
+        s.enable_timing(level)
+        s.step(2)
+        s.step(3)
+        out.append((s.history(), s.field("rho"), s.field("dt")))
+        s.close()
+        g.close()
+    assert out[0][0].shape == (5, 7) and np.isfinite(out[0][0]).all()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
