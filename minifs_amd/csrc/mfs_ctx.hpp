@@ -92,7 +92,7 @@ struct mfs_ctx {
     } sweep[2];
     unsigned short* cdep = nullptr;  // per cell and direction: first dependency in the chunk, count
     int* snb = nullptr;         // lpc per device cell: neighbour across the slot's face
-    double4* sgeo = nullptr;    // lpc per device cell: normal away from the cell, area
+    double4* sgeo = nullptr;    // per slot and device cell: normal away from the cell, area
     float4* sgeo32 = nullptr;   // the same in FP32 (mixed precision)
     int sweep_by_tiles = 0;
     int ntiles = 0;
@@ -101,7 +101,7 @@ struct mfs_ctx {
     int* gface = nullptr;    // nB: device face of each ghost cell nC+k
     int4* cnode = nullptr;   // tetrahedral meshes: the cells' nodes and the gradient's choices (k_tet_tables)
     unsigned short* gsel = nullptr;
-    double* sdn = nullptr;   // per slot: |(x_fc - x_cc).n| on this cell's side
+    double* sdn = nullptr;   // per slot and cell: |(x_fc - x_cc).n| on this cell's side
     int* sflip = nullptr;    // per cell: slots whose face has this cell second (bits 0-7), face count (8-11)
     int ghost_refresh = 0;   // SetGhostVariables after each update in mfs_step
     // mfs_step's gradient on a second stream (gradient_stream options 2-5):

@@ -1313,6 +1313,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     ok = ok && dalloc(ctx, ctx->sym_node, L.sym_node.size(), "sym_node") &&
          dalloc(ctx, ctx->sym_n, L.sym_n.size(), "sym_n");
     const bool mixed = precision == MFS_MIXED;
+    const size_t nslot = (size_t)(L.lpc == 4 ? dev::kSlots<4> : dev::kSlots<8>) * L.nC;
     for (int d = 0; d < 2; ++d) {
         mfs_ctx::Sweep& S = ctx->sweep[d];
         const SweepLayout& H = L.sweep[d];
@@ -1329,14 +1330,14 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
          dalloc(ctx, ctx->dev_of_node, (size_t)L.nN, "node map");
     ok = ok && dalloc(ctx, ctx->cdep, L.cdep.size(), "cell dependencies") &&
          dalloc(ctx, ctx->snb, L.cfs.size(), "slot neighbours") &&
-         dalloc(ctx, ctx->sgeo, L.cfs.size(), "slot geometry") && dalloc(ctx, ctx->depmask, L.nC, "depmask");
+         dalloc(ctx, ctx->sgeo, nslot, "slot geometry") && dalloc(ctx, ctx->depmask, L.nC, "depmask");
     if (mixed) {
         ok = ok && dalloc(ctx, ctx->q32, 5 * n, "q32") && dalloc(ctx, ctx->diag32, L.nC, "diag32") &&
              dalloc(ctx, ctx->dqf32, 5 * (size_t)L.nC, "dq_forward32") && dalloc(ctx, ctx->dq32, 5 * n, "dq32") &&
              dalloc(ctx, ctx->gx32, 5 * n, "dqdx32") && dalloc(ctx, ctx->gy32, 5 * n, "dqdy32") &&
              dalloc(ctx, ctx->gz32, 5 * n, "dqdz32") && dalloc(ctx, ctx->qn32, 5 * (size_t)L.nN, "qnode32") &&
              dalloc(ctx, ctx->ell_w32, ell_w.size(), "ell_w32") && dalloc(ctx, ctx->fgeo32, L.nF, "fgeo32") &&
-             dalloc(ctx, ctx->sgeo32, L.cfs.size(), "slot geometry (FP32)");
+             dalloc(ctx, ctx->sgeo32, nslot, "slot geometry (FP32)");
     }
     ok = ok && dalloc(ctx, ctx->part, partial_doubles((int)ctx->nblk_cell), "partials") && dalloc(ctx, ctx->run, 8, "run") &&
          dalloc(ctx, ctx->err, 4, "err") &&
@@ -1345,7 +1346,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     if (L.tri_slots)
         ok = ok && dalloc(ctx, ctx->cnode, (size_t)L.nC, "cell nodes") &&
              dalloc(ctx, ctx->gsel, (size_t)L.nC, "gradient choices");
-    ok = ok && dalloc(ctx, ctx->sdn, L.cfs.size(), "slot distances") && dalloc(ctx, ctx->sflip, L.nC, "slot sides");
+    ok = ok && dalloc(ctx, ctx->sdn, nslot, "slot distances") && dalloc(ctx, ctx->sflip, L.nC, "slot sides");
     ok = ok && ensure_hist(ctx, 64);
     // per-device set-up: the sweep order's event and the address of the
     // static scratch of mfs_step_noalloc on this device
@@ -1422,7 +1423,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                 for (int d = 0; d < 2 && ok; ++d) {
                     const mfs_ctx::Sweep& S = ctx->sweep[d];
                     hipLaunchKernelGGL(dep, dim3(nblk((size_t)S.nchunk, kBlock / 64)), dim3(kBlock), 0, ctx->stream,
-                                       S.nchunk, S.crec, ctx->cdep, d, ctx->depmask, ctx->snb, ctx->sgeo, S.dnb,
+                                       L.nC, S.nchunk, S.crec, ctx->cdep, d, ctx->depmask, ctx->snb, ctx->sgeo, S.dnb,
                                        S.dgeo, S.dgeo32);
                     ok = check_launch(ctx, "k_dep_tables");
                 }

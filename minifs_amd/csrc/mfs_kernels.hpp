@@ -398,6 +398,18 @@ __global__ __launch_bounds__(kBlock) void k_timestep(int nC, const int* __restri
     block_minmax(vmin, vmax, part + (size_t)5 * gridDim.x + blockIdx.x, part + (size_t)6 * gridDim.x + blockIdx.x);
 }
 
+// Slots of a cell that can hold a face, of the LPC its neighbour and face
+// rows have room for, and the place of slot s of cell c in the slot geometry
+// and distances: slot by slot, so that a wave's load of one slot's 32 bytes a
+// cell spans 16 lines.  Stored cell by cell, every lane's load was in a line
+// of its own, and the CU's cache takes a cycle or more per line.
+// Before and after (residual pass, gradient): 6.0M tetrahedra FP64 565 -> 513
+// and 440 -> 397 us, 1.3M 128 -> 117 and 2.9M mixed 297 -> 276 us (residual);
+// 262k hexahedra, whose pass also took the two empty slots along, 47 -> 39 us.
+template <int LPC>
+constexpr int kSlots = LPC == 4 ? 4 : 6;
+__device__ __forceinline__ size_t slot_at(int s, int c, int nC) { return (size_t)s * nC + c; }
+
 // Residual, local time step and LU-SGS diagonal in one pass over a cell's
 // faces, for the fused iteration: the arithmetic of k_flux<false> and
 // k_timestep<true>, which both read the state at the start of the
@@ -486,6 +498,7 @@ __device__ __forceinline__ void flux_ts_slot_body(int c, int nC, const int* __re
                                                   double* __restrict__ pblk, int pstride, const FlowConst& K, double cfl,
                                                   double cfl_min, float* __restrict__ q32,
                                                   float* __restrict__ diag32) {
+    constexpr int NS = kSlots<LPC>;
     double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double vmin = kBIGd, vmax = 0.0;
     if (c < nC) {
@@ -493,21 +506,21 @@ __device__ __forceinline__ void flux_ts_slot_body(int c, int nC, const int* __re
         load5(q + (size_t)c * 5, qc);
         const unsigned sf = (unsigned)sflip[c];
         const int nf = (int)((sf >> 8) & 15u);
-        int oth[LPC];
-        double4 g[LPC];
-        double dnv[LPC];
-        bool first[LPC];
+        int oth[NS];
+        double4 g[NS];
+        double dnv[NS];
+        bool first[NS];
 #pragma unroll
-        for (int s = 0; s < LPC; ++s) {
-            const size_t i = (size_t)c * LPC + s;
+        for (int s = 0; s < NS; ++s) {
+            const size_t i = slot_at(s, c, nC);
             const double4 v = sgeo[i];
             first[s] = ((sf >> s) & 1u) == 0;
             g[s] = first[s] ? v : make_double4(-v.x, -v.y, -v.z, v.w);
-            oth[s] = snb[i];
+            oth[s] = snb[(size_t)c * LPC + s];
             dnv[s] = sdn[i];
         }
         double dtc;
-        flux_ts_cell<LPC, MIXED>(c, qc, nf, oth, g, dnv, first, q, vol, res, dt, diag, K, cfl, cfl_min, q32, diag32,
+        flux_ts_cell<NS, MIXED>(c, qc, nf, oth, g, dnv, first, q, vol, res, dt, diag, K, cfl, cfl_min, q32, diag32,
                                  r, dtc);
         vmin = dtc;
         vmax = dtc;
@@ -1045,7 +1058,8 @@ __device__ __forceinline__ void grad_body(int c, int nC, int n, const int* __res
 // of two bits, taken by selects (a + b commutes; a leading 0 + would only turn
 // a sum of negative zeros positive, which the accumulators do anyway).
 // Measured alone, before and after: 6.0M cells FP64 650 -> 440 us (1.8 GB of
-// compulsory reads and writes, 4.1 TB/s), 2.9M cells FP32 215 -> 134 us.
+// compulsory reads and writes, 4.1 TB/s), 2.9M cells FP32 215 -> 134 us; with
+// the slot geometry stored slot by slot (slot_at) 397 us, 4.5 TB/s.
 template <typename R>
 __device__ __forceinline__ void grad_tet_body(int c, int nC, int n, const int* __restrict__ snb,
                                               const typename Real<R>::vec4* __restrict__ sgeo,
@@ -1058,7 +1072,7 @@ __device__ __forceinline__ void grad_tet_body(int c, int nC, int n, const int* _
     const unsigned sel = gsel[c];
     typename Real<R>::vec4 g[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) g[s] = sgeo[(size_t)c * 4 + s];
+    for (int s = 0; s < 4; ++s) g[s] = sgeo[slot_at(s, c, nC)];
     R v[4][5];
     load5r(qn + (size_t)nd.x * 5, v[0]);
     load5r(qn + (size_t)nd.y * 5, v[1]);

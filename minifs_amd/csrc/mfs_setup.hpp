@@ -344,11 +344,13 @@ __global__ __launch_bounds__(kBlock) void k_slot_tables(int nC, const int* __res
     for (int sl = 0; sl < LPC; ++sl) {
         const size_t i = (size_t)d * LPC + sl;
         const int f = cfs[i];
+        const size_t ig = slot_at(sl, d, nC);
         if (f < 0) {
             snb[i] = d;
-            sgeo[i] = make_double4(0.0, 0.0, 0.0, 0.0);
-            if (sgeo32) sgeo32[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            sdn[i] = 0.0;
+            if (sl >= kSlots<LPC>) continue;
+            sgeo[ig] = make_double4(0.0, 0.0, 0.0, 0.0);
+            if (sgeo32) sgeo32[ig] = make_float4(0.f, 0.f, 0.f, 0.f);
+            sdn[ig] = 0.0;
             continue;
         }
         const int2 cc = fcell[f];
@@ -357,10 +359,10 @@ __global__ __launch_bounds__(kBlock) void k_slot_tables(int nC, const int* __res
         const double4 g = fgeo[f];
         const double4 o = flip ? make_double4(-g.x, -g.y, -g.z, g.w) : g;
         snb[i] = flip ? cc.x : cc.y;
-        sgeo[i] = o;
-        if (sgeo32) sgeo32[i] = make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w);
+        sgeo[ig] = o;
+        if (sgeo32) sgeo32[ig] = make_float4((float)o.x, (float)o.y, (float)o.z, (float)o.w);
         const double2 dn = fdn[f];
-        sdn[i] = flip ? dn.y : dn.x;
+        sdn[ig] = flip ? dn.y : dn.x;
     }
     sflip[d] = flips;
 }
@@ -416,7 +418,7 @@ __global__ __launch_bounds__(kBlock) void k_tet_tables(int nC, const int* __rest
 // from the slot tables.  One wave per chunk, one lane per cell; mask_shift
 // selects the direction's slots in depmask (0 forward, 8 backward).
 template <int LPC>
-__global__ __launch_bounds__(kBlock) void k_dep_tables(int nchunk, const int4* __restrict__ crec,
+__global__ __launch_bounds__(kBlock) void k_dep_tables(int nC, int nchunk, const int4* __restrict__ crec,
                                                       const unsigned short* __restrict__ cdep, int dir,
                                                       const int* __restrict__ depmask, const int* __restrict__ snb,
                                                       const double4* __restrict__ sgeo, int* __restrict__ dnb,
@@ -428,11 +430,10 @@ __global__ __launch_bounds__(kBlock) void k_dep_tables(int nchunk, const int4* _
     const int c = rec.x + lane;
     const unsigned m = ((unsigned)depmask[c] >> (8 * dir)) & 0xffu;
     size_t k = (size_t)rec.z + (cdep[2 * (size_t)c + dir] & 0xffu);
-    for (int s = 0; s < LPC; ++s) {
+    for (int s = 0; s < kSlots<LPC>; ++s) {
         if (!((m >> s) & 1u)) continue;
-        const size_t i = (size_t)c * LPC + s;
-        const double4 g = sgeo[i];
-        dnb[k] = snb[i];
+        const double4 g = sgeo[slot_at(s, c, nC)];
+        dnb[k] = snb[(size_t)c * LPC + s];
         if (dgeo) dgeo[k] = g;
         if (dgeo32) dgeo32[k] = make_float4((float)g.x, (float)g.y, (float)g.z, (float)g.w);
         ++k;
