@@ -416,6 +416,13 @@ __device__ __forceinline__ size_t slot_at(int s, int c, int nC) { return (size_t
 // iteration.  The cell's own state is loaded once and only the neighbour's
 // is gathered per face.  With MIXED the FP32 inputs of the implicit
 // operator (state snapshot, Diag) are written as well.
+// The pass is near its bytes (6.0M cells FP64: 1.84 GB, 367 us at the rate of
+// a copy, 513 us taken) with 316 us of FP64 arithmetic beside them, so the
+// cell's own enthalpy and its quotient are formed once instead of at every
+// face and the pressure jump is decided without a division where it can be:
+// 10% fewer instructions, 6.0M 513 -> 491 us, 2.9M mixed 276 -> 265 us.  (Four
+// waves a SIMD instead of three: spills, 6.0M 5% slower iterations.  One lane
+// per face instead of per cell: 6.0M 538 -> 567, 262k hexahedra 47 -> 75 us.)
 // Per cell: the faces' fluxes added in slot order (the cell's ascending
 // face order), the time step from the smallest dn/eig, the CFL choice and
 // the diagonal.  NS slots, the first nf used; oth = the face's other cell,
@@ -430,6 +437,7 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
                                              double& dtc) {
     const double c2tmp = K.gam * (qc[4] + K.p_bar) / qc[0];
     const double a = sqrt(c2tmp);
+    const double hc = total_enthalpy(qc, K.gamm1, K.p_bar), hqc = hc / qc[0];
     dtc = kBIGd;
     int det = 1;
     double eig[NS];
@@ -442,11 +450,17 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
             ql[j] = first[s] ? qc[j] : qo[j];
             qr[j] = first[s] ? qo[j] : qc[j];
         }
-        roe_flux<double>(ql, qr, g[s].x, g[s].y, g[s].z, g[s].w, K.gamm1, K.p_bar, K.alf_l, kTINYd, F);
+        const double ho = total_enthalpy(qo, K.gamm1, K.p_bar), hqo = ho / qo[0];
+        roe_flux<double>(ql, qr, first[s] ? hc : ho, first[s] ? ho : hc, first[s] ? hqc : hqo, first[s] ? hqo : hqc,
+                         g[s].x, g[s].y, g[s].z, g[s].w, K.gamm1, K.alf_l, kTINYd, F);
         double vn = qc[1] * g[s].x + qc[2] * g[s].y + qc[3] * g[s].z;
         vn = fabs(vn);
         eig[s] = vn + a;
-        const double dp = fabs(qr[4] - ql[4]) / (qr[4] + ql[4] + K.p_bar + K.p_bar);
+        // dp > 0.1 without the division where no lane of the wave is near it:
+        // at most 0.0999 of a positive sum, the rounded quotient is below 0.1
+        const double pd = fabs(qr[4] - ql[4]), ps = qr[4] + ql[4] + K.p_bar + K.p_bar;
+        bool jump = !((pd <= 0.0999 * ps) & (ps > 1e-280));
+        if (__builtin_amdgcn_ballot_w64(jump) != 0) jump = pd / ps > 0.1;
         if (s < nf) {
             if (first[s]) {
 #pragma unroll
@@ -456,7 +470,7 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
                 for (int j = 0; j < 5; ++j) r[j] += F[j];
             }
             dtc = smin(dtc, dnv[s] / eig[s]);
-            if (dp > 0.1) det = 0;
+            if (jump) det = 0;
         }
     }
 #pragma unroll

@@ -28,14 +28,17 @@ struct FlowConst {
 };
 
 // RoeFlux_noprec live loop body (src/Kernels/cal_flux.cpp:682-833):
-// flux of face (ql -> qr) with unit normal (ax,ay,az) and area.
+// flux of face (ql -> qr) with unit normal (ax,ay,az) and area.  The total
+// enthalpy of each side (ht = rho*H) and its quotient by the density depend
+// on that side's state alone: a pass over a cell's faces forms its own once.
 template <typename R>
-MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R gamm1, R p_bar, R alf_l, R tiny,
-                     R f[5]) {
-    R et_l = (ql[4] + p_bar) / gamm1 + R(0.5) * ql[0] * (ql[1] * ql[1] + ql[2] * ql[2] + ql[3] * ql[3]);
-    R et_r = (qr[4] + p_bar) / gamm1 + R(0.5) * qr[0] * (qr[1] * qr[1] + qr[2] * qr[2] + qr[3] * qr[3]);
-    R ht_l = et_l + ql[4] + p_bar;
-    R ht_r = et_r + qr[4] + p_bar;
+MFS_HD R total_enthalpy(const R q[5], R gamm1, R p_bar) {
+    const R et = (q[4] + p_bar) / gamm1 + R(0.5) * q[0] * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+    return et + q[4] + p_bar;
+}
+template <typename R>
+MFS_HD void roe_flux(const R ql[5], const R qr[5], R ht_l, R ht_r, R hl, R hr, R ax, R ay, R az, R area, R gamm1,
+                     R alf_l, R tiny, R f[5]) {
     R vn_l = ax * ql[1] + ay * ql[2] + az * ql[3];
     R vn_r = ax * qr[1] + ay * qr[2] + az * qr[3];
     R tmp0 = vn_l * ql[0];
@@ -53,7 +56,7 @@ MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R g
     R v_a = (ql[2] + qr[2] * tmp0) * tmp1;
     R w_a = (ql[3] + qr[3] * tmp0) * tmp1;
     R vn_a = u_a * ax + v_a * ay + w_a * az;
-    R h_a = (ht_l / ql[0] + ht_r / qr[0] * tmp0) * tmp1;
+    R h_a = (hl + hr * tmp0) * tmp1;
     R q2 = R(0.5) * (u_a * u_a + v_a * v_a + w_a * w_a);
     R c2_a = gamm1 * (h_a - q2);
     c2_a = fabs(c2_a);
@@ -100,6 +103,13 @@ MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R g
     f[2] *= tmp0;
     f[3] *= tmp0;
     f[4] *= tmp0;
+}
+
+template <typename R>
+MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R gamm1, R p_bar, R alf_l, R tiny,
+                     R f[5]) {
+    const R ht_l = total_enthalpy(ql, gamm1, p_bar), ht_r = total_enthalpy(qr, gamm1, p_bar);
+    roe_flux(ql, qr, ht_l, ht_r, ht_l / ql[0], ht_r / qr[0], ax, ay, az, area, gamm1, alf_l, tiny, f);
 }
 
 // FluxLUSGS3D (src/Kernels/forward_lusgs.cpp:1271-1324): neighbour state q,

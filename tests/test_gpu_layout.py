@@ -144,3 +144,38 @@ def test_history_of_the_residual_pass_and_of_its_own_launch(cells, dims, mixed):
     assert out[0][0].shape == (5, 7) and np.isfinite(out[0][0]).all()
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("cells,dims", [("tet", (4, 3, 5)), ("hex", (7, 5, 6)), ("prism", (4, 6, 3))])
+@pytest.mark.parametrize("jump", [0.0998, 0.0999, 0.09995, 0.1, 0.1001, 0.5])
+def test_pressure_jump_test_near_its_limit(tmp_path, cells, dims, jump):
+    """The time step takes the smaller CFL where a face's pressure jump,
+    |dp| / (sum of both), exceeds 0.1; away from the limit the residual pass
+    decides that without the division.  Two pressures whose jump lies below,
+    at and above the limit (and a rounding around it), cell by cell at random:
+    bit for bit against the oracle."""
+    print(f"[layout] pressure jump {cells} {dims} {jump}", flush=True)
+    mach, alpha, cfl = 0.8, 1.25, 10.0
+    p = mfs.make_params(mach=mach, alpha=alpha, cfl=cfl)
+    g = mfs.Grid.box_bump(*dims, seed=2, cells=cells).decouple(2, 64)
+    mesh, bc = str(tmp_path / "m.mfl"), str(tmp_path / "m.bc")
+    g.save(mesh, bc)
+    n = g.info["nTCell"] + g.info["nBFace"]
+    g.preprocess(p)
+    rng = np.random.default_rng(11)
+    ratio = (1.0 + jump) / (1.0 - jump)
+    total = p.p_bar * np.where(rng.random(n) < 0.3, ratio, 1.0) * (1.0 + rng.integers(-2, 3, n) * 2.0**-52)
+    st = {"rho": np.full(n, p.rho_s), "u": np.full(n, p.u_s), "v": np.full(n, p.v_s), "w": np.full(n, p.w_s),
+          "p": total - p.p_bar}
+    o = Oracle(mesh, bc, mach, alpha, cfl)
+    s = mfs.Solver(g, p)
+    for k, a in st.items():
+        o.set(k, a)
+        s.upload(k, a)
+    o.run(1, 0)
+    s.step(1)
+    for nm in FIELDS:
+        np.testing.assert_array_equal(s.field(nm), o.get(nm), err_msg=nm)
+    s.close()
+    o.close()
+    g.close()
