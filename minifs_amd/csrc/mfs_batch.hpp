@@ -23,7 +23,6 @@ struct BatchSolve {
     const int *cfo, *cf;
     const int2* fcell;
     const double4* fgeo;
-    const double2* fdn;
     const double* vol;
     const double* q;              // state at the start of the iteration
     const double* qnew;           // state written by the backward sweep
@@ -72,14 +71,17 @@ __global__ __launch_bounds__(kReduceBlock) void k_b_reduce(const BatchSolve<R>* 
     reduce_body(S.nblk_cell, S.part, S.run, S.hist, S.hist_slot, 1 | 2 | 4, S.ratio_dtmax);
 }
 
+// The ratio_dtmax clamp, kBatchClampBlocks workgroups per solve that return
+// at once where it is off, the rule at the reference's ratio_dtmax (a
+// workgroup per 256 cells took 8.4 us of a 12-solve iteration, these 4.4).
+constexpr int kBatchClampBlocks = 64;
 template <int MAXF, typename R>
-__global__ __launch_bounds__(kBlock) void k_b_clamp(const BatchSolve<R>* __restrict__ T,
-                                                    const int* __restrict__ cell_solve) {
-    const BatchSolve<R>& S = T[cell_solve[blockIdx.x]];
-    const int lb = (int)blockIdx.x - S.blk0_cell;
-    const int lg = (lb % kXcd) * (S.nblk_cell / kXcd) + lb / kXcd;
-    diag_body<MAXF>(lg * kBlock + (int)threadIdx.x, S.nC, S.cfo, S.cf, S.fgeo, S.q, S.vol, S.dt, S.diag, S.run,
-                    S.ratio_dtmax, S.K, S.q32 ? S.diag32 : nullptr);
+__global__ __launch_bounds__(kBlock) void k_b_clamp(const BatchSolve<R>* __restrict__ T) {
+    const BatchSolve<R>& S = T[blockIdx.x / kBatchClampBlocks];
+    if (S.run[2] == 0.0) return;
+    for (int c = (int)(blockIdx.x % kBatchClampBlocks * kBlock + threadIdx.x); c < S.nC; c += kBatchClampBlocks * kBlock)
+        diag_body<MAXF == 4 ? 4 : 8>(c, S.nC, S.sgeo64, S.sflip, S.q, S.vol, S.dt, S.diag, S.run, S.ratio_dtmax, S.K,
+                                     S.q32 ? S.diag32 : nullptr);
 }
 
 template <bool FWD, int MAXD, typename R>

@@ -669,38 +669,30 @@ bool ensure_hist(mfs_ctx* ctx, int need) {
 
 // ---- launch helpers
 template <int MAXF>
-bool launch_flux_t(mfs_ctx* ctx, bool accum) {
+constexpr int lpc_of = MAXF == 4 ? 4 : 8;  // slots per cell of the slot tables
+
+template <int MAXF>
+bool launch_flux_t(mfs_ctx* ctx) {
     Timed t(ctx, "flux");
     const double* q = ctx->q[ctx->cur];
-    if (accum)
-        hipLaunchKernelGGL((dev::k_flux<true, MAXF>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC,
-                           ctx->cfo, ctx->cf, ctx->fcell, ctx->fgeo, q, ctx->res, ctx->part, ctx->K);
-    else
-        hipLaunchKernelGGL((dev::k_flux<false, MAXF>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC,
-                           ctx->cfo, ctx->cf, ctx->fcell, ctx->fgeo, q, ctx->res, ctx->part, ctx->K);
+    hipLaunchKernelGGL((dev::k_flux<lpc_of<MAXF>>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC, ctx->snb, ctx->sgeo,
+                       ctx->sflip, q, ctx->res, ctx->part, ctx->K);
     return check_launch(ctx, "k_flux");
 }
-bool launch_flux(mfs_ctx* ctx, bool accum) {
-    return ctx->maxf == 4 ? launch_flux_t<4>(ctx, accum) : launch_flux_t<6>(ctx, accum);
+bool launch_flux(mfs_ctx* ctx) {
+    return ctx->maxf == 4 ? launch_flux_t<4>(ctx) : launch_flux_t<6>(ctx);
 }
 
 template <int MAXF>
-bool launch_timestep_t(mfs_ctx* ctx, bool with_diag, double cfl, double cfl_min) {
+bool launch_timestep_t(mfs_ctx* ctx, double cfl, double cfl_min) {
     Timed t(ctx, "timestep");
     const double* q = ctx->q[ctx->cur];
-    if (with_diag)
-        hipLaunchKernelGGL((dev::k_timestep<true, MAXF>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC,
-                           ctx->cfo, ctx->cf, ctx->fcell, ctx->fgeo, ctx->fdn, q, ctx->vol, ctx->dt, ctx->diag, ctx->part,
-                           ctx->K, cfl, cfl_min);
-    else
-        hipLaunchKernelGGL((dev::k_timestep<false, MAXF>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC,
-                           ctx->cfo, ctx->cf, ctx->fcell, ctx->fgeo, ctx->fdn, q, ctx->vol, ctx->dt, ctx->diag, ctx->part,
-                           ctx->K, cfl, cfl_min);
+    hipLaunchKernelGGL((dev::k_timestep<lpc_of<MAXF>>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC, ctx->snb, ctx->sgeo,
+                       ctx->sdn, ctx->sflip, q, ctx->dt, ctx->part, ctx->K, cfl, cfl_min);
     return check_launch(ctx, "k_timestep");
 }
-bool launch_timestep(mfs_ctx* ctx, bool with_diag, double cfl, double cfl_min) {
-    return ctx->maxf == 4 ? launch_timestep_t<4>(ctx, with_diag, cfl, cfl_min)
-                          : launch_timestep_t<6>(ctx, with_diag, cfl, cfl_min);
+bool launch_timestep(mfs_ctx* ctx, double cfl, double cfl_min) {
+    return ctx->maxf == 4 ? launch_timestep_t<4>(ctx, cfl, cfl_min) : launch_timestep_t<6>(ctx, cfl, cfl_min);
 }
 
 // Whether mfs_step's residual pass ends with its reduction (timing every
@@ -711,7 +703,7 @@ bool inline_reduce(const mfs_ctx* ctx) { return ctx->nblk_cell <= dev::kInlineRe
 template <int MAXF>
 bool launch_flux_ts_t(mfs_ctx* ctx, double cfl, double cfl_min) {
     Timed t(ctx, "flux_ts");
-    constexpr int LPC = MAXF == 4 ? 4 : 8;  // slots per cell of the slot tables
+    constexpr int LPC = lpc_of<MAXF>;
     const dev::InlineReduce I{inline_reduce(ctx) ? ctx->err + 1 : nullptr, ctx->run, ctx->hist, ctx->hist_n,
                               ctx->P.ratio_dtmax};
     if (ctx->precision == MFS_MIXED)
@@ -766,12 +758,12 @@ template <int MAXF>
 bool launch_diag_t(mfs_ctx* ctx, bool clamp_only) {
     Timed t(ctx, clamp_only ? "clamp" : "diag");
     if (clamp_only)  // usually off: a small grid that returns at once
-        hipLaunchKernelGGL((dev::k_clamp<MAXF>), dim3(std::min<unsigned>(ctx->nblk_cell, dev::kClampBlocks)), dim3(kBlock),
-                           0, ctx->stream, ctx->nC, ctx->cfo, ctx->cf, ctx->fgeo, ctx->q[ctx->cur], ctx->vol, ctx->dt,
+        hipLaunchKernelGGL((dev::k_clamp<lpc_of<MAXF>>), dim3(std::min<unsigned>(ctx->nblk_cell, dev::kClampBlocks)), dim3(kBlock),
+                           0, ctx->stream, ctx->nC, ctx->sgeo, ctx->sflip, ctx->q[ctx->cur], ctx->vol, ctx->dt,
                            ctx->diag, ctx->run, ctx->P.ratio_dtmax, ctx->K, ctx->diag32);
     else
-        hipLaunchKernelGGL((dev::k_diag<MAXF>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC, ctx->cfo,
-                           ctx->cf, ctx->fgeo, ctx->q[ctx->cur], ctx->vol, ctx->dt, ctx->diag, nullptr,
+        hipLaunchKernelGGL((dev::k_diag<lpc_of<MAXF>>), dim3(ctx->nblk_cell), dim3(kBlock), 0, ctx->stream, ctx->nC, ctx->sgeo,
+                           ctx->sflip, ctx->q[ctx->cur], ctx->vol, ctx->dt, ctx->diag, nullptr,
                            ctx->P.ratio_dtmax, ctx->K, ctx->diag32);
     return check_launch(ctx, "k_diag");
 }
@@ -1521,7 +1513,7 @@ extern "C" int mfs_zero_residuals(mfs_ctx* ctx) {
 
 extern "C" int mfs_inviscid_flux(mfs_ctx* ctx) {
     if (!usable(ctx)) return MFS_ERR_STATE;
-    if (!launch_flux(ctx, true)) return MFS_ERR_HIP;
+    if (!launch_flux(ctx)) return MFS_ERR_HIP;
     return launch_reduce(ctx, 1, -1) ? MFS_OK : MFS_ERR_HIP;
 }
 
@@ -1530,7 +1522,7 @@ extern "C" int mfs_compute_timestep(mfs_ctx* ctx) {
     const double cfl = cfl_of_iter(ctx->P, ctx->iter_done);
     const double cfl_min = 0.5 * cfl;
     ctx->cfl_min = cfl_min;
-    if (!launch_timestep(ctx, false, cfl, cfl_min)) return MFS_ERR_HIP;
+    if (!launch_timestep(ctx, cfl, cfl_min)) return MFS_ERR_HIP;
     if (!launch_reduce(ctx, 2, -1)) return MFS_ERR_HIP;
     // ratio_dtmax clamp (compute_timestep.cpp:929-945)
     return launch_diag(ctx, true) ? MFS_OK : MFS_ERR_HIP;
@@ -2095,7 +2087,6 @@ void fill_entry(dev::BatchSolve<R>& E, mfs_ctx* c, int cur, int blk0_cell, int b
     E.cf = c->cf;
     E.fcell = c->fcell;
     E.fgeo = c->fgeo;
-    E.fdn = c->fdn;
     E.vol = c->vol;
     E.q = c->q[cur];
     E.qnew = c->q[1 - cur];
@@ -2250,8 +2241,8 @@ int batch_step_t(mfs_batch* b, int nsteps) {
             hipLaunchKernelGGL((dev::k_b_flux_ts<MAXF, MIXED, R>), dim3(b->ncell_blk), dim3(kBlock), 0, b->stream,
                                Tf, b->cell_solve);
         hipLaunchKernelGGL((dev::k_b_reduce<R>), dim3(ns), dim3(dev::kReduceBlock), 0, b->stream, Tf);
-        hipLaunchKernelGGL((dev::k_b_clamp<MAXF, R>), dim3(b->ncell_blk), dim3(kBlock), 0, b->stream, Tf,
-                           b->cell_solve);
+        hipLaunchKernelGGL((dev::k_b_clamp<MAXF, R>), dim3(ns * dev::kBatchClampBlocks), dim3(kBlock), 0, b->stream,
+                           Tf);
         if (!batch_ok(b, hipGetLastError(), "batch flux/time step")) return MFS_ERR_HIP;
         const int par = (int)(b->iters & 1);
         if (side && b->gpend[par]) {

@@ -273,45 +273,109 @@ __device__ __forceinline__ int cell_faces(const int* __restrict__ cfo, const int
     return nf;
 }
 
+// Slots of a cell that can hold a face, of the LPC its neighbour and face
+// rows have room for, and the place of slot s of cell c in the slot geometry
+// and distances: slot by slot, so that a wave's load of one slot's 32 bytes a
+// cell spans 16 lines.  Stored cell by cell, every lane's load was in a line
+// of its own, and the CU's cache takes a cycle or more per line.
+// Before and after (residual pass, gradient): 6.0M tetrahedra FP64 565 -> 513
+// and 440 -> 397 us, 1.3M 128 -> 117 and 2.9M mixed 297 -> 276 us (residual);
+// 262k hexahedra, whose pass also took the two empty slots along, 47 -> 39 us.
+// The separate entry points' passes read these tables too, where each face's
+// cells, normal and distances were a gather of their own (384k cells: residual
+// 36 -> 31, time step 24.5 -> 17.4, diagonal 12.8 -> 11.4 us).
+template <int LPC>
+constexpr int kSlots = LPC == 4 ? 4 : 6;
+__device__ __forceinline__ size_t slot_at(int s, int c, int nC) { return (size_t)s * nC + c; }
+
+// A cell's slots: neighbour, the face's stored normal and area, this side's
+// distance, and whether the cell is the face's first (the slot normal points
+// away from the cell; negated back where the cell is second, exactly).
+template <int NS>
+struct CellSlots {
+    int nf, oth[NS];
+    double4 g[NS];
+    double dn[NS];
+    bool first[NS];
+};
+template <int LPC, bool DN>
+__device__ __forceinline__ void load_slots(int c, int nC, const int* __restrict__ snb,
+                                           const double4* __restrict__ sgeo, const double* __restrict__ sdn,
+                                           const int* __restrict__ sflip, CellSlots<kSlots<LPC>>& L) {
+#pragma unroll
+    for (int s = 0; s < kSlots<LPC>; ++s) L.oth[s] = snb[(size_t)c * LPC + s];
+    const unsigned sf = (unsigned)sflip[c];
+    L.nf = (int)((sf >> 8) & 15u);
+#pragma unroll
+    for (int s = 0; s < kSlots<LPC>; ++s) {
+        const size_t i = slot_at(s, c, nC);
+        const double4 v = sgeo[i];
+        L.first[s] = ((sf >> s) & 1u) == 0;
+        L.g[s] = L.first[s] ? v : make_double4(-v.x, -v.y, -v.z, v.w);
+        if (DN) L.dn[s] = sdn[i];
+    }
+}
+
+// The cell's flux across one slot, added with the face's sign.  hc = the
+// cell's total enthalpy, hqc = that by its density, qo = the other state.
+__device__ __forceinline__ void add_face_flux(const double (&qc)[5], double hc, double hqc, const double (&qo)[5],
+                                              bool first, const double4& g, bool used, const FlowConst& K,
+                                              double (&r)[5]) {
+    double ql[5], qr[5], F[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        ql[j] = first ? qc[j] : qo[j];
+        qr[j] = first ? qo[j] : qc[j];
+    }
+    const double ho = total_enthalpy(qo, K.gamm1, K.p_bar), hqo = ho / qo[0];
+    roe_flux<double>(ql, qr, first ? hc : ho, first ? ho : hc, first ? hqc : hqo, first ? hqo : hqc, g.x, g.y, g.z,
+                     g.w, K.gamm1, K.alf_l, kTINYd, F);
+    if (used) {
+        if (first) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) r[j] -= F[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) r[j] += F[j];
+        }
+    }
+}
+
+// CellIsMG's test of one face: |dp| / (sum of both total pressures) > 0.1,
+// without the division where no lane of the wave is near the limit (at most
+// 0.0999 of a positive sum, the rounded quotient is below 0.1).
+__device__ __forceinline__ bool pressure_jump(double pl, double pr, double p_bar) {
+    const double pd = fabs(pr - pl), ps = pr + pl + p_bar + p_bar;
+    bool jump = !((pd <= 0.0999 * ps) & (ps > 1e-280));
+    if (__builtin_amdgcn_ballot_w64(jump) != 0) jump = pd / ps > 0.1;
+    return jump;
+}
+
 // ---------------------------------------------------------------------------
 // Residual: InviscidFlux + RoeFlux_noprec + LoadFlux (cal_flux.cpp:84-192,
-// 682-833, 1219-1254).  res[c] starts at 0 (after ZeroResiduals) or at its
-// current value (ACCUM) and receives -F for faces where c is c1 and +F where
-// c is c2, in ascending face order.  Block partial sums of res^2 feed the
+// 682-833, 1219-1254).  res[c] starts at its current value and receives -F for
+// faces where c is c1 and +F where c is c2, in ascending face order.  Block partial sums of res^2 feed the
 // residual norm of main.cpp:294-317.
-template <bool ACCUM, int MAXF>
-__global__ __launch_bounds__(kBlock) void k_flux(int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                                 const int2* __restrict__ fcell, const double4* __restrict__ fgeo,
+template <int LPC>
+__global__ __launch_bounds__(kBlock) void k_flux(int nC, const int* __restrict__ snb,
+                                                 const double4* __restrict__ sgeo, const int* __restrict__ sflip,
                                                  const double* __restrict__ q, double* __restrict__ res,
                                                  double* __restrict__ part, FlowConst K) {
+    constexpr int NS = kSlots<LPC>;
     const int c = xcd_block() * kBlock + (int)threadIdx.x;
     double r[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     if (c < nC) {
-        if (ACCUM) load5(res + (size_t)c * 5, r);
-        int fs[MAXF];
-        const int nf = cell_faces<MAXF>(cfo, cf, c, fs);
-        int2 cc[MAXF];
-        double4 g[MAXF];
+        load5(res + (size_t)c * 5, r);
+        double qc[5];
+        load5(q + (size_t)c * 5, qc);
+        CellSlots<NS> L;
+        load_slots<LPC, false>(c, nC, snb, sgeo, nullptr, sflip, L);
+        const double hc = total_enthalpy(qc, K.gamm1, K.p_bar), hqc = hc / qc[0];
 #pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            cc[s] = fcell[fs[s]];
-            g[s] = fgeo[fs[s]];
-        }
-#pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            double ql[5], qr[5], F[5];
-            load5(q + (size_t)cc[s].x * 5, ql);
-            load5(q + (size_t)cc[s].y * 5, qr);
-            roe_flux<double>(ql, qr, g[s].x, g[s].y, g[s].z, g[s].w, K.gamm1, K.p_bar, K.alf_l, kTINYd, F);
-            if (s < nf) {
-                if (cc[s].x == c) {
-#pragma unroll
-                    for (int j = 0; j < 5; ++j) r[j] -= F[j];
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 5; ++j) r[j] += F[j];
-                }
-            }
+        for (int s = 0; s < NS; ++s) {
+            double qo[5];
+            load5(q + (size_t)L.oth[s] * 5, qo);
+            add_face_flux(qc, hc, hqc, qo, L.first[s], L.g[s], s < L.nf, K, r);
         }
 #pragma unroll
         for (int j = 0; j < 5; ++j) res[(size_t)c * 5 + j] = r[j];
@@ -324,55 +388,40 @@ __global__ __launch_bounds__(kBlock) void k_flux(int nC, const int* __restrict__
 
 // ---------------------------------------------------------------------------
 // Local time step: TimeStepNormal_new + CellIsMG + LimitTimeStep
-// (compute_timestep.cpp:758-823, 1315-1338, 836-918), fused with the
-// LU-SGS diagonal Diag = vol/dt + sum 0.5*A*(|u.n|+a)*lhs_omga
-// (forward_lusgs.cpp:94-99, 554-595) when WITH_DIAG.  Both use the cell's
-// own |u.n| + a on every face.
-template <bool WITH_DIAG, int MAXF>
-__global__ __launch_bounds__(kBlock) void k_timestep(int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                                     const int2* __restrict__ fcell, const double4* __restrict__ fgeo,
-                                                     const double2* __restrict__ fdn, const double* __restrict__ q,
-                                                     const double* __restrict__ vol, double* __restrict__ dt,
-                                                     double* __restrict__ diag, double* __restrict__ part, FlowConst K,
+// (compute_timestep.cpp:758-823, 1315-1338, 836-918), with the cell's own
+// |u.n| + a on every face.
+template <int LPC>
+__global__ __launch_bounds__(kBlock) void k_timestep(int nC, const int* __restrict__ snb,
+                                                     const double4* __restrict__ sgeo, const double* __restrict__ sdn,
+                                                     const int* __restrict__ sflip, const double* __restrict__ q,
+                                                     double* __restrict__ dt, double* __restrict__ part, FlowConst K,
                                                      double cfl, double cfl_min) {
+    constexpr int NS = kSlots<LPC>;
     const int c = xcd_block() * kBlock + (int)threadIdx.x;
     double vmin = kBIGd, vmax = 0.0;
     if (c < nC) {
         double qc[5];
         load5(q + (size_t)c * 5, qc);
         const double rho = qc[0], u = qc[1], v = qc[2], w = qc[3], p = qc[4];
-        int fs[MAXF];
-        const int nf = cell_faces<MAXF>(cfo, cf, c, fs);
-        int2 cc[MAXF];
-        double4 g[MAXF];
-        double2 d[MAXF];
-        double pa[MAXF], pb[MAXF];
+        CellSlots<NS> L;
+        load_slots<LPC, true>(c, nC, snb, sgeo, sdn, sflip, L);
+        double po[NS];
 #pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            cc[s] = fcell[fs[s]];
-            g[s] = fgeo[fs[s]];
-            d[s] = fdn[fs[s]];
-        }
-#pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            pa[s] = q[(size_t)cc[s].x * 5 + 4];
-            pb[s] = q[(size_t)cc[s].y * 5 + 4];
-        }
+        for (int s = 0; s < NS; ++s) po[s] = q[(size_t)L.oth[s] * 5 + 4];
         const double c2tmp = K.gam * (p + K.p_bar) / rho;
         const double a = sqrt(c2tmp);
         double dtc = kBIGd;
         int det = 1;
-        double eig[MAXF];
+        double eig[NS];
 #pragma unroll
-        for (int s = 0; s < MAXF; ++s) {
-            const double dn = (cc[s].x == c) ? d[s].x : d[s].y;
-            double vn = u * g[s].x + v * g[s].y + w * g[s].z;
+        for (int s = 0; s < NS; ++s) {
+            double vn = u * L.g[s].x + v * L.g[s].y + w * L.g[s].z;
             vn = fabs(vn);
             eig[s] = vn + a;
-            const double dp = fabs(pb[s] - pa[s]) / (pb[s] + pa[s] + K.p_bar + K.p_bar);
-            if (s < nf) {
-                dtc = smin(dtc, dn / eig[s]);
-                if (dp > 0.1) det = 0;
+            const bool jump = pressure_jump(p, po[s], K.p_bar);
+            if (s < L.nf) {
+                dtc = smin(dtc, L.dn[s] / eig[s]);
+                if (jump) det = 0;
             }
         }
         double cfl_tmp;
@@ -387,32 +436,13 @@ __global__ __launch_bounds__(kBlock) void k_timestep(int nC, const int* __restri
         dt[c] = dtc;
         vmin = dtc;
         vmax = dtc;
-        if (WITH_DIAG) {
-            double dg = vol[c] / dtc;
-#pragma unroll
-            for (int s = 0; s < MAXF; ++s)
-                if (s < nf) dg += 0.5 * g[s].w * eig[s] * K.lhs_omga;
-            diag[c] = dg;
-        }
     }
     block_minmax(vmin, vmax, part + (size_t)5 * gridDim.x + blockIdx.x, part + (size_t)6 * gridDim.x + blockIdx.x);
 }
 
-// Slots of a cell that can hold a face, of the LPC its neighbour and face
-// rows have room for, and the place of slot s of cell c in the slot geometry
-// and distances: slot by slot, so that a wave's load of one slot's 32 bytes a
-// cell spans 16 lines.  Stored cell by cell, every lane's load was in a line
-// of its own, and the CU's cache takes a cycle or more per line.
-// Before and after (residual pass, gradient): 6.0M tetrahedra FP64 565 -> 513
-// and 440 -> 397 us, 1.3M 128 -> 117 and 2.9M mixed 297 -> 276 us (residual);
-// 262k hexahedra, whose pass also took the two empty slots along, 47 -> 39 us.
-template <int LPC>
-constexpr int kSlots = LPC == 4 ? 4 : 6;
-__device__ __forceinline__ size_t slot_at(int s, int c, int nC) { return (size_t)s * nC + c; }
-
 // Residual, local time step and LU-SGS diagonal in one pass over a cell's
-// faces, for the fused iteration: the arithmetic of k_flux<false> and
-// k_timestep<true>, which both read the state at the start of the
+// faces, for the fused iteration: the arithmetic of k_flux (from zero),
+// k_timestep and k_diag, which all read the state at the start of the
 // iteration.  The cell's own state is loaded once and only the neighbour's
 // is gathered per face.  With MIXED the FP32 inputs of the implicit
 // operator (state snapshot, Diag) are written as well.
@@ -428,8 +458,7 @@ __device__ __forceinline__ size_t slot_at(int s, int c, int nC) { return (size_t
 // the diagonal.  NS slots, the first nf used; oth = the face's other cell,
 // g = the face's stored normal and area (c1 -> c2), first = this cell is c1.
 template <int NS, bool MIXED>
-__device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int nf, const int (&oth)[NS],
-                                             const double4 (&g)[NS], const double (&dnv)[NS], const bool (&first)[NS],
+__device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], const CellSlots<NS>& L,
                                              const double* __restrict__ q, const double* __restrict__ vol,
                                              double* __restrict__ res, double* __restrict__ dt,
                                              double* __restrict__ diag, const FlowConst& K, double cfl, double cfl_min,
@@ -443,33 +472,15 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
     double eig[NS];
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
-        double qo[5], ql[5], qr[5], F[5];
-        load5(q + (size_t)oth[s] * 5, qo);
-#pragma unroll
-        for (int j = 0; j < 5; ++j) {
-            ql[j] = first[s] ? qc[j] : qo[j];
-            qr[j] = first[s] ? qo[j] : qc[j];
-        }
-        const double ho = total_enthalpy(qo, K.gamm1, K.p_bar), hqo = ho / qo[0];
-        roe_flux<double>(ql, qr, first[s] ? hc : ho, first[s] ? ho : hc, first[s] ? hqc : hqo, first[s] ? hqo : hqc,
-                         g[s].x, g[s].y, g[s].z, g[s].w, K.gamm1, K.alf_l, kTINYd, F);
-        double vn = qc[1] * g[s].x + qc[2] * g[s].y + qc[3] * g[s].z;
+        double qo[5];
+        load5(q + (size_t)L.oth[s] * 5, qo);
+        add_face_flux(qc, hc, hqc, qo, L.first[s], L.g[s], s < L.nf, K, r);
+        double vn = qc[1] * L.g[s].x + qc[2] * L.g[s].y + qc[3] * L.g[s].z;
         vn = fabs(vn);
         eig[s] = vn + a;
-        // dp > 0.1 without the division where no lane of the wave is near it:
-        // at most 0.0999 of a positive sum, the rounded quotient is below 0.1
-        const double pd = fabs(qr[4] - ql[4]), ps = qr[4] + ql[4] + K.p_bar + K.p_bar;
-        bool jump = !((pd <= 0.0999 * ps) & (ps > 1e-280));
-        if (__builtin_amdgcn_ballot_w64(jump) != 0) jump = pd / ps > 0.1;
-        if (s < nf) {
-            if (first[s]) {
-#pragma unroll
-                for (int j = 0; j < 5; ++j) r[j] -= F[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 5; ++j) r[j] += F[j];
-            }
-            dtc = smin(dtc, dnv[s] / eig[s]);
+        const bool jump = pressure_jump(qc[4], qo[4], K.p_bar);
+        if (s < L.nf) {
+            dtc = smin(dtc, L.dn[s] / eig[s]);
             if (jump) det = 0;
         }
     }
@@ -489,7 +500,7 @@ __device__ __forceinline__ void flux_ts_cell(int c, const double (&qc)[5], int n
     double dg = vol[c] / dtc;
 #pragma unroll
     for (int s = 0; s < NS; ++s)
-        if (s < nf) dg += 0.5 * g[s].w * eig[s] * K.lhs_omga;
+        if (s < L.nf) dg += 0.5 * L.g[s].w * eig[s] * K.lhs_omga;
     diag[c] = dg;
     if (MIXED) {
         diag32[c] = (float)dg;
@@ -518,23 +529,10 @@ __device__ __forceinline__ void flux_ts_slot_body(int c, int nC, const int* __re
     if (c < nC) {
         double qc[5];
         load5(q + (size_t)c * 5, qc);
-        const unsigned sf = (unsigned)sflip[c];
-        const int nf = (int)((sf >> 8) & 15u);
-        int oth[NS];
-        double4 g[NS];
-        double dnv[NS];
-        bool first[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const size_t i = slot_at(s, c, nC);
-            const double4 v = sgeo[i];
-            first[s] = ((sf >> s) & 1u) == 0;
-            g[s] = first[s] ? v : make_double4(-v.x, -v.y, -v.z, v.w);
-            oth[s] = snb[(size_t)c * LPC + s];
-            dnv[s] = sdn[i];
-        }
+        CellSlots<NS> L;
+        load_slots<LPC, true>(c, nC, snb, sgeo, sdn, sflip, L);
         double dtc;
-        flux_ts_cell<NS, MIXED>(c, qc, nf, oth, g, dnv, first, q, vol, res, dt, diag, K, cfl, cfl_min, q32, diag32,
+        flux_ts_cell<NS, MIXED>(c, qc, L, q, vol, res, dt, diag, K, cfl, cfl_min, q32, diag32,
                                  r, dtc);
         vmin = dtc;
         vmax = dtc;
@@ -555,12 +553,12 @@ __device__ __forceinline__ void flux_ts_slot_body(int c, int nC, const int* __re
 // With `run`, only cells whose dt exceeds ratio_dtmax*dt_min are clamped
 // and recomputed (compute_timestep.cpp:929-945), and only when the
 // reduction found the ratio exceeded.
-template <int MAXF>
-__device__ __forceinline__ void diag_body(int c, int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                          const double4* __restrict__ fgeo, const double* __restrict__ q,
-                                          const double* __restrict__ vol, double* __restrict__ dt,
-                                          double* __restrict__ diag, const double* __restrict__ run,
-                                          double ratio_dtmax, const FlowConst& K, float* __restrict__ diag32) {
+template <int LPC>
+__device__ __forceinline__ void diag_body(int c, int nC, const double4* __restrict__ sgeo, const int* __restrict__ sflip,
+                                          const double* __restrict__ q, const double* __restrict__ vol,
+                                          double* __restrict__ dt, double* __restrict__ diag,
+                                          const double* __restrict__ run, double ratio_dtmax, const FlowConst& K,
+                                          float* __restrict__ diag32) {
     if (c >= nC) return;
     double dtc = dt[c];
     if (run) {
@@ -572,13 +570,12 @@ __device__ __forceinline__ void diag_body(int c, int nC, const int* __restrict__
     }
     double qc[5];
     load5(q + (size_t)c * 5, qc);
-    int fs[MAXF];
-    const int nf = cell_faces<MAXF>(cfo, cf, c, fs);
+    const int nf = (sflip[c] >> 8) & 15;
     const double a = sqrt(K.gam * (qc[4] + K.p_bar) / qc[0]);
     double dg = vol[c] / dtc;
 #pragma unroll
-    for (int s = 0; s < MAXF; ++s) {
-        const double4 g = fgeo[fs[s]];
+    for (int s = 0; s < kSlots<LPC>; ++s) {
+        const double4 g = sgeo[slot_at(s, c, nC)];  // either side's normal: |u.n| is the same
         double vn = qc[1] * g.x + qc[2] * g.y + qc[3] * g.z;
         vn = fabs(vn);
         if (s < nf) dg += 0.5 * g.w * (vn + a) * K.lhs_omga;
@@ -586,28 +583,28 @@ __device__ __forceinline__ void diag_body(int c, int nC, const int* __restrict__
     diag[c] = dg;
     if (diag32) diag32[c] = (float)dg;
 }
-template <int MAXF>
-__global__ __launch_bounds__(kBlock) void k_diag(int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                                 const double4* __restrict__ fgeo, const double* __restrict__ q,
+template <int LPC>
+__global__ __launch_bounds__(kBlock) void k_diag(int nC, const double4* __restrict__ sgeo,
+                                                 const int* __restrict__ sflip, const double* __restrict__ q,
                                                  const double* __restrict__ vol, double* __restrict__ dt,
                                                  double* __restrict__ diag, const double* __restrict__ run,
                                                  double ratio_dtmax, FlowConst K, float* __restrict__ diag32) {
-    diag_body<MAXF>(xcd_block() * kBlock + (int)threadIdx.x, nC, cfo, cf, fgeo, q, vol, dt, diag, run, ratio_dtmax, K,
-                    diag32);
+    diag_body<LPC>(xcd_block() * kBlock + (int)threadIdx.x, nC, sgeo, sflip, q, vol, dt, diag, run, ratio_dtmax, K,
+                   diag32);
 }
 
 // The ratio_dtmax clamp alone (compute_timestep.cpp:929-945) over a small
 // grid: every workgroup reads the reduction's flag first and returns when
 // the clamp is off, which is the rule at the reference's ratio_dtmax.
-template <int MAXF>
-__global__ __launch_bounds__(kBlock) void k_clamp(int nC, const int* __restrict__ cfo, const int* __restrict__ cf,
-                                                  const double4* __restrict__ fgeo, const double* __restrict__ q,
+template <int LPC>
+__global__ __launch_bounds__(kBlock) void k_clamp(int nC, const double4* __restrict__ sgeo,
+                                                  const int* __restrict__ sflip, const double* __restrict__ q,
                                                   const double* __restrict__ vol, double* __restrict__ dt,
                                                   double* __restrict__ diag, const double* __restrict__ run,
                                                   double ratio_dtmax, FlowConst K, float* __restrict__ diag32) {
     if (run[2] == 0.0) return;
     for (int c = (int)(blockIdx.x * kBlock + threadIdx.x); c < nC; c += (int)(gridDim.x * kBlock))
-        diag_body<MAXF>(c, nC, cfo, cf, fgeo, q, vol, dt, diag, run, ratio_dtmax, K, diag32);
+        diag_body<LPC>(c, nC, sgeo, sflip, q, vol, dt, diag, run, ratio_dtmax, K, diag32);
 }
 
 // FP32 operator inputs of a mixed-precision context from the FP64 state and

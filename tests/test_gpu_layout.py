@@ -179,3 +179,28 @@ def test_pressure_jump_test_near_its_limit(tmp_path, cells, dims, jump):
     s.close()
     o.close()
     g.close()
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED])
+@pytest.mark.parametrize("cells,sizes", [("tet", (2, 8, 16)), ("hex", (5, 27, 3))])
+def test_batch_time_step_clamp_equals_standalone(precision, cells, sizes):
+    """The ratio_dtmax clamp of a batch walks each solve's cells on a fixed
+    number of workgroups (64 of 256 cells: the middle and last tetrahedral
+    meshes and the middle hexahedral one need a second turn or part of one);
+    one solve has it off.  Every member equals the same solve alone."""
+    print(f"[layout] batch clamp precision={precision} {cells} {sizes}", flush=True)
+    cases = []
+    for k, n in enumerate(sizes):
+        p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0, ratio_dtmax=1e80 if k == 0 else 1.2)
+        cases.append((mfs.Grid.box_bump(n, seed=k + 1, cells=cells).decouple().preprocess(p), p))
+    b = mfs.Batch(precision)
+    members = [b.add(g, p) for g, p in cases]
+    b.step(3)
+    for m, (g, p) in zip(members, cases):
+        s = mfs.Solver(g, p, precision=precision)
+        s.step(3)
+        for nm in FIELDS:
+            np.testing.assert_array_equal(m.field(nm), s.field(nm), err_msg=nm)
+        np.testing.assert_array_equal(m.history(), s.history())
+        s.close()
+    b.close()
