@@ -238,9 +238,9 @@ def mode_fp64(args, cpu_dir: str | None = None) -> dict:
     sweeps = None
     if kern:
         # the dominant kernel launch of the critical path: the solver
-        # stream's launches (node values and the gradient run on the
-        # context's second stream beside them); a split sweep counts as its
-        # two launches
+        # stream's launches (node values and the gradient run inside the thin
+        # tails' launches, or on the context's second stream beside them); a
+        # split sweep counts as its two launches
         split = [k for k in SWEEP_LAUNCHES if SWEEP_LAUNCHES[k][0] in kern]
         launches = [k for k in kern if k not in SIDE_KERNELS and k not in split]
         dom = max(launches, key=lambda k: kern[k][0])

@@ -263,7 +263,8 @@ typedef struct mfs_ctx_info {
     size_t device_bytes;   /* device memory held by the context */
     int tile_cells, sweep_waves, sweep_tiles, sweep_workgroups, sweep_by_tiles;
     int compute_units;     /* CUs of the context's device (the sweep grid is sized on them) */
-    int sweep_tail_chunks; /* chunks of the sweeps' thin-tail launch (0: one launch per sweep) */
+    int sweep_tail_chunks; /* the thin-tail launch in groups of 16 cells of a tile (8 on meshes with more than 4
+                            * faces per cell; 0: one launch per sweep) */
     int sweep_tail_cells;  /* their cells */
     int sweep_tail_workgroups;
 } mfs_ctx_info;

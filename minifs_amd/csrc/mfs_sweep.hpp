@@ -24,11 +24,11 @@
 // 433 / 452 us.
 //
 // Schedule: cells are stored by tile (4096 consecutive mesh ids, a compact
-// region in TDTree numbering), then forward level; a chunk is up to 64/LPC
-// cells of one (tile, level) group, so its cells never depend on one
-// another.  Two schedules, both on a grid sized to be resident at once:
-//   flat (default): the chunks in forward level order (`run`), the backward
-//     sweep walking it from the end; the steps go to the ticket groups in
+// region in TDTree numbering), then forward level; a chunk is as many cells
+// of one (tile, level) group as have 64 dependencies together, so its cells
+// never depend on one another.  Two schedules, both on a grid sized to be resident at once:
+//   flat (default): the chunks in forward level order, the backward sweep's
+//     by level from the end; the steps go to the ticket groups in
 //     runs of 2^run_shift consecutive steps, run k to group k mod ngroups,
 //     and a free wave of the group takes the group's next step from the
 //     group's counter, so waves that finish early take more chunks and no
@@ -677,7 +677,7 @@ struct XcdArgs {
 // XCD's issue slots and L2: on a second stream their workgroups landed there
 // too, and a tail of 303 us took 605 us beside the node values and 436 beside
 // the gradient (6.0M cells, FP64); inside, the two launches take 373 us with
-// the node values (290 us alone) and 519 with the gradient (440 alone).
+// the node values (292 us alone) and 481 with the gradient (397 alone).
 template <bool FWD, int MAXF, typename R>
 __global__ __launch_bounds__(kBlock) void k_sweep_xcd(XcdArgs<R> P) {
     const SweepArgs<R>& A = P.A;
