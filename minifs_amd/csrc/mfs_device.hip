@@ -113,9 +113,18 @@ constexpr int kDefaultBatchGradientStreamMixed = 4;
 // 64 groups of cells), when it holds at least kMinTailChunks of them.
 constexpr int kDefaultTailGrid = 64;
 constexpr int kThinWaves = 2;  // waves that a workgroup of the tail grid stands for
-// Workgroups per CU of a thin launch with side work (4 waves each, the
-// registers' limit).
-constexpr int kSideGroups = 4;
+// Workgroups per CU of a thin launch with side work.  The fewer, the less
+// their traffic delays the thin levels' hops, and the fewer nodes' cells
+// compete for an L2 (with 4 per CU the node values read 1.9 GB instead of 1.0
+// at 6.0M cells): one, as long as the tail still hides the gradient (6.0M
+// cells take it 590 us at one per CU, so a level of 1.2 us hides 12,000
+// cells), else three.  ms per iteration, gradient at 4 / 3 / 2 / 1 per CU with
+// the node values at 1 (both at 4): 262k hexahedra 0.608 / 0.603 / 0.594 /
+// 0.586 (0.622), 195k prisms mixed 0.431 / 0.430 / 0.427 / 0.425 (0.437), 1.3M
+// tetrahedra 0.918 / 0.913 / 0.905 / 0.896 (0.936), 6.0M (25,600 cells per
+// thin level) 2.716 / 2.709 / 2.718 / 2.828 (2.753).
+constexpr int kSideFewGroups = 1, kSideGroups = 3;
+constexpr int kSideFewCellsPerLevel = 12000;
 // The gradient runs inside the thin launches up to this many cells per thin
 // level, and on the second stream above, where the thin levels are too short
 // to hide it and the second stream spreads it over the wide levels too.
@@ -939,7 +948,9 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
         g.x = (unsigned)(join * dev::kXcd);
         if (P.W.nblk > 0) {
             const int most = (int)g.x + P.W.nblk;
-            g.x = std::max<unsigned>(g.x, (unsigned)std::min(dev::kSideGroups * ctx->compute_units, most));
+            const bool few = fwd || ctx->nC <= (long long)dev::kSideFewCellsPerLevel * ctx->thin_levels;
+            const int groups = few ? dev::kSideFewGroups : dev::kSideGroups;
+            g.x = std::max<unsigned>(g.x, (unsigned)std::min(groups * ctx->compute_units, most));
         }
         void* args[] = {&P};
         return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(kBlock), args, dev::stage_bytes(W), ctx->stream, ev0, ev1, 0),

@@ -204,3 +204,24 @@ def test_batch_time_step_clamp_equals_standalone(precision, cells, sizes):
         np.testing.assert_array_equal(m.history(), s.history())
         s.close()
     b.close()
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED])
+@pytest.mark.parametrize("cells,dims,tree", [("tet", (40, 40, 40), (2, 64)), ("tet", (40, 40, 40), (4, 512)),
+                                             ("hex", (72, 70, 71), (2, 32)), ("hex", (31, 30, 32), (4, 512))])
+def test_gradient_inside_the_tails_equals_the_solver_stream(precision, cells, dims, tree):
+    """The gradient as side work of the thin launches, on few or more
+    workgroups per CU (many cells per thin level: the shallow orders; few: the
+    deep ones), equals the gradient on the solver stream."""
+    print(f"[layout] gradient inside {cells} {dims} {tree} precision={precision}", flush=True)
+    p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0)
+    g = mfs.Grid.box_bump(*dims, seed=4, cells=cells).decouple(*tree).preprocess(p)
+    out = []
+    for stream in (5, 1):
+        s = mfs.Solver(g, p, precision=precision, gradient_stream=stream)
+        s.step(3)
+        out.append([s.field(nm) for nm in ("rho", "dqdx", "dqdy", "dqdz")])
+        s.close()
+    g.close()
+    for a, b in zip(*out):
+        np.testing.assert_array_equal(a, b)
