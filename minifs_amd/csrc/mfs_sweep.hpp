@@ -676,7 +676,7 @@ struct XcdArgs {
 // The side blocks fill the CUs that the sweep leaves idle without sharing its
 // XCD's issue slots and L2: on a second stream their workgroups landed there
 // too, and a tail of 303 us took 605 us beside the node values and 436 beside
-// the gradient (6.0M cells, FP64); inside, the two launches take 373 us with
+// the gradient (6.0M cells, FP64); inside, the two launches take 340 us with
 // the node values (292 us alone) and 481 with the gradient (397 alone).
 template <bool FWD, int MAXF, typename R>
 __global__ __launch_bounds__(kBlock) void k_sweep_xcd(XcdArgs<R> P) {
