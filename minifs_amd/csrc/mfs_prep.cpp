@@ -3,6 +3,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <exception>
 #include <numeric>
 #include <sstream>
 #include <thread>
@@ -574,9 +575,21 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
             });
         };
         {
-            std::thread fwd([&] { build(0); });
-            build(1);
+            // an exception (out of memory) of either direction reaches the
+            // caller, after both have ended
+            std::exception_ptr thrown[2];
+            auto guarded = [&](int dir) {
+                try {
+                    build(dir);
+                } catch (...) {
+                    thrown[dir] = std::current_exception();
+                }
+            };
+            std::thread fwd(guarded, 0);
+            guarded(1);
             fwd.join();
+            for (const std::exception_ptr& e : thrown)
+                if (e) std::rethrow_exception(e);
         }
         for (const std::string& e : err)
             if (!e.empty()) return e;
