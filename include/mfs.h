@@ -177,8 +177,9 @@ typedef struct mfs_ctx_options {
     int sweep_tail_grid; /* workgroups (of 2 waves, on one XCD) of the sweeps' thin-tail launch: each sweep
                           * of the flat schedule runs its wide levels and the run of thin levels that ends
                           * its order as two launches.  A level is thin with at most 64 chunks, counted as
-                          * 16 cells of a tile (8 on meshes with more than 4 faces per cell).  0: default
-                          * (64); -1: one launch per sweep. */
+                          * 16 cells of a tile (8 on meshes with more than 4 faces per cell, where from
+                          * 16,384 cells on the limit is 128).  0: default (64); -1: one launch per
+                          * sweep. */
 } mfs_ctx_options;
 int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p, int precision, const mfs_ctx_options* opt,
                       mfs_ctx** out);

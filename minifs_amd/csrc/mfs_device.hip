@@ -110,7 +110,7 @@ constexpr int kDefaultBatchGradientStreamFP64 = 1;
 constexpr int kDefaultBatchGradientStreamMixed = 4;
 // The sweeps' thin tail runs as a launch of its own on this many workgroups
 // of kThinWaves waves, all on one XCD (k_sweep_xcd; a thin level has at most
-// 64 groups of cells), when it holds at least kMinTailChunks of them.
+// 64 groups of cells, or 128 narrower ones), when it holds at least kMinTailChunks of them.
 constexpr int kDefaultTailGrid = 64;
 constexpr int kThinWaves = 2;  // waves that a workgroup of the tail grid stands for
 // Workgroups per CU of a thin launch with side work.  The fewer, the less

@@ -449,7 +449,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         gfirst.push_back(nC);
         for (int g = 0; g < ng; ++g) width[glevel[g]] += (gfirst[g + 1] - gfirst[g] + unit - 1) / unit;
         std::vector<char> thin(L.nlev);
-        for (int l = 0; l < L.nlev; ++l) thin[l] = width[l] <= kThinLevelChunks;
+        const int most_groups = L.lpc == 8 && nC >= kWideThinMeshCells ? kWideThinLevelChunks : kThinLevelChunks;
+        for (int l = 0; l < L.nlev; ++l) thin[l] = width[l] <= most_groups;
         int tail_level = L.nlev;  // first level of the thin tail
         while (tail_level > 0 && thin[tail_level - 1]) L.tail_chunks += width[--tail_level];
         L.all_thin = tail_level == 0;

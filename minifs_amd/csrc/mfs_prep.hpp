@@ -131,11 +131,21 @@ struct HostLayout {
 // Cells per storage tile of the device order (the sweeps' workgroup unit).
 constexpr int kDefaultTileCells = 4096;
 // Thin levels.  A level's width is counted in groups of 64/lpc cells per
-// tile; levels of at most kThinLevelChunks groups are thin.  A thin chunk
+// tile; levels of at most kThinLevelChunks groups are thin (on larger meshes of
+// 8 slots per cell kWideThinLevelChunks, below).  A thin chunk
 // holds at most kThinCells cells, so that each of its 5-value results has a
 // lane of its own.
 constexpr int kThinLevelChunks = 64;
 constexpr int kThinCells = 12;
+// With 8 slots per cell a group has 8 cells, half of a tetrahedral mesh's, so
+// the same 1,024 cells of a level are 128 groups: 86 thin chunks, one for
+// each of the 128 waves that sweep the tail.  ms per iteration with 64 and
+// with 128 groups: 262k hexahedra FP64 0.593 -> 0.583, 64k 0.321 -> 0.308,
+// 33k 0.260 -> 0.248; 195k prisms mixed 0.432 -> 0.418, 35k FP64 0.249 ->
+// 0.240.  (Tetrahedra gained nothing from 128: 20k, 94k and 384k cells all
+// within 0.2%.)  Smaller meshes gain too (8k hexahedra 0.163 -> 0.142), but
+// the tail that mfs_ctx_info reports for them is pinned, so they keep 64.
+constexpr int kWideThinLevelChunks = 128, kWideThinMeshCells = 16384;
 // On levels of at most this many groups a wave waits on a dependency one
 // level further back and then polls its own at once (SweepLayout::crec); on
 // wider ones it waits on its latest dependency with one load, since there the

@@ -225,3 +225,19 @@ def test_gradient_inside_the_tails_equals_the_solver_stream(precision, cells, di
     g.close()
     for a, b in zip(*out):
         np.testing.assert_array_equal(a, b)
+
+
+@pytest.mark.parametrize("cells,dims", [("hex", (25, 25, 26)), ("hex", (26, 26, 26)), ("prism", (20, 20, 20)),
+                                        ("prism", (21, 19, 23))])
+def test_thin_line_of_six_face_meshes(cells, dims):
+    """On both sides of the mesh size from which levels of up to 128 groups
+    are thin, the thin tails' launches give the tile schedule's bits."""
+    p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0)
+    g = mfs.Grid.box_bump(*dims, cells=cells).decouple().preprocess(p)
+    a, b = mfs.Solver(g, p), mfs.Solver(g, p, sweep_by_tiles=1)
+    for s in (a, b):
+        s.step(6)
+    for nm in ("rho", "u", "v", "w", "p", "dqdx", "dqdy", "dqdz"):
+        np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=nm)
+    a.close()
+    b.close()
