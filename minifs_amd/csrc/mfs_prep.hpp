@@ -142,7 +142,9 @@ constexpr int kThinCells = 12;
 // each of the 128 waves that sweep the tail.  ms per iteration with 64 and
 // with 128 groups: 262k hexahedra FP64 0.593 -> 0.583, 64k 0.321 -> 0.308,
 // 33k 0.260 -> 0.248; 195k prisms mixed 0.432 -> 0.418, 35k FP64 0.249 ->
-// 0.240.  (Tetrahedra gained nothing from 128: 20k, 94k and 384k cells all
+// 0.240; 1M hexahedra FP64 1.206 -> 1.179, on a shallow order 0.938 -> 0.910.
+// Batches, whose waits do not use the line, change by less than 1% (8 solves
+// of hexahedra 0.924 -> 0.921, of prisms 1.205 -> 1.212).  (Tetrahedra gained nothing from 128: 20k, 94k and 384k cells all
 // within 0.2%.)  Smaller meshes gain too (8k hexahedra 0.163 -> 0.142), but
 // the tail that mfs_ctx_info reports for them is pinned, so they keep 64.
 constexpr int kWideThinLevelChunks = 128, kWideThinMeshCells = 16384;
