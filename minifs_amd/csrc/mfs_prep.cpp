@@ -3,7 +3,6 @@
 
 #include <algorithm>
 #include <cmath>
-#include <exception>
 #include <numeric>
 #include <sstream>
 #include <thread>
@@ -123,13 +122,22 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
     // and a cell's face neighbours are mostly in its own tile (gathers of
     // the face kernels stay in a small window of memory).
     std::vector<int> dcell(nC);
+    std::vector<int> gfirst, glevel, gtile;  // (tile, level) groups: first device cell (and nC), level, tile
     {
         const int ntile = (nC + kTileCells - 1) / kTileCells;
         const size_t nkey = (size_t)ntile * L.nlev;
         std::vector<int> cnt(nkey + 1, 0);
         auto key = [&](int c) { return (size_t)(c / kTileCells) * L.nlev + L.flevel[c]; };
         for (int c = 0; c < nC; ++c) cnt[key(c) + 1]++;
-        for (size_t k = 0; k < nkey; ++k) cnt[k + 1] += cnt[k];
+        for (size_t k = 0; k < nkey; ++k) {
+            if (cnt[k + 1] > 0) {
+                gfirst.push_back(cnt[k]);
+                glevel.push_back((int)(k % L.nlev));
+                gtile.push_back((int)(k / L.nlev));
+            }
+            cnt[k + 1] += cnt[k];
+        }
+        gfirst.push_back(nC);
         L.cell_of_dev.resize(nC);
         for (int c = 0; c < nC; ++c) {
             const int d = cnt[key(c)]++;
@@ -158,8 +166,16 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         }
         if (next != nF) return "face not attached to any cell";
     }
-    // per device cell: device face ids, still in ascending mesh face id,
-    // and the sweep dependency masks
+    // per device cell: device face ids, still in ascending mesh face id, the
+    // sweep dependency masks and, per direction, the cell's latest dependency:
+    // 2 * its depth (the levels before it in the sweep's order) + 1 for
+    // another tile's, and its device cell; -1 without one.  The first of
+    // equal rank in the cell's face order is taken.
+    struct Latest {
+        int rank, cell;
+    };
+    lvec<Latest> latest[2];
+    for (auto& l : latest) l.resize(nC);
     L.cfo.assign(nC + 1, 0);
     L.cf.resize(mcf.size());
     L.depmask.assign(nC, 0);
@@ -171,6 +187,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
             const int c = L.cell_of_dev[d];
             int s = 0;
             unsigned mask = 0;
+            Latest late[2] = {{-1, -1}, {-1, -1}};
             for (int k = mcfo[c]; k < mcfo[c + 1]; ++k, ++s) {
                 const int f = mcf[k];
                 L.cf[pos++] = dface[f];
@@ -179,6 +196,11 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                 if (nb > c) {
                     mask |= 1u << (8 + s);
                     if (nb < nC) mask |= 1u << (16 + s);
+                }
+                if (nb < nC) {
+                    const int dir = nb < c ? 0 : 1, l = L.flevel[nb];
+                    const int rank = 2 * (dir == 0 ? l : L.nlev - l) + (nb / kTileCells != c / kTileCells ? 1 : 0);
+                    if (rank > late[dir].rank) late[dir] = {rank, dcell[nb]};
                 }
                 // gradient: boundary faces other than SYMM and INTERFACE take
                 // the face-centre average of cell and ghost instead of the
@@ -189,6 +211,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                 }
             }
             L.depmask[d] = (int)mask;
+            for (int dir = 0; dir < 2; ++dir) latest[dir][d] = late[dir];
         }
     });
 
@@ -433,20 +456,10 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
     // backward dependency in a later one.
     L.lpc = L.max_faces <= 4 ? 4 : 8;
     {
-        // (tile, level) groups of consecutive device cells, and the levels'
-        // widths in 64/lpc-cell units
+        // the levels' widths in 64/lpc-cell units
         const int unit = 64 / L.lpc;
-        std::vector<int> gfirst, glevel, width(L.nlev, 0);
-        for (int d = 0, tile = -1, lev = -1; d < nC; ++d) {
-            const int c = L.cell_of_dev[d];
-            if (c / kTileCells == tile && L.flevel[c] == lev) continue;
-            tile = c / kTileCells;
-            lev = L.flevel[c];
-            gfirst.push_back(d);
-            glevel.push_back(lev);
-        }
-        const int ng = (int)gfirst.size();
-        gfirst.push_back(nC);
+        const int ng = (int)glevel.size();
+        std::vector<int> width(L.nlev, 0);
         for (int g = 0; g < ng; ++g) width[glevel[g]] += (gfirst[g + 1] - gfirst[g] + unit - 1) / unit;
         std::vector<char> thin(L.nlev);
         const int most_groups = L.lpc == 8 && nC >= kWideThinMeshCells ? kWideThinLevelChunks : kThinLevelChunks;
@@ -463,137 +476,96 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         for (int g = 0; g < ng; ++g)
             if (glevel[g] >= tail_level) L.tail_cells += gfirst[g + 1] - gfirst[g];
         L.cdep.resize(2 * (size_t)nC);
-        std::string err[2];
-        auto build = [&](int dir) {
+        std::vector<int> gchunk(ng + 1);
+        for (int dir = 0; dir < 2; ++dir) {
             SweepLayout& S = L.sweep[dir];
-            auto deps = [&](int d) {
-                const unsigned m = (unsigned)L.depmask[d];
-                return __builtin_popcount(dir == 0 ? (m & 0xffu) : ((m >> 8) & 0xffu));
-            };
-            // chunks in device order: first cell, cells, dependencies, level
-            struct Chunk {
-                int first, cells, deps, level;
-            };
-            std::vector<Chunk> ch;
-            ch.reserve((size_t)nC / 24 + ng);
-            S.tile_chunk.clear();
-            int cur_tile = -1;
-            for (int g = 0; g < ng; ++g) {
-                const int tile = L.cell_of_dev[gfirst[g]] / kTileCells;
-                while (cur_tile < tile) {
-                    S.tile_chunk.push_back((int)ch.size());
-                    ++cur_tile;
-                }
+            // The chunks of group g in device order: fn(first cell, cells,
+            // dependencies) for each, cell(d, dependencies before it in its
+            // chunk, its own) for each cell.
+            auto cut = [&](int g, auto&& fn, auto&& cell) {
                 const int most = thin[glevel[g]] ? kThinCells : 64;
                 for (int d = gfirst[g]; d < gfirst[g + 1];) {
-                    Chunk k{d, 0, 0, glevel[g]};
-                    while (d < gfirst[g + 1] && k.cells < most) {
-                        const int n = deps(d);
-                        if (k.deps + n > 64) break;
-                        k.deps += n;
-                        ++k.cells;
+                    const int first = d;
+                    int deps = 0;
+                    while (d < gfirst[g + 1] && d - first < most) {
+                        const int n = __builtin_popcount(((unsigned)L.depmask[d] >> (8 * dir)) & 0xffu);
+                        if (deps + n > 64) break;
+                        cell(d, deps, n);
+                        deps += n;
                         ++d;
                     }
-                    ch.push_back(k);
+                    fn(first, d - first, deps);
                 }
-            }
-            const int nchunk = (int)ch.size();
+            };
+            parallel_ranges(ng, layout_threads(nC), [&](size_t b, size_t e, int) {
+                for (int g = (int)b; g < (int)e; ++g) {
+                    int k = 0;
+                    cut(g, [&](int, int, int) { ++k; },
+                        [&](int d, int start, int n) { L.cdep[2 * (size_t)d + dir] = (unsigned short)(start | (n << 8)); });
+                    gchunk[g + 1] = k;
+                }
+            });
+            gchunk[0] = 0;
+            for (int g = 0; g < ng; ++g) gchunk[g + 1] += gchunk[g];
+            const int nchunk = gchunk[ng];
             S.nchunk = nchunk;
+            S.tile_chunk.clear();
+            for (int g = 0; g < ng; ++g)
+                if (g == 0 || gtile[g] != gtile[g - 1]) S.tile_chunk.push_back(gchunk[g]);
             S.tile_chunk.push_back(nchunk);
             // flat order: forward by level, then device order (a stable
-            // counting sort); backward exactly from the end
+            // counting sort over the groups); backward exactly from the end
             std::vector<int> at(L.nlev + 1, 0);
-            for (const Chunk& k : ch) at[k.level + 1]++;
+            for (int g = 0; g < ng; ++g) at[glevel[g] + 1] += gchunk[g + 1] - gchunk[g];
             for (int l = 0; l < L.nlev; ++l) at[l + 1] += at[l];
             S.tail = nchunk - at[tail_level];
             S.pos.resize(nchunk);
-            std::vector<int> chunk_at(nchunk);
-            for (int t = 0; t < nchunk; ++t) {
-                const int u = at[ch[t].level]++;
-                S.pos[t] = dir == 0 ? u : nchunk - 1 - u;
-                chunk_at[S.pos[t]] = t;
-            }
             S.crec.resize(4 * (size_t)nchunk);
             S.batch_wait.resize(nchunk);
+            std::vector<int> gat(ng);  // forward position of the group's first chunk
+            for (int g = 0; g < ng; ++g) {
+                gat[g] = at[glevel[g]];
+                at[glevel[g]] += gchunk[g + 1] - gchunk[g];
+            }
+            parallel_ranges(ng, layout_threads(nC), [&](size_t b, size_t e, int) {
+                for (int g = (int)b; g < (int)e; ++g) {
+                    int k = 0;
+                    cut(g,
+                        [&](int first, int cells, int deps) {
+                            const int u = dir == 0 ? gat[g] + k : nchunk - 1 - (gat[g] + k);
+                            S.pos[gchunk[g] + k] = u;
+                            S.crec[4 * (size_t)u] = first;
+                            S.crec[4 * (size_t)u + 1] = cells | (deps << 8) | (thin[glevel[g]] ? kThinChunkFlag : 0);
+                            ++k;
+                        },
+                        [](int, int, int) {});
+                }
+            });
             size_t nd = 0;
             for (int u = 0; u < nchunk; ++u) {
-                const Chunk& k = ch[chunk_at[u]];
-                S.crec[4 * (size_t)u] = k.first;
-                S.crec[4 * (size_t)u + 1] = k.cells | (k.deps << 8) | (thin[k.level] ? kThinChunkFlag : 0);
                 S.crec[4 * (size_t)u + 2] = (int)nd;
-                nd += k.deps;
+                nd += (S.crec[4 * (size_t)u + 1] >> 8) & 0xff;
             }
             S.ndep = nd;
-            if (nd > 0x7fffffffu - 64) {
-                err[dir] = "mesh too large for the sweep tables";
-                return;
-            }
+            if (nd > 0x7fffffffu - 64) return "mesh too large for the sweep tables";
             // the tile schedule walks a tile's chunks in the sweep's order
             if (dir == 1)
                 for (size_t t = 0; t + 1 < S.tile_chunk.size(); ++t)
                     std::reverse(S.pos.begin() + S.tile_chunk[t], S.pos.begin() + S.tile_chunk[t + 1]);
-            // per cell its place among the chunk's dependencies; per chunk
-            // the dependency of the latest level, another tile's first, the
-            // first of equal rank in the chunk's cell and face order (narrow
-            // levels: that dependency's own latest)
-            parallel_for(nchunk, [&](size_t uu) {
-                const int u = (int)uu;
-                const int d0 = S.crec[4 * uu], cells = S.crec[4 * uu + 1] & 0xff;
-                long long best = -1;
-                int rep = -1, start = 0;
-                // the dependency of cell c that ranks above `best`, if any
-                auto latest = [&](int c, long long& best, int& rep) {
-                    for (int k = mcfo[c]; k < mcfo[c + 1]; ++k) {
-                        const int f = mcf[k];
-                        if (f < nB) continue;
-                        const int nb = other(c, f);
-                        if (dir == 0 ? nb > c : nb < c) continue;
-                        const int foreign = (nb / kTileCells != c / kTileCells) ? 1 : 0;
-                        const int l = L.flevel[nb];
-                        const long long r = 2LL * (dir == 0 ? l : L.nlev - l) + foreign;
-                        if (r > best) {
-                            best = r;
-                            rep = dcell[nb];
-                        }
-                    }
-                };
-                for (int d = d0; d < d0 + cells; ++d) {
-                    const int c = L.cell_of_dev[d];
-                    const int n = deps(d);
-                    L.cdep[2 * (size_t)d + dir] = (unsigned short)(start | (n << 8));
-                    start += n;
-                    latest(c, best, rep);
-                }
-                // narrow levels wait on that dependency's own latest instead
-                int further = -1;
-                if (rep >= 0) {
-                    best = -1;
-                    latest(L.cell_of_dev[rep], best, further);
-                }
+            // per chunk the dependency of the latest level, another tile's
+            // first, the first of equal rank in the chunk's cell and face
+            // order; narrow levels wait on that dependency's own latest
+            parallel_for(nchunk, [&](size_t u) {
+                const int d0 = S.crec[4 * u], cells = S.crec[4 * u + 1] & 0xff;
+                Latest rep = latest[dir][d0];
+                for (int d = d0 + 1; d < d0 + cells; ++d)
+                    if (latest[dir][d].rank > rep.rank) rep = latest[dir][d];
+                const int further = rep.cell >= 0 ? latest[dir][rep.cell].cell : -1;
                 const int groups = width[L.flevel[L.cell_of_dev[d0]]];
-                S.batch_wait[u] = groups <= kBatchDirectLevelChunks ? further : rep;
-                S.crec[4 * (size_t)u + 3] = groups <= kDirectLevelChunks ? further : rep;
+                S.batch_wait[u] = groups <= kBatchDirectLevelChunks ? further : rep.cell;
+                S.crec[4 * u + 3] = groups <= kDirectLevelChunks ? further : rep.cell;
             });
-        };
-        {
-            // an exception (out of memory) of either direction reaches the
-            // caller, after both have ended
-            std::exception_ptr thrown[2];
-            auto guarded = [&](int dir) {
-                try {
-                    build(dir);
-                } catch (...) {
-                    thrown[dir] = std::current_exception();
-                }
-            };
-            std::thread fwd(guarded, 0);
-            guarded(1);
-            fwd.join();
-            for (const std::exception_ptr& e : thrown)
-                if (e) std::rethrow_exception(e);
         }
-        for (const std::string& e : err)
-            if (!e.empty()) return e;
         // face slots per device cell (device face ids, ascending mesh face id, -1 = none)
         L.cfs.assign((size_t)nC * L.lpc, -1);
         parallel_for(nC, [&](size_t d) {
