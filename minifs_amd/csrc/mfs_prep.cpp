@@ -2,6 +2,7 @@
 #include "mfs_prep.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <numeric>
 #include <sstream>
@@ -38,6 +39,40 @@ void parallel_for(size_t n, F&& fn) {
     });
 }
 }  // namespace
+
+std::string check_sweep_order(const HostLayout& L, int dir, const lvec<LatestDep>& latest) {
+    const SweepLayout& S = L.sweep[dir];
+    const int n = S.nchunk;
+    auto first = [&](int u) { return S.crec[4 * (size_t)u]; };
+    auto cells = [&](int u) { return S.crec[4 * (size_t)u + 1] & 0xff; };
+    auto depth = [&](int d) {
+        const int l = L.flevel[L.cell_of_dev[d]];
+        return dir == 0 ? l : L.nlev - l;
+    };
+    // the chunks of all tiles, forward or backward in each, cover the cells
+    bool ok = true;
+    int next = 0;
+    for (size_t t = 0; t + 1 < S.tile_chunk.size() && ok; ++t) {
+        const int b = S.tile_chunk[t], e = S.tile_chunk[t + 1];
+        for (int k = 0; k < e - b && ok; ++k) {
+            const int i = dir == 0 ? b + k : e - 1 - k, u = S.pos[i];
+            ok = u >= 0 && u < n && first(u) == next && cells(u) > 0 && (i == b || S.pos[i - 1] < u);
+            if (ok) next += cells(u);
+        }
+    }
+    ok = ok && S.tile_chunk.back() == n && next == L.nC;
+    // each has cells of one depth, none less deep than the chunk before, and
+    // every cell's latest dependency is less deep
+    std::atomic<bool> ordered{true};
+    if (ok)
+        parallel_for(n, [&](size_t uu) {
+            const int u = (int)uu, l = depth(first(u));
+            bool good = u == 0 || depth(first(u - 1)) <= l;
+            for (int d = first(u); d < first(u) + cells(u); ++d) good = good && depth(d) == l && latest[d].rank < 2 * l;
+            if (!good) ordered = false;
+        });
+    return ok && ordered ? "" : std::string(dir == 0 ? "forward" : "backward") + " sweep chunks are not topological";
+}
 
 std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) {
     if (kTileCells < 64) return "tile size must be at least 64 cells";
@@ -167,14 +202,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         if (next != nF) return "face not attached to any cell";
     }
     // per device cell: device face ids, still in ascending mesh face id, the
-    // sweep dependency masks and, per direction, the cell's latest dependency:
-    // 2 * its depth (the levels before it in the sweep's order) + 1 for
-    // another tile's, and its device cell; -1 without one.  The first of
-    // equal rank in the cell's face order is taken.
-    struct Latest {
-        int rank, cell;
-    };
-    lvec<Latest> latest[2];
+    // sweep dependency masks and, per direction, the cell's latest dependency
+    lvec<LatestDep> latest[2];
     for (auto& l : latest) l.resize(nC);
     L.cfo.assign(nC + 1, 0);
     L.cf.resize(mcf.size());
@@ -187,7 +216,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
             const int c = L.cell_of_dev[d];
             int s = 0;
             unsigned mask = 0;
-            Latest late[2] = {{-1, -1}, {-1, -1}};
+            LatestDep late[2] = {{-1, -1}, {-1, -1}};
             for (int k = mcfo[c]; k < mcfo[c + 1]; ++k, ++s) {
                 const int f = mcf[k];
                 L.cf[pos++] = dface[f];
@@ -557,7 +586,7 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
             // order; narrow levels wait on that dependency's own latest
             parallel_for(nchunk, [&](size_t u) {
                 const int d0 = S.crec[4 * u], cells = S.crec[4 * u + 1] & 0xff;
-                Latest rep = latest[dir][d0];
+                LatestDep rep = latest[dir][d0];
                 for (int d = d0 + 1; d < d0 + cells; ++d)
                     if (latest[dir][d].rank > rep.rank) rep = latest[dir][d];
                 const int further = rep.cell >= 0 ? latest[dir][rep.cell].cell : -1;
@@ -565,6 +594,8 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
                 S.batch_wait[u] = groups <= kBatchDirectLevelChunks ? further : rep.cell;
                 S.crec[4 * u + 3] = groups <= kDirectLevelChunks ? further : rep.cell;
             });
+            const std::string e = check_sweep_order(L, dir, latest[dir]);
+            if (!e.empty()) return e;
         }
         // face slots per device cell (device face ids, ascending mesh face id, -1 = none)
         L.cfs.assign((size_t)nC * L.lpc, -1);

@@ -161,6 +161,18 @@ constexpr int kDirectLevelChunks = 1024, kBatchDirectLevelChunks = 64;
 constexpr int kMinTailChunks = 256;  // shorter tails stay with the wide levels
 constexpr int kThinChunkFlag = 0x10000;
 
+// A device cell's latest dependency in one direction: its device cell and its
+// rank, 2 * its depth (the levels before its own in the sweep's order, plus
+// one in the backward sweep) + 1 for another tile's; the first of equal rank
+// in the cell's face order, -1 without one.
+struct LatestDep {
+    int rank, cell;
+};
+// What the sweeps' progress rests on: each direction's chunks cover the cells
+// once, in the order of their depth, in the tile schedule too, and every
+// dependency is less deep than its cell.  Returns "" where that holds.
+std::string check_sweep_order(const HostLayout& L, int dir, const lvec<LatestDep>& latest);
+
 // Returns "" on success.
 std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int tile_cells = kDefaultTileCells);
 

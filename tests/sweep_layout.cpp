@@ -1,8 +1,9 @@
 // Checks of the sweeps' tables (SweepLayout, minifs_amd/csrc/mfs_prep.hpp)
 // against the mesh, from their definitions.  Built and run by
 // test_sweep_layout.py; one argument list per mesh:
-//   sweep_layout cells nx ny nz nb_parts part_size tile_cells
-// prints "ok", or what is wrong.
+//   sweep_layout cells nx ny nz nb_parts part_size tile_cells [spoil direction]
+// prints "ok", or what is wrong.  With `spoil` the order is made wrong in one
+// place and the library's own check of it is printed.
 #include <cstdio>
 #include <cstdlib>
 #include <string>
@@ -121,12 +122,54 @@ std::string check(const mfs::HostLayout& L, int dir, int tile_cells) {
     return "";
 }
 
+// The latest dependencies of every cell, as check_sweep_order takes them.
+mfs::lvec<mfs::LatestDep> latest_of(const mfs::HostLayout& L, int dir, int tile_cells) {
+    mfs::lvec<mfs::LatestDep> out(L.nC);
+    for (int d = 0; d < L.nC; ++d) {
+        out[d] = {-1, -1};
+        const int c = L.cell_of_dev[d];
+        for (int k = L.cfo[d]; k < L.cfo[d + 1]; ++k) {
+            const int f = L.cf[k], nb = L.c1[f] == d ? L.c2[f] : L.c1[f];
+            if (nb >= L.nC) continue;
+            const int m = L.cell_of_dev[nb], l = L.flevel[m];
+            const int r = 2 * (dir == 0 ? l : L.nlev - l) + (m / tile_cells != c / tile_cells ? 1 : 0);
+            if ((dir == 0 ? m < c : m > c) && r > out[d].rank) out[d] = {r, nb};
+        }
+    }
+    return out;
+}
+
+std::string spoiled(mfs::HostLayout& L, const std::string& how, int dir, int tile_cells) {
+    mfs::SweepLayout& S = L.sweep[dir];
+    mfs::lvec<mfs::LatestDep> latest = latest_of(L, dir, tile_cells);
+    const std::string before = mfs::check_sweep_order(L, dir, latest);
+    if (!before.empty()) return "wrong before: " + before;
+    const int mid = S.nchunk / 2;
+    if (how == "dependency")  // a cell that waits for one of its own level
+        latest[S.crec[4 * mid]].rank = 2 * (dir == 0 ? L.flevel[L.cell_of_dev[S.crec[4 * mid]]]
+                                                     : L.nlev - L.flevel[L.cell_of_dev[S.crec[4 * mid]]]);
+    if (how == "level")  // a cell of another level among a chunk's
+        L.flevel[L.cell_of_dev[S.crec[4 * mid]]] += 1;
+    if (how == "order") {  // the first and the last chunk change places
+        for (int k = 0; k < 4; ++k) std::swap(S.crec[k], S.crec[4 * (S.nchunk - 1) + k]);
+        for (int& u : S.pos) u = u == 0 ? S.nchunk - 1 : u == S.nchunk - 1 ? 0 : u;
+    }
+    if (how == "cells") S.crec[4 * mid + 1] += 1;  // a cell in two chunks
+    if (how == "position") S.pos[mid] = S.pos[mid - 1];  // a chunk twice, another never
+    return mfs::check_sweep_order(L, dir, latest);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    if (argc != 8) return 2;
+    if (argc != 8 && argc != 10) return 2;
     Mesh m(argv + 1);
     std::string e = m.error;
+    if (argc == 10 && e.empty()) e = spoiled(m.L, argv[8], atoi(argv[9]), atoi(argv[7]));
+    if (argc == 10) {
+        puts(e.c_str());
+        return 0;
+    }
     for (int dir = 0; dir < 2 && e.empty(); ++dir) e = check(m.L, dir, atoi(argv[7]));
     puts(e.empty() ? "ok" : e.c_str());
     return e.empty() ? 0 : 1;

@@ -37,3 +37,12 @@ def test_tables_follow_from_the_mesh(sweep_layout, cells, dims, tree, tile):
     dependency counts and waits are those of the mesh's faces.  Meshes of one
     chunk up to ones laid out on several threads."""
     assert sweep_layout(cells, dims, tree, tile) == "ok"
+
+
+@pytest.mark.parametrize("direction", [0, 1])
+@pytest.mark.parametrize("spoil", ["dependency", "level", "order", "cells", "position"])
+def test_order_that_cannot_progress_is_refused(sweep_layout, spoil, direction):
+    """A schedule in which a wave could wait for a chunk that comes later, or
+    that no wave takes, is an error when the context is created."""
+    said = sweep_layout("tet", (14, 12, 13), (2, 64), 1000, spoil, direction)
+    assert said == ("forward", "backward")[direction] + " sweep chunks are not topological"
