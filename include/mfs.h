@@ -174,12 +174,13 @@ typedef struct mfs_ctx_options {
                           * (nothing in an iteration reads the gradient).  With 5, and a tail long enough
                           * to hide it, the gradient runs inside the tails' launches instead, on the CUs
                           * they leave idle.  Default 5 (the fastest on 6.0M cells in both precisions). */
-    int sweep_tail_grid; /* workgroups (of 2 waves, on one XCD) of the sweeps' thin-tail launch: each sweep
-                          * of the flat schedule runs its wide levels and the run of thin levels that ends
-                          * its order as two launches.  A level is thin with at most 64 chunks, counted as
+    int sweep_tail_grid; /* pairs of waves, on one XCD, that sweep in the thin-tail launch (rounded up to
+                          * workgroups of 4 waves): each sweep of the flat schedule runs its wide levels and
+                          * the run of thin levels that ends its order as two launches.  A level is thin with at most 64 chunks, counted as
                           * 16 cells of a tile (8 on meshes with more than 4 faces per cell, where from
                           * 16,384 cells on the limit is 128).  0: default (64); -1: one launch per
-                          * sweep. */
+                          * sweep.  A mesh of thin levels only runs each sweep as one launch on one XCD,
+                          * whatever this is. */
 } mfs_ctx_options;
 int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p, int precision, const mfs_ctx_options* opt,
                       mfs_ctx** out);
@@ -264,12 +265,26 @@ typedef struct mfs_ctx_info {
     size_t device_bytes;   /* device memory held by the context */
     int tile_cells, sweep_waves, sweep_tiles, sweep_workgroups, sweep_by_tiles;
     int compute_units;     /* CUs of the context's device (the sweep grid is sized on them) */
-    int sweep_tail_chunks; /* the thin-tail launch in groups of 16 cells of a tile (8 on meshes with more than 4
+    int sweep_tail_chunks; /* the thin tail's levels in groups of 16 cells of a tile (8 on meshes with more than 4
                             * faces per cell; 0: one launch per sweep) */
     int sweep_tail_cells;  /* their cells */
-    int sweep_tail_workgroups;
+    int sweep_tail_workgroups; /* sweep_tail_grid, at most the resident grid and one per sweep_waves groups */
 } mfs_ctx_info;
 int mfs_ctx_get_info(mfs_ctx* ctx, mfs_ctx_info* info);
+/* What the context's steps launch (no counterpart in the reference).  [0] is
+ * the forward sweep, [1] the backward sweep. */
+#define MFS_GRADIENT_INSIDE 6
+typedef struct mfs_ctx_launches {
+    int thin_launch;     /* launches of thin levels on one XCD: 0 none, 1 each sweep's tail, 2 each sweep whole */
+    int thin_workgroups; /* workgroups of 4 waves that sweep in such a launch */
+    int thin_levels;     /* levels that it holds */
+    int wide_workgroups; /* workgroups of sweep_waves waves of the sweeps' other launches */
+    int chunks[2];       /* chunks of cells of each sweep */
+    int thin_chunks[2];  /* those in the launches of thin levels */
+    int gradient;        /* where mfs_step runs its gradients (a call's last one in launches of its own):
+                          * gradient_stream of mfs_ctx_options, or MFS_GRADIENT_INSIDE the thin launches */
+} mfs_ctx_launches;
+int mfs_ctx_get_launches(mfs_ctx* ctx, mfs_ctx_launches* out);
 /* Kernel time accounting: when enabled, every launch of the named kernel
  * group is bracketed with HIP events on the stream it runs on.  enable: 0
  * off, 1 every kernel group, 2 the two sweeps only.  The sweeps' events are

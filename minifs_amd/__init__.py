@@ -221,6 +221,12 @@ class Solver:
         check(lib().mfs_ctx_get_info(self._h, C.byref(i)), "mfs_ctx_get_info")
         return {f: getattr(i, f) for f, _ in i._fields_}
 
+    def launches(self) -> dict:
+        """What the solver's steps launch (mfs_ctx_get_launches)."""
+        i = _lib.MfsCtxLaunches()
+        check(lib().mfs_ctx_get_launches(self._h, C.byref(i)), "mfs_ctx_get_launches")
+        return {f: (v if isinstance(v, int) else tuple(v)) for f, v in ((f, getattr(i, f)) for f, _ in i._fields_)}
+
     def enable_timing(self, on: bool | int = True):
         """True/1: time every kernel group; 2: the two sweeps only; False/0: off."""
         check(lib().mfs_ctx_enable_timing(self._h, int(on)), "mfs_ctx_enable_timing")

@@ -15,6 +15,7 @@ LIB_PATH = os.path.join(_HERE, "libmfs_hip.so")
 MFS_OK = 0
 MFS_FP64 = 0
 MFS_MIXED = 1
+MFS_GRADIENT_INSIDE = 6
 
 F_RHO, F_U, F_V, F_W, F_P, F_RES, F_DT, F_DQ, F_DQDX, F_DQDY, F_DQDZ, F_DIAG, F_QNODE = range(13)
 FIELD_IDS = {
@@ -61,6 +62,12 @@ class MfsCtxInfo(C.Structure):
                 ("tile_cells", C.c_int), ("sweep_waves", C.c_int), ("sweep_tiles", C.c_int),
                 ("sweep_workgroups", C.c_int), ("sweep_by_tiles", C.c_int), ("compute_units", C.c_int),
                 ("sweep_tail_chunks", C.c_int), ("sweep_tail_cells", C.c_int), ("sweep_tail_workgroups", C.c_int)]
+
+
+class MfsCtxLaunches(C.Structure):
+    _fields_ = [("thin_launch", C.c_int), ("thin_workgroups", C.c_int), ("thin_levels", C.c_int),
+                ("wide_workgroups", C.c_int), ("chunks", C.c_int * 2), ("thin_chunks", C.c_int * 2),
+                ("gradient", C.c_int)]
 
 
 class MfsCtxOptions(C.Structure):
@@ -115,6 +122,7 @@ _SIGS = {
     "mfs_upload": (C.c_int, [C.c_void_p, C.c_int, _DP, C.c_size_t]),
     "mfs_get_scalars": (C.c_int, [C.c_void_p, C.POINTER(MfsScalars)]),
     "mfs_ctx_get_info": (C.c_int, [C.c_void_p, C.POINTER(MfsCtxInfo)]),
+    "mfs_ctx_get_launches": (C.c_int, [C.c_void_p, C.POINTER(MfsCtxLaunches)]),
     "mfs_ctx_enable_timing": (C.c_int, [C.c_void_p, C.c_int]),
     "mfs_ctx_get_timing": (C.c_int, [C.c_void_p, C.c_char_p, _DP, _IP]),
     "mfs_ctx_reset_timing": (C.c_int, [C.c_void_p]),

@@ -785,10 +785,39 @@ bool sweep_split(const mfs_ctx* ctx) {
     return !ctx->sweep_by_tiles && ctx->tail_grid > 0 && ctx->tail_chunks > 0;
 }
 
-// Workgroups of the thin-tail launch of a split sweep.
+// Whether the sweeps run whole on one XCD: a mesh of thin levels only.
+bool sweep_local(const mfs_ctx* ctx) { return !ctx->sweep_by_tiles && !sweep_split(ctx) && ctx->all_thin; }
+
+// Whether each sweep has a launch of thin levels, on one XCD.
+bool thin_launch(const mfs_ctx* ctx) { return sweep_split(ctx) || sweep_local(ctx); }
+
+// Workgroups, of sweep_waves waves, of a launch on the resident grid.
+int sweep_workgroups(const mfs_ctx* ctx) {
+    const int chunks = std::max(ctx->sweep[0].nchunk, ctx->sweep[1].nchunk);
+    const int units = ctx->sweep_by_tiles ? ctx->ntiles : (chunks + ctx->sweep_waves - 1) / ctx->sweep_waves;
+    return std::max(1, std::min(ctx->sweep_grid, units));
+}
+
+// The tail grid of a split sweep, in groups of kThinWaves waves.
 int tail_workgroups(const mfs_ctx* ctx) {
     const int units = (ctx->tail_chunks + ctx->sweep_waves - 1) / ctx->sweep_waves;
     return std::max(1, std::min({ctx->tail_grid, ctx->sweep_grid, units}));
+}
+
+// Workgroups of kBlock threads that sweep in a launch of thin levels: enough
+// for the waves of the tail grid, or of the default one where each sweep is
+// such a launch whole.
+int thin_workgroups(const mfs_ctx* ctx) {
+    constexpr int W = kBlock / 64;
+    const int g = sweep_split(ctx) ? tail_workgroups(ctx) : std::min(sweep_workgroups(ctx), dev::kDefaultTailGrid);
+    return (g * dev::kThinWaves + W - 1) / W;
+}
+
+// Whether mfs_step's gradients run inside the launches of thin levels
+// (timing every kernel group needs them in launches of their own).
+bool gradient_inside(const mfs_ctx* ctx) {
+    return ctx->gstream && ctx->gradient_stream == 5 && thin_launch(ctx) && ctx->timing != 1 &&
+           ctx->nC <= (long long)dev::kSideCellsPerLevel * ctx->thin_levels;
 }
 
 // The sweeps' arguments for an iteration that starts from state buffer `cur`;
@@ -830,9 +859,6 @@ void sweep_args(dev::SweepArgs<R>& A, const mfs_ctx* ctx, int cur) {
     A.err = ctx->err;
     A.cell0 = ctx->cell0;
 }
-
-// Whether each sweep has a launch of thin levels, on one XCD.
-bool thin_launch(const mfs_ctx* ctx) { return sweep_split(ctx) || (!ctx->sweep_by_tiles && ctx->all_thin); }
 
 // Symmetry-plane projection of the node values.
 template <typename R>
@@ -908,17 +934,13 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     sweep_args(A, ctx, ctx->cur);
     const bool flat = !ctx->sweep_by_tiles;
     const int nf = ctx->sweep[0].nchunk, nb = ctx->sweep[1].nchunk;
-    const int units = flat ? (std::max(nf, nb) + ctx->sweep_waves - 1) / ctx->sweep_waves : A.ntiles;
-    const dim3 grid((unsigned)std::max(1, std::min(ctx->sweep_grid, units)));
+    const dim3 grid((unsigned)sweep_workgroups(ctx));
     // A split sweep runs its wide levels on the resident grid and its thin
     // tail on a small one: the forward sweep ends with the tail and the
-    // backward sweep starts with it.
-    const bool split = sweep_split(ctx);
+    // backward sweep starts with it.  A mesh of thin levels only runs its
+    // sweeps on one XCD whole.
+    const bool split = sweep_split(ctx), local = sweep_local(ctx);
     const int wf = nf - ctx->sweep[0].tail, tb = ctx->sweep[1].tail;  // forward: wide chunks; backward: tail chunks
-    const dim3 tgrid((unsigned)(split ? tail_workgroups(ctx) : 1));
-    // A mesh of thin levels only runs its sweeps on one XCD whole.
-    const bool local = flat && !split && ctx->all_thin;
-    const dim3 lgrid(std::min<unsigned>(grid.x, dev::kDefaultTailGrid));
     // Each launch takes its tickets from one counter set and zeroes the
     // other for the next launch.  The launches of an iteration alternate
     // between the two sets and are even in number, so every iteration's
@@ -926,26 +948,25 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
     int* const tk[2] = {ctx->tickets, ctx->tickets + kTicketGroups * kTicketStride};
     int set = 0;
     // ev0 / ev1: the timing events that this launch's start / end set
-    auto launch = [&](const void* fn, bool fwd, bool thin, dim3 g, int ubeg, int uend, const char* what, hipEvent_t ev0,
+    auto launch = [&](const void* fn, bool fwd, bool thin, int ubeg, int uend, const char* what, hipEvent_t ev0,
                       hipEvent_t ev1) {
         A.ubeg = ubeg;
         A.uend = uend;
-        A.ngroups = std::min(kTicketGroups, (int)g.x);
+        A.ngroups = std::min(kTicketGroups, (int)grid.x);
         A.run_shift = dev::kWideRunShift;
         A.tickets = tk[set];
         A.tickets_next = tk[1 - set];
         set ^= 1;
         if (!thin) {
             void* args[] = {&A, &ctx->K};
-            return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(64 * ctx->sweep_waves), args,
+            return hip_ok(ctx, hipExtLaunchKernel(fn, grid, dim3(64 * ctx->sweep_waves), args,
                                                  dev::stage_bytes(ctx->sweep_waves), ctx->stream, ev0, ev1, 0), what);
         }
-        // the tail grid's waves on one XCD; with side work, workgroups for
-        // every CU
-        constexpr int W = kBlock / 64;
-        const int join = std::max(1, ((int)g.x * dev::kThinWaves + W - 1) / W);
+        // as many workgroups on every XCD as sweep on one; with side work,
+        // workgroups for every CU
+        const int join = thin_workgroups(ctx);
         dev::XcdArgs<R> P{A, ctx->K, side_work<R>(ctx, fwd, grad_q), join};
-        g.x = (unsigned)(join * dev::kXcd);
+        dim3 g((unsigned)(join * dev::kXcd));
         if (P.W.nblk > 0) {
             const int most = (int)g.x + P.W.nblk;
             const bool few = fwd || ctx->nC <= (long long)dev::kSideFewCellsPerLevel * ctx->thin_levels;
@@ -953,7 +974,8 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
             g.x = std::max<unsigned>(g.x, (unsigned)std::min(groups * ctx->compute_units, most));
         }
         void* args[] = {&P};
-        return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(kBlock), args, dev::stage_bytes(W), ctx->stream, ev0, ev1, 0),
+        return hip_ok(ctx, hipExtLaunchKernel(fn, g, dim3(kBlock), args, dev::stage_bytes(kBlock / 64), ctx->stream, ev0, ev1,
+                                             0),
                       what);
     };
     SweepTurn turn(ctx->device, ctx->stream);
@@ -964,13 +986,13 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
                           : flat ? (const void*)dev::k_sweep<true, MAXD, R, dev::kAnyChunks>
                                  : (const void*)dev::k_sweep_tiles<true, MAXD, R>;
         if (split) {
-            if (!launch((const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>, true, false, grid, 0, wf, "k_sweep<fwd>",
+            if (!launch((const void*)dev::k_sweep<true, MAXD, R, dev::kWideChunks>, true, false, 0, wf, "k_sweep<fwd>",
                         t.start(0), t.stop(0)))
                 return false;
             if (at_tail && after && !after()) return false;
-            if (!launch((const void*)dev::k_sweep_xcd<true, MAXD, R>, true, true, tgrid, wf, nf, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
+            if (!launch((const void*)dev::k_sweep_xcd<true, MAXD, R>, true, true, wf, nf, "k_sweep<fwd> (thin tail)", t.start(1), t.stop(1)))
                 return false;
-        } else if (!launch(fwd, true, local, local ? lgrid : grid, 0, nf, "k_sweep<fwd>", t.start(0), t.stop(0))) {
+        } else if (!launch(fwd, true, local, 0, nf, "k_sweep<fwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("fwd_sweep", "fwd_sweep_wide", "fwd_sweep_tail");
@@ -983,12 +1005,12 @@ bool launch_sweeps_t(mfs_ctx* ctx, const std::function<bool()>& after, bool at_t
                           : flat ? (const void*)dev::k_sweep<false, MAXD, R, dev::kAnyChunks>
                                  : (const void*)dev::k_sweep_tiles<false, MAXD, R>;
         if (split) {
-            if (!launch((const void*)dev::k_sweep_xcd<false, MAXD, R>, false, true, tgrid, 0, tb,
+            if (!launch((const void*)dev::k_sweep_xcd<false, MAXD, R>, false, true, 0, tb,
                         "k_sweep<bwd> (thin tail)", t.start(0), t.stop(0)) ||
-                !launch((const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>, false, false, grid, tb, nb, "k_sweep<bwd>",
+                !launch((const void*)dev::k_sweep<false, MAXD, R, dev::kWideChunks>, false, false, tb, nb, "k_sweep<bwd>",
                         t.start(1), t.stop(1)))
                 return false;
-        } else if (!launch(bwd, false, local, local ? lgrid : grid, 0, nb, "k_sweep<bwd>", t.start(0), t.stop(0))) {
+        } else if (!launch(bwd, false, local, 0, nb, "k_sweep<bwd>", t.start(0), t.stop(0))) {
             return false;
         }
         t.done("bwd_sweep", "bwd_sweep_tail", "bwd_sweep_wide");
@@ -1591,10 +1613,8 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
     const bool side = mode >= 2;
     const bool fuse = !side && gradient_fuses_next(ctx);
     // Mode 5 with thin launches: the pending gradient is their side work, on
-    // the solver stream.  (Timing every kernel group needs it in launches of
-    // its own.)
-    const bool inside = mode == 5 && thin_launch(ctx) && ctx->timing != 1 &&
-                        ctx->nC <= (long long)dev::kSideCellsPerLevel * ctx->thin_levels;
+    // the solver stream.
+    const bool inside = gradient_inside(ctx);
     const double* grad_q = nullptr;  // state of the gradient not yet launched
     int grad_par = 0;
     // records `ev` on the solver stream and starts the pending gradient
@@ -1931,14 +1951,30 @@ extern "C" int mfs_ctx_get_info(mfs_ctx* ctx, mfs_ctx_info* info) {
     info->tile_cells = ctx->tile_cells;
     info->sweep_waves = ctx->sweep_waves;
     info->sweep_tiles = ctx->ntiles;
-    const int chunks = std::max(ctx->sweep[0].nchunk, ctx->sweep[1].nchunk);
-    info->sweep_workgroups =
-        std::min(ctx->sweep_grid, ctx->sweep_by_tiles ? ctx->ntiles : (chunks + ctx->sweep_waves - 1) / ctx->sweep_waves);
+    info->sweep_workgroups = sweep_workgroups(ctx);
     info->sweep_by_tiles = ctx->sweep_by_tiles;
     info->compute_units = ctx->compute_units;
     info->sweep_tail_chunks = ctx->tail_grid > 0 ? ctx->tail_chunks : 0;
     info->sweep_tail_cells = ctx->tail_grid > 0 ? ctx->tail_cells : 0;
     info->sweep_tail_workgroups = ctx->tail_grid > 0 ? tail_workgroups(ctx) : 0;
+    return MFS_OK;
+}
+
+extern "C" int mfs_ctx_get_launches(mfs_ctx* ctx, mfs_ctx_launches* out) {
+    if (!ctx || !out) {
+        set_error("mfs_ctx_get_launches: bad argument");
+        return MFS_ERR_ARG;
+    }
+    const bool split = sweep_split(ctx), local = sweep_local(ctx);
+    out->thin_launch = split ? 1 : local ? 2 : 0;
+    out->thin_workgroups = split || local ? thin_workgroups(ctx) : 0;
+    out->thin_levels = split || local ? ctx->thin_levels : 0;
+    out->wide_workgroups = local ? 0 : sweep_workgroups(ctx);
+    for (int d = 0; d < 2; ++d) {
+        out->chunks[d] = ctx->sweep[d].nchunk;
+        out->thin_chunks[d] = local ? ctx->sweep[d].nchunk : split ? ctx->sweep[d].tail : 0;
+    }
+    out->gradient = gradient_inside(ctx) ? MFS_GRADIENT_INSIDE : ctx->gstream ? ctx->gradient_stream : 1;
     return MFS_OK;
 }
 
