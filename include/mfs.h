@@ -224,6 +224,12 @@ int mfs_step(mfs_ctx* ctx, int n);
  * shares that GPU's array: calls that overlap on one GPU (contexts stepped
  * from several threads at once) race and must be serialised by the caller. */
 int mfs_step_noalloc(mfs_ctx* ctx, int n, double* hist_dev);
+/* Whether mfs_step and mfs_step_noalloc end with the gradient of their last
+ * iteration (default 1).  With 0 the gradient fields hold the iteration
+ * before's, as its own place in the schedule left them (those of a call of one
+ * iteration stay as they were); nothing else changes.  No counterpart in the
+ * reference. */
+int mfs_ctx_set_last_gradient(mfs_ctx* ctx, int enable);
 int mfs_sync(mfs_ctx* ctx);
 
 /* Per-iteration history: record k = {norm_rho, norm_mx, norm_my, norm_mz,

@@ -168,6 +168,11 @@ class Solver:
         main.cpp:283 leaves commented out)."""
         check(lib().mfs_ctx_set_ghost_refresh(self._h, 1 if on else 0), "mfs_ctx_set_ghost_refresh")
 
+    def last_gradient(self, on: bool = True):
+        """Make step() end with its last iteration's gradient (the default),
+        or leave the gradient fields with the iteration before's."""
+        check(lib().mfs_ctx_set_last_gradient(self._h, 1 if on else 0), "mfs_ctx_set_last_gradient")
+
     def calculate_gradient(self):
         check(lib().mfs_calculate_gradient(self._h), "mfs_calculate_gradient")
 

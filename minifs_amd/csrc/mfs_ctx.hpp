@@ -104,6 +104,7 @@ struct mfs_ctx {
     double* sdn = nullptr;   // per slot and cell: |(x_fc - x_cc).n| on this cell's side
     int* sflip = nullptr;    // per cell: slots whose face has this cell second (bits 0-7), face count (8-11)
     int ghost_refresh = 0;   // SetGhostVariables after each update in mfs_step
+    bool last_gradient = true;  // mfs_step ends with its last iteration's gradient
     // mfs_step's gradient on a second stream (gradient_stream options 2-5):
     // iteration k's node values and gradient run beside iteration k+1's
     // residual pass and sweeps.  sdone: recorded on `stream` where the

@@ -1575,6 +1575,15 @@ extern "C" int mfs_set_ghost_variables(mfs_ctx* ctx) {
     return launch_ghosts(ctx) ? MFS_OK : MFS_ERR_HIP;
 }
 
+extern "C" int mfs_ctx_set_last_gradient(mfs_ctx* ctx, int enable) {
+    if (!ctx) {
+        set_error("null context");
+        return MFS_ERR_ARG;
+    }
+    ctx->last_gradient = enable != 0;
+    return MFS_OK;
+}
+
 extern "C" int mfs_ctx_set_ghost_refresh(mfs_ctx* ctx, int enable) {
     if (!ctx) {
         set_error("mfs_ctx_set_ghost_refresh: null context");
@@ -1617,6 +1626,7 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
     const bool inside = gradient_inside(ctx);
     const double* grad_q = nullptr;  // state of the gradient not yet launched
     int grad_par = 0;
+    int joins = -1;  // parity of the latest gradient on the second stream
     // records `ev` on the solver stream and starts the pending gradient
     // behind it on the second stream
     auto side_gradient = [&](hipEvent_t ev) -> bool {
@@ -1627,6 +1637,7 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
             !hip_ok(ctx, hipEventRecord(ctx->gdone[grad_par], ctx->gstream), "record gradient"))
             return false;
         ctx->gpend[grad_par] = true;
+        joins = grad_par;
         grad_q = nullptr;
         return true;
     };
@@ -1660,25 +1671,24 @@ int step_iterations(mfs_ctx* ctx, int nsteps) {
         // SetGhostVariables, when enabled (main.cpp:283 has the call commented out)
         if (ctx->ghost_refresh && !launch_ghosts(ctx)) return MFS_ERR_HIP;
         // CalculateGradient (fused: with the next iteration's first pass)
-        if (inside) {
-            grad_q = ctx->q[ctx->cur];
-            if (s + 1 == nsteps && !launch_gradient(ctx)) return MFS_ERR_HIP;
-        } else if (side) {
+        const bool last = s + 1 == nsteps;
+        if (side) {
             grad_q = ctx->q[ctx->cur];
             grad_par = par;
-            if ((mode == 2 || s + 1 == nsteps) && !side_gradient(ctx->sdone)) return MFS_ERR_HIP;
-        } else {
-            const bool next = fuse && s + 1 < nsteps;
+            if (last ? ctx->last_gradient && !(inside ? launch_gradient(ctx) : side_gradient(ctx->sdone))
+                     : mode == 2 && !side_gradient(ctx->sdone))
+                return MFS_ERR_HIP;
+        } else if (!last || ctx->last_gradient) {
+            const bool next = fuse && !last;
             if (!launch_gradient(ctx, next, next ? cfl_of_iter(ctx->P, ctx->iter_done + 1) : 0.0)) return MFS_ERR_HIP;
         }
         ctx->hist_n++;
         ctx->iter_done++;
     }
-    if (side && !inside && nsteps > 0) {
+    if (joins >= 0) {
         // join: everything later on the solver stream (entry points,
         // downloads, mfs_sync) comes after the last gradient
-        const int last = (ctx->iter_done - 1) & 1;
-        if (!hip_ok(ctx, hipStreamWaitEvent(ctx->stream, ctx->gdone[last], 0), "join gradient")) return MFS_ERR_HIP;
+        if (!hip_ok(ctx, hipStreamWaitEvent(ctx->stream, ctx->gdone[joins], 0), "join gradient")) return MFS_ERR_HIP;
         ctx->gpend[0] = ctx->gpend[1] = false;
     }
     return MFS_OK;

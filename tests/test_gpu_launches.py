@@ -50,3 +50,90 @@ def test_launches(cells, n, opts, thin, workgroups, gradient):
     assert s.launches()["gradient"] == min(gradient, 5)
     s.close()
     g.close()
+
+
+def _remapped(tmp_path, dims, tree, bc_text, p):
+    """A tetrahedral box whose two patches take other boundary types."""
+    g0 = mfs.Grid.box_bump(*dims, seed=4).decouple(*tree)
+    mesh, bc = str(tmp_path / "m.mfl"), str(tmp_path / "m.bc")
+    g0.save(mesh, bc)
+    g0.close()
+    open(bc, "w").write(bc_text)
+    return mfs.Grid.load(mesh, bc).preprocess(p)
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("cells,dims,tree,ghosts,thin", [("tet", (1, 1, 1), (4, 512), False, 2),
+                                                         ("tet", (9, 7, 8), (4, 512), True, 2),
+                                                         ("tet", (23, 20, 22), (4, 512), True, 1),
+                                                         ("tet", (40, 40, 40), (4, 512), False, 1),
+                                                         ("tet", (40, 40, 40), (2, 64), False, 1),
+                                                         ("symm", (22, 21, 20), (4, 512), False, 1),
+                                                         ("hex", (8, 9, 7), (4, 512), False, 2),
+                                                         ("hex", (43, 41, 40), (4, 512), True, 1),
+                                                         ("hex", (72, 70, 71), (2, 32), False, 1),
+                                                         ("prism", (33, 30, 31), (4, 512), False, 1)])
+def test_gradient_written_inside_the_thin_launches(tmp_path, cells, dims, tree, ghosts, thin, precision):
+    """The node values and gradients that the side work of the thin launches
+    writes, left by calls without their last gradient, are those of the
+    iteration before as launches of their own write them: bit for bit, for
+    tails and sweeps run whole, few and many cells per thin level, symmetry
+    nodes, and calls of different lengths after one another."""
+    print(f"[launches] gradient inside {cells} {dims} {tree} ghosts={ghosts} precision={precision}", flush=True)
+    p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0)
+    if cells == "symm":
+        g = _remapped(tmp_path, dims, tree, "2\n1 4\n2 6\n", p)
+    else:
+        g, p = _grid(cells, dims, tree)
+    a, b = mfs.Solver(g, p, precision=precision), mfs.Solver(g, p, precision=precision, gradient_stream=1)
+    assert a.launches()["gradient"] == MFS_GRADIENT_INSIDE and a.launches()["thin_launch"] == thin
+    assert b.launches()["gradient"] == 1
+    a.last_gradient(False)
+    for s in (a, b):
+        s.ghost_refresh(ghosts)
+    before = a.field("dqdx")
+    a.step(1)  # has no gradient but its last
+    b.step(1)
+    np.testing.assert_array_equal(a.field("dqdx"), before)
+    for n in (2, 3, 5, 2):
+        a.step(n)
+        b.step(n - 1)
+        for nm in ("qnode", "dqdx", "dqdy", "dqdz"):
+            np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=f"{n}: {nm}")
+        assert not np.array_equal(a.field("dqdx"), before)
+        before = a.field("dqdx")
+        b.step(1)
+        np.testing.assert_array_equal(a.field("rho"), b.field("rho"), err_msg=f"{n}")
+    a.last_gradient(True)
+    a.step(2)
+    b.step(2)
+    for nm in FIELDS:
+        np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=nm)
+    a.close()
+    b.close()
+    g.close()
+
+
+@pytest.mark.parametrize("stream", [1, 2, 3, 4, 5])
+def test_last_gradient_left_out_on_every_stream(stream):
+    """Without its last gradient a call on any of the gradient's streams ends
+    with the iteration before's gradient, and everything else as with it."""
+    print(f"[launches] last gradient left out, stream {stream}", flush=True)
+    g, p = _grid("tet", (12, 11, 13), (4, 512))
+    a = mfs.Solver(g, p, gradient_stream=stream, sweep_by_tiles=1 if stream == 5 else 0)
+    b = mfs.Solver(g, p, gradient_stream=1)
+    assert a.launches()["gradient"] == stream
+    a.last_gradient(False)
+    for n in (1, 4, 2):
+        a.step(n)
+        b.step(n - 1)
+        if n > 1:
+            for nm in ("qnode", "dqdx", "dqdy", "dqdz"):
+                np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=f"{n}: {nm}")
+        b.step(1)
+        for nm in ("rho", "u", "v", "w", "p", "res", "dq"):
+            np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=f"{n}: {nm}")
+    np.testing.assert_array_equal(a.history(), b.history())
+    a.close()
+    b.close()
+    g.close()
