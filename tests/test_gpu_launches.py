@@ -137,3 +137,38 @@ def test_last_gradient_left_out_on_every_stream(stream):
     a.close()
     b.close()
     g.close()
+
+
+@pytest.mark.parametrize("cells,dims,tree,precision,ghosts",
+                         [("tet", (57, 55, 56), (2, 64), mfs.MFS_FP64, False),
+                          ("tet", (57, 55, 56), (2, 64), mfs.MFS_MIXED, False),
+                          ("tet", (57, 55, 56), (2, 64), mfs.MFS_MIXED, True),
+                          ("tet", (57, 55, 56), (2, 64), mfs.MFS_FP64, True),
+                          ("hex", (100, 99, 101), (2, 32), mfs.MFS_MIXED, True),
+                          ("prism", (80, 81, 79), (2, 16), mfs.MFS_FP64, False)])
+def test_second_stream_gradient_beside_a_split_sweep(cells, dims, tree, precision, ghosts):
+    """Shallow orders, whose tails are too short to hide the gradient: it
+    starts on the second stream between a sweep's wide launch and its tail.
+    Every field and history record equals the solver stream's, across calls
+    and with the entry points in between."""
+    print(f"[launches] second stream {cells} {dims} {tree} precision={precision} ghosts={ghosts}", flush=True)
+    g, p = _grid(cells, dims, tree)
+    a, b = (mfs.Solver(g, p, precision=precision, gradient_stream=k) for k in (5, 1))
+    assert a.launches()["gradient"] == 5 and a.launches()["thin_launch"] == 1
+    for s in (a, b):
+        s.ghost_refresh(ghosts)
+        s.step(3)
+        s.step(1)
+        s.iterate_reference_order(1)
+        s.step(2)
+    for nm in FIELDS:
+        np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=nm)
+    np.testing.assert_array_equal(a.history(), b.history())
+    a.last_gradient(False)
+    a.step(3)
+    b.step(2)
+    for nm in ("qnode", "dqdx", "dqdy", "dqdz"):
+        np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=nm)
+    a.close()
+    b.close()
+    g.close()
