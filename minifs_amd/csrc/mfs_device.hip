@@ -9,12 +9,10 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <functional>
 #include <mutex>
 #include <sstream>
-#include <thread>
 #include <vector>
 #include <cstdio>
 #include <cstring>
@@ -24,6 +22,7 @@
 #include "mfs_ctx.hpp"
 #include "mfs_mesh.hpp"
 #include "mfs_grid.hpp"
+#include "mfs_io.hpp"
 #include "mfs_prep.hpp"
 
 #include <hipcub/hipcub.hpp>
@@ -555,98 +554,17 @@ void* noalloc_scratch(int device) {
     return g_noalloc_scratch[device];
 }
 
-// ---------------------------------------------------------------------------
-// Staging of downloads and uploads.  A field crosses in chunks: a kernel
-// reorders a chunk on the device, one copy moves it between a device slot and
-// a pinned host slot, and a host thread copies between the slot and the
-// caller's array, which is pageable and often not yet backed by memory (its
-// page faults are most of a large download's host time).  Several threads
-// work chunks at once, each with a slot, so that the reorder, the link and
-// the host's copies overlap.  Before, one host thread scattered the whole
-// field out of a pageable copy of its device array: the five state fields of
-// 6.0M cells took 340 ms and the three gradients 238.
-// Now they take 10 and 22 ms, and uploading the five state fields 10 instead
-// of 430 (in part the reads and writes of whole state buffers per field).
-//
-// The slots of a device are shared by its contexts (one download or upload at
-// a time), allocated as chunks need them and freed with the device's last
-// context.
-constexpr int kIoSlots = 8;
-constexpr size_t kIoValues = (size_t)1 << 18;  // values per chunk (2 MiB)
-struct IoSlot {
-    double *host = nullptr, *dev = nullptr;
-    hipEvent_t done = nullptr;
-};
-struct IoPool {
-    std::mutex mu;  // held for a whole download or upload
-    int users = 0;
-    IoSlot slot[kIoSlots];
-};
+// The staging slots of downloads and uploads, per device.
 IoPool* const g_io = new IoPool[kMaxDevices];  // never freed, as the sweep order table
 
 void io_join(mfs_ctx* ctx) {
-    IoPool& P = g_io[ctx->device];
-    std::lock_guard<std::mutex> lk(P.mu);
-    ++P.users;
+    g_io[ctx->device].join();
     ctx->io_member = true;
 }
 void io_leave(mfs_ctx* ctx) {
     if (!ctx->io_member) return;
     ctx->io_member = false;
-    IoPool& P = g_io[ctx->device];
-    std::lock_guard<std::mutex> lk(P.mu);
-    if (--P.users > 0) return;
-    for (IoSlot& s : P.slot) {
-        if (s.host) (void)hipHostFree(s.host);
-        if (s.dev) (void)hipFree(s.dev);
-        if (s.done) (void)hipEventDestroy(s.done);
-        s = IoSlot{};
-    }
-}
-
-// Moves `count` values, chunk by chunk: move(slot, first value, values)
-// enqueues a chunk's work on the context's stream, up to the record of the
-// slot's event, and finish(slot, first, values) does its host part after the
-// event.  Returns the first error.
-template <typename Move, typename Finish>
-hipError_t io_chunks(mfs_ctx* ctx, size_t count, Move&& move, Finish&& finish) {
-    IoPool& P = g_io[ctx->device];
-    std::lock_guard<std::mutex> lk(P.mu);
-    const size_t chunks = (count + kIoValues - 1) / kIoValues;
-    std::atomic<size_t> next{0};
-    std::atomic<int> failed{(int)hipSuccess};
-    auto work = [&](int k) {
-        hipError_t e = hipSetDevice(ctx->device);
-        IoSlot& s = P.slot[k];
-        auto stop = [&] {
-            if (e == hipSuccess) return false;
-            int none = (int)hipSuccess;
-            failed.compare_exchange_strong(none, (int)e);
-            return true;
-        };
-        while (!stop() && failed.load() == (int)hipSuccess) {
-            const size_t c = next.fetch_add(1);
-            if (c >= chunks) return;
-            if (!s.host) e = hipHostMalloc((void**)&s.host, kIoValues * sizeof(double));
-            if (e == hipSuccess && !s.dev) e = hipMalloc((void**)&s.dev, kIoValues * sizeof(double));
-            if (e == hipSuccess && !s.done) e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
-            const size_t t0 = c * kIoValues, n = std::min(kIoValues, count - t0);
-            if (e == hipSuccess) e = move(s, t0, n);
-            if (e == hipSuccess) e = hipEventSynchronize(s.done);
-            if (e == hipSuccess) finish(s, t0, n);
-        }
-    };
-    const int threads = (int)std::min<size_t>(
-        {(size_t)kIoSlots, chunks, std::max<size_t>(1, std::thread::hardware_concurrency())});
-    std::vector<std::thread> th;
-    try {
-        th.reserve(threads);
-        for (int k = 1; k < threads; ++k) th.emplace_back(work, k);
-    } catch (...) {  // fewer helpers: the calling thread takes every chunk that is left
-    }
-    work(0);
-    for (auto& t : th) t.join();
-    return (hipError_t)failed.load();
+    g_io[ctx->device].leave();
 }
 
 double cfl_of_iter(const mfs_params& P, int iter_done) {
@@ -1878,8 +1796,8 @@ extern "C" int mfs_download(mfs_ctx* ctx, int field, double* dst, size_t count) 
     int r = mfs_sync(ctx);
     if (r != MFS_OK) return r;
     const dev::FieldMap M = field_map(ctx, f);
-    const hipError_t e = io_chunks(
-        ctx, count,
+    const hipError_t e = g_io[ctx->device].transfer(
+        ctx->device, ctx->stream, count,
         [&](IoSlot& s, size_t t0, size_t n) {
             hipLaunchKernelGGL(dev::k_field_out, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, M, t0, n, f.dev, f.dev32,
                                s.dev);
@@ -1910,8 +1828,8 @@ extern "C" int mfs_upload(mfs_ctx* ctx, int field, const double* src, size_t cou
                           hipMemcpyAsync(second, f.dev, sizeof(double) * all, hipMemcpyDeviceToDevice, ctx->stream),
                           "upload state"))
         return MFS_ERR_HIP;
-    const hipError_t e = io_chunks(
-        ctx, count,
+    const hipError_t e = g_io[ctx->device].transfer(
+        ctx->device, ctx->stream, count,
         [&](IoSlot& s, size_t t0, size_t n) {
             std::memcpy(s.host, src + t0, n * sizeof(double));
             hipError_t e = hipMemcpyAsync(s.dev, s.host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
