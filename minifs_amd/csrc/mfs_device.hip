@@ -664,6 +664,14 @@ size_t partial_doubles(int nblk) {
     return std::max<size_t>(8 * (size_t)nblk, 7 * (size_t)nblk + 7 * (size_t)dev::kReduceBlock);
 }
 
+// IoPool::transfer on the context's stream, whose work has ended: the
+// residual pass's partials are idle until the next one writes them.
+template <typename Move, typename Finish>
+hipError_t io_transfer(mfs_ctx* ctx, size_t count, Move&& move, Finish&& finish) {
+    return g_io[ctx->device].transfer(ctx->device, ctx->stream, count, ctx->part, partial_doubles(ctx->nblk_cell), move,
+                                      finish);
+}
+
 bool launch_reduce(mfs_ctx* ctx, int mode, int slot) {
     Timed t(ctx, "reduce");
     const int nb = (int)ctx->nblk_cell;
@@ -1796,15 +1804,15 @@ extern "C" int mfs_download(mfs_ctx* ctx, int field, double* dst, size_t count) 
     int r = mfs_sync(ctx);
     if (r != MFS_OK) return r;
     const dev::FieldMap M = field_map(ctx, f);
-    const hipError_t e = g_io[ctx->device].transfer(
-        ctx->device, ctx->stream, count,
+    const hipError_t e = io_transfer(
+        ctx, count,
         [&](IoSlot& s, size_t t0, size_t n) {
             hipLaunchKernelGGL(dev::k_field_out, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, M, t0, n, f.dev, f.dev32,
                                s.dev);
-            hipError_t e = hipGetLastError();
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(s.host, s.dev, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream);
-            return e == hipSuccess ? hipEventRecord(s.done, ctx->stream) : e;
+            const hipError_t e = hipGetLastError();
+            return e == hipSuccess
+                       ? hipMemcpyAsync(s.host, s.dev, n * sizeof(double), hipMemcpyDeviceToHost, ctx->stream)
+                       : e;
         },
         [&](IoSlot& s, size_t t0, size_t n) { std::memcpy(dst + t0, s.host, n * sizeof(double)); });
     return hip_ok(ctx, e, "download") ? MFS_OK : MFS_ERR_HIP;
@@ -1828,16 +1836,15 @@ extern "C" int mfs_upload(mfs_ctx* ctx, int field, const double* src, size_t cou
                           hipMemcpyAsync(second, f.dev, sizeof(double) * all, hipMemcpyDeviceToDevice, ctx->stream),
                           "upload state"))
         return MFS_ERR_HIP;
-    const hipError_t e = g_io[ctx->device].transfer(
-        ctx->device, ctx->stream, count,
+    const hipError_t e = io_transfer(
+        ctx, count,
         [&](IoSlot& s, size_t t0, size_t n) {
             std::memcpy(s.host, src + t0, n * sizeof(double));
-            hipError_t e = hipMemcpyAsync(s.dev, s.host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
+            const hipError_t e = hipMemcpyAsync(s.dev, s.host, n * sizeof(double), hipMemcpyHostToDevice, ctx->stream);
             if (e != hipSuccess) return e;
             hipLaunchKernelGGL(dev::k_field_in, dim3(nblk(n)), dim3(kBlock), 0, ctx->stream, M, t0, n, s.dev, f.dev,
                                second);
-            e = hipGetLastError();
-            return e == hipSuccess ? hipEventRecord(s.done, ctx->stream) : e;
+            return hipGetLastError();
         },
         [](IoSlot&, size_t, size_t) {});
     if (!hip_ok(ctx, e, "upload")) return MFS_ERR_HIP;

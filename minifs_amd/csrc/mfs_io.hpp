@@ -27,7 +27,7 @@ constexpr int kIoSlots = 8;
 constexpr size_t kIoValues = (size_t)1 << 18;  // values per chunk (2 MiB)
 struct IoSlot {
     double *host = nullptr, *dev = nullptr;
-    hipEvent_t done = nullptr;
+    hipEvent_t done = nullptr;  // set: the slot has its memory
     bool taken = false;
 };
 
@@ -43,40 +43,49 @@ class IoPool {
     void leave() {
         std::lock_guard<std::mutex> lk(mu_);
         if (--users_ > 0) return;
-        for (IoSlot& s : slot_) {
-            if (s.host) (void)hipHostFree(s.host);
-            if (s.dev) (void)hipFree(s.dev);
-            if (s.done) (void)hipEventDestroy(s.done);
-            s = IoSlot{};
-        }
+        for (IoSlot& s : slot_) strip(s);
     }
     // Moves `count` values of a context on `device`, chunk by chunk:
-    // move(slot, first value, values) enqueues a chunk's work on `stream`, up
-    // to the record of the slot's event, and finish(slot, first, values) does
-    // its host part after the event.  Returns the first error.
+    // move(slot, first value, values) enqueues a chunk's work on `stream` and
+    // finish(slot, first, values) does its host part after it.  Returns the
+    // first error.  Where there is no memory for further slots the threads
+    // share those there are; without any the calling thread goes through
+    // `spare`, device memory of spare_values values that the context has idle,
+    // and pageable memory.
     template <typename Move, typename Finish>
-    hipError_t transfer(int device, hipStream_t stream, size_t count, Move&& move, Finish&& finish) {
+    hipError_t transfer(int device, hipStream_t stream, size_t count, double* spare, size_t spare_values, Move&& move,
+                        Finish&& finish) {
         const size_t chunks = (count + kIoValues - 1) / kIoValues;
         std::atomic<size_t> next{0};
         std::atomic<int> failed{(int)hipSuccess};
+        std::atomic<bool> more{true}, none{false};  // memory for further slots; no slot at all
         auto work = [&] {
             hipError_t e = hipSetDevice(device);
-            while (e == hipSuccess && failed.load() == (int)hipSuccess) {
+            while (e == hipSuccess && failed.load() == (int)hipSuccess && !none) {
                 const size_t c = next.fetch_add(1);
                 if (c >= chunks) return;
-                IoSlot& s = take();
-                e = complete(s);
+                IoSlot* s = take(more);
+                if (s && !complete(*s)) {
+                    more = false;
+                    put(*s);
+                    s = take(false);
+                }
+                if (!s) {
+                    none = true;
+                    return;
+                }
                 const size_t t0 = c * kIoValues, n = std::min(kIoValues, count - t0);
-                if (e == hipSuccess) e = move(s, t0, n);
-                if (e == hipSuccess) e = hipEventSynchronize(s.done);
+                e = move(*s, t0, n);
+                if (e == hipSuccess) e = hipEventRecord(s->done, stream);
+                if (e == hipSuccess) e = hipEventSynchronize(s->done);
                 if (e == hipSuccess)
-                    finish(s, t0, n);
+                    finish(*s, t0, n);
                 else
                     (void)hipStreamSynchronize(stream);  // nothing enqueued touches the slot any more
-                put(s);
+                put(*s);
             }
-            int none = (int)hipSuccess;
-            if (e != hipSuccess) failed.compare_exchange_strong(none, (int)e);
+            int unset = (int)hipSuccess;
+            if (e != hipSuccess) failed.compare_exchange_strong(unset, (int)e);
         };
         const int threads =
             (int)std::min<size_t>({(size_t)kIoSlots, chunks, std::max<size_t>(1, std::thread::hardware_concurrency())});
@@ -88,21 +97,45 @@ class IoPool {
         }
         work();
         for (auto& t : th) t.join();
-        return (hipError_t)failed.load();
+        hipError_t e = (hipError_t)failed.load();
+        if (!none || e != hipSuccess) return e;
+        std::lock_guard<std::mutex> lk(spare_mu_);  // two transfers of one context share its spare memory
+        std::vector<double> host;
+        try {
+            host.resize(std::min(count, spare_values));
+        } catch (...) {
+            return hipErrorOutOfMemory;
+        }
+        IoSlot s;
+        s.host = host.data();
+        s.dev = spare;
+        for (size_t t0 = 0; t0 < count && e == hipSuccess; t0 += host.size()) {
+            const size_t n = std::min(host.size(), count - t0);
+            e = move(s, t0, n);
+            const hipError_t w = hipStreamSynchronize(stream);
+            if (e == hipSuccess) e = w;
+            if (e == hipSuccess) finish(s, t0, n);
+        }
+        return e;
     }
 
   private:
-    // A free slot, one that has its memory first.
-    IoSlot& take() {
+    // A free slot, one that has its memory first; with `more` one that has
+    // none yet, otherwise null where no slot has any.
+    IoSlot* take(bool more) {
         std::unique_lock<std::mutex> lk(mu_);
         while (true) {
             IoSlot* best = nullptr;
-            for (IoSlot& s : slot_)
-                if (!s.taken && (!best || (s.done && !best->done))) best = &s;
+            bool busy = false;
+            for (IoSlot& s : slot_) {
+                busy = busy || s.taken;
+                if (!s.taken && (s.done || more) && (!best || (s.done && !best->done))) best = &s;
+            }
             if (best) {
                 best->taken = true;
-                return *best;
+                return best;
             }
+            if (!busy) return nullptr;
             freed_.wait(lk);
         }
     }
@@ -111,17 +144,28 @@ class IoPool {
             std::lock_guard<std::mutex> lk(mu_);
             s.taken = false;
         }
-        freed_.notify_one();
+        freed_.notify_all();
     }
-    hipError_t complete(IoSlot& s) {
-        hipError_t e = hipSuccess;
-        if (!s.host) e = hipHostMalloc((void**)&s.host, kIoValues * sizeof(double), 0);
-        if (e == hipSuccess && !s.dev) e = hipMalloc((void**)&s.dev, kIoValues * sizeof(double));
-        if (e == hipSuccess && !s.done) e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
-        return e;
+    // Gives a taken slot its memory, all or none of it.
+    static bool complete(IoSlot& s) {
+        if (s.done) return true;
+        const size_t bytes = kIoValues * sizeof(double);
+        if (hipHostMalloc((void**)&s.host, bytes, 0) == hipSuccess && hipMalloc((void**)&s.dev, bytes) == hipSuccess &&
+            hipEventCreateWithFlags(&s.done, hipEventDisableTiming) == hipSuccess)
+            return true;
+        strip(s);
+        (void)hipGetLastError();  // a launch check that follows must not find it
+        return false;
+    }
+    static void strip(IoSlot& s) {
+        if (s.host) (void)hipHostFree(s.host);
+        if (s.dev) (void)hipFree(s.dev);
+        if (s.done) (void)hipEventDestroy(s.done);
+        s.host = s.dev = nullptr;
+        s.done = nullptr;
     }
 
-    std::mutex mu_;
+    std::mutex mu_, spare_mu_;
     std::condition_variable freed_;
     int users_ = 0;
     IoSlot slot_[kIoSlots];

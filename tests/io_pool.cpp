@@ -14,9 +14,10 @@
 namespace {
 std::mutex mu;
 int room = 1000, held = 0, most = 0, syncs = 0;  // allocations that succeed, held, most held; stream waits
+thread_local hipError_t last_error = hipSuccess;
 hipError_t allocate(void** p, size_t bytes) {
     std::lock_guard<std::mutex> lk(mu);
-    if (held >= room) return hipErrorOutOfMemory;
+    if (held >= room) return last_error = hipErrorOutOfMemory;
     most = std::max(most, ++held);
     *p = std::malloc(bytes);
     return hipSuccess;
@@ -42,6 +43,7 @@ hipError_t hipEventDestroy(hipEvent_t e) {
     delete reinterpret_cast<char*>(e);
     return hipSuccess;
 }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t) { return e ? hipSuccess : hipErrorInvalidHandle; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) {
     std::lock_guard<std::mutex> lk(mu);
@@ -49,7 +51,11 @@ hipError_t hipStreamSynchronize(hipStream_t) {
     return hipSuccess;
 }
 hipError_t hipSetDevice(int) { return hipSuccess; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+    const hipError_t e = last_error;
+    last_error = hipSuccess;
+    return e;
+}
 }
 
 namespace {
@@ -58,13 +64,13 @@ using mfs::IoSlot;
 // A download of `count` values k -> base + k; hold() runs in every chunk.
 template <typename Hold>
 std::string download(mfs::IoPool& pool, size_t count, double base, Hold&& hold) {
-    std::vector<double> out(count, -1.0);
+    std::vector<double> out(count, -1.0), spare(777);
     const hipError_t e = pool.transfer(
-        0, nullptr, count,
+        0, nullptr, count, spare.data(), spare.size(),
         [&](IoSlot& s, size_t t0, size_t n) {
             for (size_t k = 0; k < n; ++k) s.dev[k] = base + (double)(t0 + k);
             std::memcpy(s.host, s.dev, n * sizeof(double));
-            return hipSuccess;
+            return hipGetLastError();
         },
         [&](IoSlot& s, size_t t0, size_t n) {
             hold();
@@ -120,11 +126,26 @@ std::string run(const std::string& what) {
     if (what == "failed chunk") {
         std::atomic<int> calls{0};
         const hipError_t r = pool.transfer(
-            0, nullptr, 20 * V, [&](IoSlot&, size_t, size_t) { return ++calls == 3 ? hipErrorUnknown : hipSuccess; },
+            0, nullptr, 20 * V, nullptr, 0, [&](IoSlot&, size_t, size_t) { return ++calls == 3 ? hipErrorUnknown : hipSuccess; },
             [](IoSlot&, size_t, size_t) {});
         if (r != hipErrorUnknown) e = "the error is lost";
         if (syncs == 0) e = "a slot is given back before its chunk's work has ended";
         if (e.empty()) e = download(pool, 20 * V, 3.0, nothing);  // every slot is free again
+    }
+    if (what == "no memory")  // for no slot, half of one, one, one and a half, three
+        for (int r : {0, 1, 2, 3, 6}) {
+            room = r;
+            if (e.empty()) e = download(pool, 20 * V + 5, r, nothing);
+            if (e.empty()) e = download(pool, 3, r, nothing);
+            if (e.empty() && held > r - r % 2) e = "half a slot is kept";
+        }
+    if (what == "no memory, many at once") {
+        room = 3;
+        std::vector<std::string> es(6);
+        std::vector<std::thread> th;
+        for (int k = 0; k < 6; ++k) th.emplace_back([&, k] { es[k] = download(pool, (k + 1) * V + k, k, nothing); });
+        for (auto& t : th) t.join();
+        for (auto& x : es) e += x;
     }
     pool.leave();
     if (e.empty() && held != 0) e = "memory left after the last context";

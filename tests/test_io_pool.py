@@ -21,9 +21,11 @@ def io_pool(tmp_path_factory):
     return lambda what: subprocess.run([exe, what], capture_output=True, text=True, timeout=60).stdout.strip()
 
 
-@pytest.mark.parametrize("what", ["sizes", "two contexts", "many at once", "failed chunk"])
+@pytest.mark.parametrize("what", ["sizes", "two contexts", "many at once", "failed chunk", "no memory",
+                                  "no memory, many at once"])
 def test_staging_slots(io_pool, what):
     """Transfers of no value to many chunks; a context created, downloading
     and destroyed beside another's download; more transfers than slots; a
-    chunk that fails."""
+    chunk that fails; device or pinned memory for few slots or none, where a
+    transfer has to end all the same."""
     assert io_pool(what) == "ok"
