@@ -176,11 +176,10 @@ typedef struct mfs_ctx_options {
                           * they leave idle.  Default 5 (the fastest on 6.0M cells in both precisions). */
     int sweep_tail_grid; /* pairs of waves, on one XCD, that sweep in the thin-tail launch (rounded up to
                           * workgroups of 4 waves): each sweep of the flat schedule runs its wide levels and
-                          * the run of thin levels that ends its order as two launches.  A level is thin with at most 64 chunks, counted as
-                          * 16 cells of a tile (8 on meshes with more than 4 faces per cell, where from
-                          * 16,384 cells on the limit is 128).  0: default (64); -1: one launch per
-                          * sweep.  A mesh of thin levels only runs each sweep as one launch on one XCD,
-                          * whatever this is. */
+                          * the run of thin levels that ends its order as two launches.  A level is thin
+                          * with at most 64 groups of 16 cells of a tile (128 of 8 cells on meshes with more
+                          * than 4 faces per cell).  0: default (64); -1: one launch per sweep.  A mesh of
+                          * thin levels only runs each sweep as one launch on one XCD, whatever this is. */
 } mfs_ctx_options;
 int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p, int precision, const mfs_ctx_options* opt,
                       mfs_ctx** out);
@@ -271,10 +270,10 @@ typedef struct mfs_ctx_info {
     size_t device_bytes;   /* device memory held by the context */
     int tile_cells, sweep_waves, sweep_tiles, sweep_workgroups, sweep_by_tiles;
     int compute_units;     /* CUs of the context's device (the sweep grid is sized on them) */
-    int sweep_tail_chunks; /* the thin tail's levels in groups of 16 cells of a tile (8 on meshes with more than 4
-                            * faces per cell; 0: one launch per sweep) */
-    int sweep_tail_cells;  /* their cells */
-    int sweep_tail_workgroups; /* sweep_tail_grid, at most the resident grid and one per sweep_waves groups */
+    /* the levels of at most 64 groups that end the sweep order (0: a launch for them is off, or they are few or
+     * all): groups of 16 cells of a tile (8 on meshes with more than 4 faces per cell), cells, and sweep_tail_grid
+     * at most the resident grid and one per sweep_waves groups.  The launches: mfs_ctx_get_launches */
+    int sweep_tail_chunks, sweep_tail_cells, sweep_tail_workgroups;
 } mfs_ctx_info;
 int mfs_ctx_get_info(mfs_ctx* ctx, mfs_ctx_info* info);
 /* What the context's steps launch (no counterpart in the reference).  [0] is

@@ -127,7 +127,7 @@ struct mfs_ctx {
     bool all_thin = false;  // every level is thin
     int thin_levels = 0;    // levels of the thin tail, or all
     int tail_chunks = 0;  // its width in groups of 64/lpc cells per tile
-    int tail_cells = 0;
+    int narrow_chunks = 0, narrow_cells = 0;  // what mfs_ctx_info reports of it
     int compute_units = 0;  // CUs of the device
     // reductions and history
     double* part = nullptr;  // 8 * nblk, value-major: 5 squared-norm partials, dt min, dt max, spare

@@ -707,9 +707,7 @@ bool launch_diag(mfs_ctx* ctx, bool clamp_only) {
 }
 
 // Whether the sweeps run as two launches each (wide levels, thin tail).
-bool sweep_split(const mfs_ctx* ctx) {
-    return !ctx->sweep_by_tiles && ctx->tail_grid > 0 && ctx->tail_chunks > 0;
-}
+bool sweep_split(const mfs_ctx* ctx) { return ctx->tail_grid > 0 && ctx->tail_chunks > 0; }
 
 // Whether the sweeps run whole on one XCD: a mesh of thin levels only.
 bool sweep_local(const mfs_ctx* ctx) { return !ctx->sweep_by_tiles && !sweep_split(ctx) && ctx->all_thin; }
@@ -724,9 +722,9 @@ int sweep_workgroups(const mfs_ctx* ctx) {
     return std::max(1, std::min(ctx->sweep_grid, units));
 }
 
-// The tail grid of a split sweep, in groups of kThinWaves waves.
-int tail_workgroups(const mfs_ctx* ctx) {
-    const int units = (ctx->tail_chunks + ctx->sweep_waves - 1) / ctx->sweep_waves;
+// The tail grid of a tail of `chunks` groups, in groups of kThinWaves waves.
+int tail_workgroups(const mfs_ctx* ctx, int chunks) {
+    const int units = (chunks + ctx->sweep_waves - 1) / ctx->sweep_waves;
     return std::max(1, std::min({ctx->tail_grid, ctx->sweep_grid, units}));
 }
 
@@ -735,7 +733,8 @@ int tail_workgroups(const mfs_ctx* ctx) {
 // such a launch whole.
 int thin_workgroups(const mfs_ctx* ctx) {
     constexpr int W = kBlock / 64;
-    const int g = sweep_split(ctx) ? tail_workgroups(ctx) : std::min(sweep_workgroups(ctx), dev::kDefaultTailGrid);
+    const int g = sweep_split(ctx) ? tail_workgroups(ctx, ctx->tail_chunks)
+                                    : std::min(sweep_workgroups(ctx), dev::kDefaultTailGrid);
     return (g * dev::kThinWaves + W - 1) / W;
 }
 
@@ -1206,8 +1205,9 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     ctx->all_thin = L.all_thin;
     ctx->thin_levels = L.thin_levels;
     ctx->tail_chunks = L.tail_chunks;
-    ctx->tail_cells = L.tail_cells;
-    ctx->tail_grid = (tail_grid > 0 && !sweep_by_tiles && ctx->tail_chunks > 0) ? tail_grid : 0;
+    ctx->narrow_chunks = L.narrow_chunks;
+    ctx->narrow_cells = L.narrow_cells;
+    ctx->tail_grid = tail_grid > 0 && !sweep_by_tiles ? tail_grid : 0;
     ctx->ntiles = (int)L.sweep[0].tile_chunk.size() - 1;
     ctx->lpc = L.lpc;
     ctx->nblk_cell = (int)nblk_xcd(L.nC);
@@ -1889,9 +1889,10 @@ extern "C" int mfs_ctx_get_info(mfs_ctx* ctx, mfs_ctx_info* info) {
     info->sweep_workgroups = sweep_workgroups(ctx);
     info->sweep_by_tiles = ctx->sweep_by_tiles;
     info->compute_units = ctx->compute_units;
-    info->sweep_tail_chunks = ctx->tail_grid > 0 ? ctx->tail_chunks : 0;
-    info->sweep_tail_cells = ctx->tail_grid > 0 ? ctx->tail_cells : 0;
-    info->sweep_tail_workgroups = ctx->tail_grid > 0 ? tail_workgroups(ctx) : 0;
+    const bool tail = ctx->tail_grid > 0 && ctx->narrow_chunks > 0;
+    info->sweep_tail_chunks = tail ? ctx->narrow_chunks : 0;
+    info->sweep_tail_cells = tail ? ctx->narrow_cells : 0;
+    info->sweep_tail_workgroups = tail ? tail_workgroups(ctx, ctx->narrow_chunks) : 0;
     return MFS_OK;
 }
 

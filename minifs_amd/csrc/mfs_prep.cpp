@@ -490,20 +490,29 @@ std::string build_layout(const mfs_mesh_view& v, HostLayout& L, int kTileCells) 
         const int ng = (int)glevel.size();
         std::vector<int> width(L.nlev, 0);
         for (int g = 0; g < ng; ++g) width[glevel[g]] += (gfirst[g + 1] - gfirst[g] + unit - 1) / unit;
+        // The run of levels of at most `line` groups that ends the order: its
+        // first level (nlev without one, or where it is shorter than
+        // kMinTailChunks or the whole order), groups and cells.
+        auto tail_of = [&](int line, int& levels, int& groups, int& cells) {
+            int first = L.nlev;
+            groups = cells = 0;
+            while (first > 0 && width[first - 1] <= line) groups += width[--first];
+            levels = L.nlev - first;
+            if (first == 0 || groups < kMinTailChunks) {
+                first = L.nlev;
+                groups = 0;
+            }
+            for (int g = 0; g < ng; ++g)
+                if (glevel[g] >= first) cells += gfirst[g + 1] - gfirst[g];
+            return first;
+        };
+        const int line = L.lpc == 8 ? kWideThinLevelChunks : kThinLevelChunks;
+        const int tail_level = tail_of(line, L.thin_levels, L.tail_chunks, L.tail_cells);
+        L.all_thin = L.thin_levels == L.nlev;
+        int levels = 0;
+        tail_of(kThinLevelChunks, levels, L.narrow_chunks, L.narrow_cells);
         std::vector<char> thin(L.nlev);
-        const int most_groups = L.lpc == 8 && nC >= kWideThinMeshCells ? kWideThinLevelChunks : kThinLevelChunks;
-        for (int l = 0; l < L.nlev; ++l) thin[l] = width[l] <= most_groups;
-        int tail_level = L.nlev;  // first level of the thin tail
-        while (tail_level > 0 && thin[tail_level - 1]) L.tail_chunks += width[--tail_level];
-        L.all_thin = tail_level == 0;
-        L.thin_levels = L.nlev - tail_level;
-        if (tail_level == 0 || L.tail_chunks < kMinTailChunks) {
-            tail_level = L.nlev;
-            L.tail_chunks = 0;
-        }
-        L.tail_cells = 0;
-        for (int g = 0; g < ng; ++g)
-            if (glevel[g] >= tail_level) L.tail_cells += gfirst[g + 1] - gfirst[g];
+        for (int l = 0; l < L.nlev; ++l) thin[l] = width[l] <= line;
         L.cdep.resize(2 * (size_t)nC);
         std::vector<int> gchunk(ng + 1);
         for (int dir = 0; dir < 2; ++dir) {

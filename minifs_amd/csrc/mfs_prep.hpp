@@ -123,6 +123,7 @@ struct HostLayout {
     // counted in the level-width unit below, and its cells
     int tail_chunks = 0, tail_cells = 0, thin_levels = 0;  // thin_levels: also where every level is thin
     bool all_thin = false;              // every level is thin
+    int narrow_chunks = 0, narrow_cells = 0;  // the same tail with levels of at most kThinLevelChunks groups
     bool tri_slots = false;                    // tetrahedra with triangular slots only
     // initial state, 5 blocks of nC+nB, device cell order
     lvec<double> q;
@@ -131,8 +132,8 @@ struct HostLayout {
 // Cells per storage tile of the device order (the sweeps' workgroup unit).
 constexpr int kDefaultTileCells = 4096;
 // Thin levels.  A level's width is counted in groups of 64/lpc cells per
-// tile; levels of at most kThinLevelChunks groups are thin (on larger meshes of
-// 8 slots per cell kWideThinLevelChunks, below).  A thin chunk
+// tile; levels of at most kThinLevelChunks groups are thin (on meshes of 8
+// slots per cell kWideThinLevelChunks, below).  A thin chunk
 // holds at most kThinCells cells, so that each of its 5-value results has a
 // lane of its own.
 constexpr int kThinLevelChunks = 64;
@@ -140,14 +141,15 @@ constexpr int kThinCells = 12;
 // With 8 slots per cell a group has 8 cells, half of a tetrahedral mesh's, so
 // the same 1,024 cells of a level are 128 groups: 86 thin chunks, one for
 // each of the 128 waves that sweep the tail.  ms per iteration with 64 and
-// with 128 groups: 262k hexahedra FP64 0.593 -> 0.583, 64k 0.321 -> 0.308,
-// 33k 0.260 -> 0.248; 195k prisms mixed 0.432 -> 0.418, 35k FP64 0.249 ->
-// 0.240; 1M hexahedra FP64 1.206 -> 1.179, on a shallow order 0.938 -> 0.910.
-// Batches, whose waits do not use the line, change by less than 1% (8 solves
-// of hexahedra 0.924 -> 0.921, of prisms 1.205 -> 1.212).  (Tetrahedra gained nothing from 128: 20k, 94k and 384k cells all
-// within 0.2%.)  Smaller meshes gain too (8k hexahedra 0.163 -> 0.142), but
-// the tail that mfs_ctx_info reports for them is pinned, so they keep 64.
-constexpr int kWideThinLevelChunks = 128, kWideThinMeshCells = 16384;
+// with 128 groups, FP64: 8k hexahedra 0.163 -> 0.142 (every level is thin
+// then), 10.6k 0.183 -> 0.159, 16k 0.200 -> 0.196, 33k 0.260 -> 0.248, 262k
+// 0.593 -> 0.583, 1M 1.206 -> 1.179; prisms 8.2k on a shallow order 0.148 ->
+// 0.128, 11k 0.174 -> 0.150, 16k 0.195 -> 0.191; mixed 195k 0.432 -> 0.418.
+// Smaller meshes have only thin levels with either.  Batches, whose waits do
+// not use the line, change by less than 1% (8 solves of hexahedra 0.924 ->
+// 0.921, of prisms 1.205 -> 1.212).  Tetrahedra gained nothing from 128: 20k,
+// 94k and 384k cells all within 0.2%.
+constexpr int kWideThinLevelChunks = 128;
 // On levels of at most this many groups a wave waits on a dependency one
 // level further back and then polls its own at once (SweepLayout::crec); on
 // wider ones it waits on its latest dependency with one load, since there the

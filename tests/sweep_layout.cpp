@@ -66,7 +66,8 @@ std::string check(const mfs::HostLayout& L, int dir, int tile_cells) {
     for (int u = 0; u < S.nchunk; ++u) {
         const int d0 = S.crec[4 * u], cells = S.crec[4 * u + 1] & 0xff, nk = (S.crec[4 * u + 1] >> 8) & 0xff;
         NEED(cells >= 1 && cells <= 64 && nk <= 64 && d0 >= 0 && d0 + cells <= nC);
-        NEED(!(S.crec[4 * u + 1] & mfs::kThinChunkFlag) || cells <= mfs::kThinCells);
+        const bool thin = width[level(d0)] <= (L.lpc == 8 ? mfs::kWideThinLevelChunks : mfs::kThinLevelChunks);
+        NEED(thin == ((S.crec[4 * u + 1] & mfs::kThinChunkFlag) != 0) && (!thin || cells <= mfs::kThinCells));
         NEED((size_t)S.crec[4 * u + 2] == nd);
         NEED(dir == 0 ? level(d0) >= before : level(d0) <= before);
         before = level(d0);

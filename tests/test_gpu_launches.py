@@ -172,3 +172,26 @@ def test_second_stream_gradient_beside_a_split_sweep(cells, dims, tree, precisio
     a.close()
     b.close()
     g.close()
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("cells,dims,tree,thin", [("hex", (17, 16, 18), (2, 16), 2), ("hex", (20, 20, 20), (4, 512), 2),
+                                                  ("hex", (22, 21, 23), (2, 16), 1), ("prism", (16, 16, 16), (2, 128), 2),
+                                                  ("prism", (18, 17, 18), (2, 16), 1)])
+def test_thin_levels_of_small_six_face_meshes(cells, dims, tree, thin, precision):
+    """Levels of up to 128 groups of 8 cells are thin on meshes of every size:
+    those of a few thousand cells, some of whose sweeps run whole on one XCD,
+    give the tile schedule's bits."""
+    print(f"[launches] small six-face mesh {cells} {dims} {tree} precision={precision}", flush=True)
+    p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0)
+    g = mfs.Grid.box_bump(*dims, cells=cells).decouple(*tree).preprocess(p)
+    a, b = mfs.Solver(g, p, precision=precision), mfs.Solver(g, p, precision=precision, sweep_by_tiles=1)
+    assert a.launches()["thin_launch"] == thin
+    for s in (a, b):
+        s.step(4)
+        s.iterate_reference_order(1)
+    for nm in FIELDS:
+        np.testing.assert_array_equal(a.field(nm), b.field(nm), err_msg=nm)
+    a.close()
+    b.close()
+    g.close()
