@@ -71,15 +71,21 @@ __global__ __launch_bounds__(kReduceBlock) void k_b_reduce(const BatchSolve<R>* 
     reduce_body(S.nblk_cell, S.part, S.run, S.hist, S.hist_slot, 1 | 2 | 4, S.ratio_dtmax);
 }
 
-// The ratio_dtmax clamp, kBatchClampBlocks workgroups per solve that return
-// at once where it is off, the rule at the reference's ratio_dtmax (a
-// workgroup per 256 cells took 8.4 us of a 12-solve iteration, these 4.4).
-constexpr int kBatchClampBlocks = 64;
+// The ratio_dtmax clamp, `per` workgroups per solve that return at once where
+// it is off, the rule at the reference's ratio_dtmax: 64, or more where the
+// solves are few and large and 64 would leave CUs idle with the clamp on, up to
+// kBatchClampTotal in all and one per 1,024 cells.  ms per FP64 iteration with
+// the clamp on | off: one solve of 6.0M cells, with 64 4.19 | 3.54, with 1,024
+// 3.78 | 3.54 (with 8,192 3.76 | 3.54); two of 1.3M 1.862 | 1.700 and, with
+// 512 each, 1.800 | 1.704; twelve of 48k, 64 each, 0.528 | 0.512.  A workgroup
+// per 256 cells took 8.4 us with the clamp off in a 12-solve iteration of 2.3M
+// cells, 64 a solve 4.4.
+constexpr int kBatchClampBlocks = 64, kBatchClampTotal = 1024, kBatchClampTurns = 4;
 template <int MAXF, typename R>
-__global__ __launch_bounds__(kBlock) void k_b_clamp(const BatchSolve<R>* __restrict__ T) {
-    const BatchSolve<R>& S = T[blockIdx.x / kBatchClampBlocks];
+__global__ __launch_bounds__(kBlock) void k_b_clamp(const BatchSolve<R>* __restrict__ T, int per) {
+    const BatchSolve<R>& S = T[(int)blockIdx.x / per];
     if (S.run[2] == 0.0) return;
-    for (int c = (int)(blockIdx.x % kBatchClampBlocks * kBlock + threadIdx.x); c < S.nC; c += kBatchClampBlocks * kBlock)
+    for (int c = (int)blockIdx.x % per * kBlock + (int)threadIdx.x; c < S.nC; c += per * kBlock)
         diag_body<MAXF == 4 ? 4 : 8>(c, S.nC, S.sgeo64, S.sflip, S.q, S.vol, S.dt, S.diag, S.run, S.ratio_dtmax, S.K,
                                      S.q32 ? S.diag32 : nullptr);
 }

@@ -2199,6 +2199,10 @@ int batch_step_t(mfs_batch* b, int nsteps) {
     const int most = std::max(b->nitems[0], b->nitems[1]);
     const dim3 sweep_grid((unsigned)std::max(1, std::min(b->sweep_grid, (most + kBatchSweepWaves - 1) /
                                                                          kBatchSweepWaves)));
+    int largest = 0;  // cell blocks of the largest solve
+    for (int a : b->active) largest = std::max(largest, b->slots[a]->nblk_cell);
+    const int clamp_blocks = std::max(std::min(dev::kBatchClampBlocks, largest),
+                                      std::min(dev::kBatchClampTotal / ns, largest / dev::kBatchClampTurns));
     // The gradient feeds nothing in an iteration, so with a second stream it
     // runs beside the next iteration (see step_iterations).
     const int mode = b->gstream ? b->gradient_stream : 1;
@@ -2224,8 +2228,8 @@ int batch_step_t(mfs_batch* b, int nsteps) {
             hipLaunchKernelGGL((dev::k_b_flux_ts<MAXF, MIXED, R>), dim3(b->ncell_blk), dim3(kBlock), 0, b->stream,
                                Tf, b->cell_solve);
         hipLaunchKernelGGL((dev::k_b_reduce<R>), dim3(ns), dim3(dev::kReduceBlock), 0, b->stream, Tf);
-        hipLaunchKernelGGL((dev::k_b_clamp<MAXF, R>), dim3(ns * dev::kBatchClampBlocks), dim3(kBlock), 0, b->stream,
-                           Tf);
+        hipLaunchKernelGGL((dev::k_b_clamp<MAXF, R>), dim3(ns * clamp_blocks), dim3(kBlock), 0, b->stream, Tf,
+                           clamp_blocks);
         if (!batch_ok(b, hipGetLastError(), "batch flux/time step")) return MFS_ERR_HIP;
         const int par = (int)(b->iters & 1);
         if (side && b->gpend[par]) {

@@ -195,3 +195,28 @@ def test_thin_levels_of_small_six_face_meshes(cells, dims, tree, thin, precision
     a.close()
     b.close()
     g.close()
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("cells,sizes", [("tet", (3,)), ("tet", (36,)), ("tet", (24, 30)), ("hex", (65,)),
+                                         ("tet", (10, 3, 12, 8, 5, 9, 2, 11, 4, 6, 7, 3, 5, 4, 2, 8, 9))])
+def test_clamp_of_few_and_many_solves(cells, sizes, precision):
+    """The ratio_dtmax clamp on in every solve: one small solve (fewer blocks
+    than the least), one and two of more blocks than their share, more solves
+    than get more than the least.  Each equals the solve alone."""
+    print(f"[launches] clamp {cells} {sizes} precision={precision}", flush=True)
+    p = mfs.make_params(mach=0.8, alpha=1.25, cfl=10.0, ratio_dtmax=1.2)
+    grids = [mfs.Grid.box_bump(n, seed=k + 1, cells=cells).decouple().preprocess(p) for k, n in enumerate(sizes)]
+    b = mfs.Batch(precision)
+    members = [b.add(g, p) for g in grids]
+    b.step(3)
+    for m, g in zip(members, grids):
+        s = mfs.Solver(g, p, precision=precision)
+        s.step(3)
+        for nm in FIELDS:
+            np.testing.assert_array_equal(m.field(nm), s.field(nm), err_msg=nm)
+        np.testing.assert_array_equal(m.history(), s.history())
+        s.close()
+    b.close()
+    for g in grids:
+        g.close()
