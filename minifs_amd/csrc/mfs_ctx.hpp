@@ -60,7 +60,6 @@ struct mfs_ctx {
     // faces (device order)
     int2* fcell = nullptr;
     double4* fgeo = nullptr;
-    double2* fdn = nullptr;
     int *fno = nullptr, *fn = nullptr, *btype = nullptr;
     // cells
     int *cfo = nullptr, *cf = nullptr;
@@ -96,7 +95,6 @@ struct mfs_ctx {
     float4* sgeo32 = nullptr;   // the same in FP32 (mixed precision)
     int sweep_by_tiles = 0;
     int ntiles = 0;
-    int* depmask = nullptr;
     int* tickets = nullptr;  // ticket counters of the flat sweep schedule: forward, then backward
     int* gface = nullptr;    // nB: device face of each ghost cell nC+k
     int4* cnode = nullptr;   // tetrahedral meshes: the cells' nodes and the gradient's choices (k_tet_tables)

@@ -755,7 +755,6 @@ void sweep_args(dev::SweepArgs<R>& A, const mfs_ctx* ctx, int cur) {
     A.ntiles = ctx->ntiles;
     for (int d = 0; d < 2; ++d) {
         const mfs_ctx::Sweep& S = ctx->sweep[d];
-        A.dir[d].nchunks = S.nchunk;
         A.dir[d].crec = S.crec;
         A.dir[d].batch_wait = S.batch_wait;
         A.dir[d].dnb = S.dnb;
@@ -1227,7 +1226,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
     ok = ok && dalloc(ctx, ctx->gx, 5 * n, "dqdx") && dalloc(ctx, ctx->gy, 5 * n, "dqdy") &&
          dalloc(ctx, ctx->gz, 5 * n, "dqdz") && dalloc(ctx, ctx->qn, 5 * (size_t)L.nN, "qnode");
     ok = ok && dalloc(ctx, ctx->fcell, L.nF, "fcell") && dalloc(ctx, ctx->fgeo, L.nF, "fgeo") &&
-         dalloc(ctx, ctx->fdn, L.nF, "fdn") && dalloc(ctx, ctx->fno, L.nF + 1, "fno") &&
+         dalloc(ctx, ctx->fno, L.nF + 1, "fno") &&
          dalloc(ctx, ctx->fn, L.fn.size(), "fn") && dalloc(ctx, ctx->btype, L.nB, "btype");
     if (ctx->maxf == 4) {
         // four faces per cell means tetrahedra: the gradient kernel reads
@@ -1281,7 +1280,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
          dalloc(ctx, ctx->dev_of_node, (size_t)L.nN, "node map");
     ok = ok && dalloc(ctx, ctx->cdep, L.cdep.size(), "cell dependencies") &&
          dalloc(ctx, ctx->snb, L.cfs.size(), "slot neighbours") &&
-         dalloc(ctx, ctx->sgeo, nslot, "slot geometry") && dalloc(ctx, ctx->depmask, L.nC, "depmask");
+         dalloc(ctx, ctx->sgeo, nslot, "slot geometry");
     if (mixed) {
         ok = ok && dalloc(ctx, ctx->q32, 5 * n, "q32") && dalloc(ctx, ctx->diag32, L.nC, "diag32") &&
              dalloc(ctx, ctx->dqf32, 5 * (size_t)L.nC, "dq_forward32") && dalloc(ctx, ctx->dq32, 5 * n, "dq32") &&
@@ -1333,7 +1332,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
         ok = upload(ctx, ctx->q[0], qa.data(), 5 * n, "upload q") && upload(ctx, ctx->q[1], qa.data(), 5 * n, "upload q") &&
              upload(ctx, ctx->fcell, fc.data(), L.nF, "upload fcell") &&
              upload(ctx, ctx->fgeo, reinterpret_cast<const double4*>(L.fgeo.data()), L.nF, "upload fgeo") &&
-             upload(ctx, ctx->fdn, fd.data(), L.nF, "upload fdn") && upload(ctx, ctx->fno, L.fno.data(), L.nF + 1, "upload fno") &&
+             upload(ctx, ctx->fno, L.fno.data(), L.nF + 1, "upload fno") &&
              upload(ctx, ctx->fn, L.fn.data(), L.fn.size(), "upload fn") &&
              upload(ctx, ctx->btype, L.btype.data(), L.nB, "upload btype") &&
              upload(ctx, ctx->cfo, L.cfo.data(), L.nC + 1, "upload cfo") && upload(ctx, ctx->cf, L.cf.data(), L.cf.size(), "upload cf") &&
@@ -1344,7 +1343,6 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
              upload(ctx, ctx->nden, L.nden.data(), L.nN, "upload nden") &&
              upload(ctx, ctx->sym_node, L.sym_node.data(), L.sym_node.size(), "upload sym") &&
              upload(ctx, ctx->sym_n, L.sym_n.data(), L.sym_n.size(), "upload sym_n") &&
-             upload(ctx, ctx->depmask, L.depmask.data(), L.nC, "upload depmask") &&
              upload(ctx, ctx->gface, gf.data(), (size_t)L.nB, "upload gface") &&
              upload(ctx, ctx->dev_of_cell, L.dev_of_cell.data(), (size_t)L.nC, "upload cell map") &&
              upload(ctx, ctx->dev_of_node, L.dev_of_node.data(), (size_t)L.nN, "upload node map") &&
@@ -1358,23 +1356,30 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                  upload(ctx, S.pos, H.pos.data(), H.pos.size(), "upload pos") &&
                  upload(ctx, S.tile_chunk, H.tile_chunk.data(), H.tile_chunk.size(), "upload tile_chunk");
         }
-        // the slot tables, built on the device from the slot face ids
-        int* dcfs = nullptr;
-        ok = ok && hip_ok(ctx, hipMalloc((void**)&dcfs, L.cfs.size() * sizeof(int)), "hipMalloc(slot faces)");
+        // the slot tables, built on the device from what only they are built
+        // of: the faces' distances, the slot face ids and the dependency masks
+        char* temp = nullptr;
+        const size_t at_cfs = (size_t)L.nF * sizeof(double2), at_mask = at_cfs + L.cfs.size() * sizeof(int);
+        ok = ok && hip_ok(ctx, hipMalloc((void**)&temp, at_mask + (size_t)L.nC * sizeof(int)), "hipMalloc(slot faces)");
         if (ok) {
-            ok = upload(ctx, dcfs, L.cfs.data(), L.cfs.size(), "upload slot faces");
+            auto* const fdn = reinterpret_cast<double2*>(temp);
+            int* const dcfs = reinterpret_cast<int*>(temp + at_cfs);
+            int* const depmask = reinterpret_cast<int*>(temp + at_mask);
+            ok = upload(ctx, fdn, fd.data(), L.nF, "upload face distances") &&
+                 upload(ctx, dcfs, L.cfs.data(), L.cfs.size(), "upload slot faces") &&
+                 upload(ctx, depmask, L.depmask.data(), L.nC, "upload dependency masks");
             if (ok) {
                 const unsigned gC = (unsigned)((L.nC + kBlock - 1) / kBlock);
                 auto kern = L.lpc == 4 ? dev::k_slot_tables<4> : dev::k_slot_tables<8>;
                 hipLaunchKernelGGL(kern, dim3(gC), dim3(kBlock), 0, ctx->stream, L.nC, dcfs, ctx->cfo, ctx->fcell,
-                                   ctx->fgeo, ctx->fdn, ctx->snb, ctx->sgeo, mixed ? ctx->sgeo32 : nullptr, ctx->sdn,
+                                   ctx->fgeo, fdn, ctx->snb, ctx->sgeo, mixed ? ctx->sgeo32 : nullptr, ctx->sdn,
                                    ctx->sflip);
                 ok = check_launch(ctx, "k_slot_tables");
                 auto dep = L.lpc == 4 ? dev::k_dep_tables<4> : dev::k_dep_tables<8>;
                 for (int d = 0; d < 2 && ok; ++d) {
                     const mfs_ctx::Sweep& S = ctx->sweep[d];
                     hipLaunchKernelGGL(dep, dim3(nblk((size_t)S.nchunk, kBlock / 64)), dim3(kBlock), 0, ctx->stream,
-                                       L.nC, S.nchunk, S.crec, ctx->cdep, d, ctx->depmask, ctx->snb, ctx->sgeo, S.dnb,
+                                       L.nC, S.nchunk, S.crec, ctx->cdep, d, depmask, ctx->snb, ctx->sgeo, S.dnb,
                                        S.dgeo, S.dgeo32);
                     ok = check_launch(ctx, "k_dep_tables");
                 }
@@ -1382,7 +1387,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                 if (ok && ctx->cnode) {
                     ok = hip_ok(ctx, hipMemsetAsync(ctx->err, 0, sizeof(int) * 4, ctx->stream), "memset err");
                     hipLaunchKernelGGL(dev::k_tet_tables, dim3(gC), dim3(kBlock), 0, ctx->stream, L.nC, dcfs, ctx->fn,
-                                       ctx->depmask, ctx->cnode, ctx->gsel, ctx->err + 3);
+                                       depmask, ctx->cnode, ctx->gsel, ctx->err + 3);
                     ok = ok && check_launch(ctx, "k_tet_tables") &&
                          hip_ok(ctx, hipMemcpyAsync(&bad, ctx->err + 3, sizeof(int), hipMemcpyDeviceToHost, ctx->stream),
                                 "tetrahedra check");
@@ -1390,7 +1395,7 @@ extern "C" int mfs_ctx_create_ex(const mfs_mesh_view* mesh, const mfs_params* p,
                 ok = ok && hip_ok(ctx, hipStreamSynchronize(ctx->stream), "slot tables");
                 if (bad) ctx->cnode = nullptr;  // its memory stays with the context
             }
-            (void)hipFree(dcfs);
+            (void)hipFree(temp);
         }
         const double run0[8] = {0.0, kBIGd, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
         ok = ok && upload(ctx, ctx->run, run0, 8, "upload run");

@@ -166,7 +166,6 @@ __device__ __forceinline__ bool wait_failed(int* err, unsigned spins) {
 // One direction's schedule and tables (SweepLayout in mfs_prep.hpp).
 template <typename R>
 struct SweepDir {
-    int nchunks;
     const int4* crec;                       // per position: first cell, cells | deps << 8 | flag, first dep, wait
     const int* batch_wait;                  // per position: the dependency a batch waits on
     const int* dnb;                         // per dependency: the neighbour

@@ -220,3 +220,19 @@ def test_clamp_of_few_and_many_solves(cells, sizes, precision):
     b.close()
     for g in grids:
         g.close()
+
+
+@pytest.mark.parametrize("cells,precision,per_cell", [("tet", mfs.MFS_FP64, 940), ("tet", mfs.MFS_MIXED, 1122),
+                                                      ("hex", mfs.MFS_FP64, 1300)])
+def test_device_memory_of_a_context(cells, precision, per_cell):
+    """A context holds what its steps read: bytes per cell, with room of 2%,
+    without the arrays that only its creation reads (36 bytes per tetrahedron,
+    52 per hexahedron)."""
+    n = 40 if cells == "tet" else 64
+    g, p = _grid(cells, (n, n, n), (4, 512))
+    s = mfs.Solver(g, p, precision=precision)
+    held = s.info()["device_bytes"] / g.info["nTCell"]
+    print(f"[launches] {held:.1f} bytes per {cells} cell", flush=True)
+    assert held < per_cell
+    s.close()
+    g.close()
