@@ -105,13 +105,6 @@ MFS_HD void roe_flux(const R ql[5], const R qr[5], R ht_l, R ht_r, R hl, R hr, R
     f[4] *= tmp0;
 }
 
-template <typename R>
-MFS_HD void roe_flux(const R ql[5], const R qr[5], R ax, R ay, R az, R area, R gamm1, R p_bar, R alf_l, R tiny,
-                     R f[5]) {
-    const R ht_l = total_enthalpy(ql, gamm1, p_bar), ht_r = total_enthalpy(qr, gamm1, p_bar);
-    roe_flux(ql, qr, ht_l, ht_r, ht_l / ql[0], ht_r / qr[0], ax, ay, az, area, gamm1, alf_l, tiny, f);
-}
-
 // FluxLUSGS3D (src/Kernels/forward_lusgs.cpp:1271-1324): neighbour state q,
 // neighbour increment DQ, normal n pointing from the swept cell to the
 // neighbour.
