@@ -163,13 +163,6 @@ MFS_HD void flux_lusgs_post(const FluxPre<R>& P, const R DQ[5], R nx, R ny, R nz
     for (int i = 0; i < 5; i++) flux[i] -= P.eig * DQ[i];
 }
 
-template <typename R>
-MFS_HD void flux_lusgs(const R q[5], const R DQ[5], R nx, R ny, R nz, R gam, R p_bar, R lhs_omga, R flux[5]) {
-    FluxPre<R> P;
-    flux_lusgs_pre(P, q, nx, ny, nz, gam, p_bar, lhs_omga);
-    flux_lusgs_post(P, DQ, nx, ny, nz, flux);
-}
-
 // FluxLUSGS3D in increment form, for the FP32 operator of mixed precision.
 // The reference's expression forms F(Q+DQ) and F(Q) separately and
 // subtracts them; in FP32 the energy terms ((Q4+p+peff)*v_n, peff =
@@ -219,13 +212,6 @@ MFS_HD void flux_lusgs_delta_post(const FluxDeltaPre<R>& P, const R DQ[5], R nx,
     flux[3] = P.Q3 * dvn + DQ[3] * vn1 + dp * nz;
     flux[4] = P.H * dvn + (DQ[4] + dp) * vn1;
     for (int i = 0; i < 5; i++) flux[i] -= P.eig * DQ[i];
-}
-
-template <typename R>
-MFS_HD void flux_lusgs_delta(const R q[5], const R DQ[5], R nx, R ny, R nz, R gam, R p_bar, R lhs_omga, R flux[5]) {
-    FluxDeltaPre<R> P;
-    flux_lusgs_delta_pre(P, q, nx, ny, nz, gam, p_bar, lhs_omga);
-    flux_lusgs_delta_post(P, DQ, nx, ny, nz, flux);
 }
 
 // The DQ positivity limiter (DQ_limit == 2) of both sweeps
