@@ -11,7 +11,8 @@ The mesh and state are resident in HBM before the timed region.
 Prints one JSON line.  `roofline` describes the kernel with the largest
 share of the timed region, timed with HIP events on the solver stream (the
 timed region brackets the two sweeps only; `kernel_ms_per_step` times every
-kernel group over further iterations);
+kernel group over further iterations, whose schedule is another: each group in
+launches of its own, the gradient on a second stream);
 `cpu_baseline` times the reference's own OpenMP build (oracle/_ref) on all
 host threads for a few iterations of the same mesh and flow, with its
 serial build beside it; `mixed` repeats the
@@ -68,7 +69,9 @@ KERNEL_BYTES = {
     # Green-Gauss: face nodes + geometry, q, node values, vol, 15 gradient outputs
     "gradient": (52, 128, 80, 40),
 }
-# kernels that mfs_step runs on the context's second stream by default
+# kernels that mfs_step runs inside the thin tails' launches by default, and on
+# the context's second stream where those cannot hide them or every kernel
+# group is timed
 SIDE_KERNELS = ("node", "gradient")
 # a sweep run as two launches (wide levels, thin tail) is timed as a whole
 # and per launch; each launch's algorithmic bytes are its cells' share of
@@ -76,6 +79,12 @@ SIDE_KERNELS = ("node", "gradient")
 SWEEP_LAUNCHES = {"fwd_sweep": ("fwd_sweep_wide", "fwd_sweep_tail"), "bwd_sweep": ("bwd_sweep_tail", "bwd_sweep_wide")}
 # iterations after the timed region with every kernel group timed
 KERNEL_TABLE_STEPS = 10
+KERNEL_TABLE = (f"HIP events around every kernel group, {KERNEL_TABLE_STEPS} iterations after the timed region (whose "
+                "events bracket the sweeps only).  Another schedule than the timed region's: the gradient runs on the "
+                "second stream beside the tails, the reduction in a launch of its own; `sweeps` has the timed "
+                "region's launches")
+TAIL_NOTE = ("the tails' launches also hold the iteration before's node values (forward) and gradient (backward): "
+             "their times, and so the sweeps' spans, include that work, their bytes are the sweep's alone")
 # whole iteration, plain FP64 (268 nF + 840 nC + 356 nB + 92 nN)
 ITER_BYTES = (268, 840, 356, 92)
 
@@ -204,6 +213,7 @@ def timed_steps(s, steps: int, warmup: int, kernel_timing: int):
 
 def mode_fp64(args, cpu_dir: str | None = None) -> dict:
     import minifs_amd as mfs
+    from minifs_amd._lib import MFS_GRADIENT_INSIDE
 
     t0 = time.time()
     p = mfs.make_params(mach=args.mach, alpha=args.alpha, cfl=args.cfl)
@@ -224,6 +234,7 @@ def mode_fp64(args, cpu_dir: str | None = None) -> dict:
     value = nC * args.steps / elapsed / 1e6
     hist = s.history()
     info_ctx = s.info()
+    inside = s.launches()["gradient"] == MFS_GRADIENT_INSIDE
     tail_cells = info_ctx["sweep_tail_cells"]
 
     def launch_bytes(k):
@@ -261,6 +272,8 @@ def mode_fp64(args, cpu_dir: str | None = None) -> dict:
                     pm = kern[part][0] / kern[part][1]
                     sweeps[k][part + "_ms"] = round(pm, 4)
                     sweeps[k][part + "_achieved_GBs"] = round(launch_bytes(part) / (pm / 1e3) / 1e9, 2)
+        if inside:
+            sweeps["note"] = TAIL_NOTE
         traffic = None
         tf = os.path.join(ROOT, "profiles", f"traffic_{dom}.json")
         if os.path.exists(tf):
@@ -347,8 +360,7 @@ def mode_fp64(args, cpu_dir: str | None = None) -> dict:
                                "frac": round(iter_b / (ms_per_step / 1e3) / 1e9 / HBM_PEAK_GBS, 5)},
         "sweeps": sweeps,
         "kernel_ms_per_step": {k: round(v[0] / v[1], 4) for k, v in kern_all.items()},
-        "kernel_table": f"HIP events around every kernel group, {KERNEL_TABLE_STEPS} iterations after the timed "
-                        "region (whose events bracket the sweeps only)",
+        "kernel_table": KERNEL_TABLE,
         "gradient_on_solver_stream": isolated,
         "mixed": mixed,
         "shallow_order": shallow,
