@@ -82,6 +82,19 @@ __device__ __forceinline__ void st_dev(R* p, R v) {
 }
 // The same for readers on this XCD only: the store stops at the XCD's L2,
 // where the device-scope loads of its other CUs find it.
+// This is an assumption about gfx950 and not the language's memory model, in
+// which a workgroup-scope store and another workgroup's device-scope load are
+// a race: (1) a CU's vector cache writes every store through to its XCD's L2,
+// (2) a device-scope load misses the CU's cache and goes to that L2, which
+// cannot pass over a line that it holds modified, (3) XCC_ID names the L2.
+// Where it did not hold, a reader would go on seeing the sentinel: a word is 8
+// or 4 aligned bytes, written once between two launches, and whatever an
+// earlier launch left is the sentinel.  So the bounded wait would end with the
+// error of a sweep that cannot go on, never with another value.  Readers in
+// later launches see the stores as they see any other kernel's.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "st_xcd relies on the caches of gfx950"
+#endif
 template <typename R>
 __device__ __forceinline__ void st_xcd(R* p, R v) {
     using B = typename Real<R>::bits;
