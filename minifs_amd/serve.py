@@ -142,8 +142,10 @@ class Server:
         self.workers = workers
         self.tree = tuple(tree)     # TDTree parameters of the meshes' cell order
         self.device_metrics = device_metrics  # ComputeMetrics on the GPU (bitwise the host's)
-        # device bytes per cell, refined from the contexts actually created
-        self.bytes_per_cell = bytes_per_cell or (620.0 if precision == MFS_FP64 else 900.0)
+        # device bytes per cell: those of a request of 20k cells (960 and 1,153;
+        # larger ones take less, 6.0M cells 909 and 1,087), refined from the
+        # contexts actually created
+        self.bytes_per_cell = bytes_per_cell or (965.0 if precision == MFS_FP64 else 1160.0)
 
     def run(self, requests: list[Request], progress=None) -> dict:
         reqs = sorted(requests, key=lambda r: r.arrival)

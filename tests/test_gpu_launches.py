@@ -5,6 +5,7 @@ import pytest
 
 import minifs_amd as mfs
 from minifs_amd._lib import MFS_GRADIENT_INSIDE
+from minifs_amd.serve import Server
 
 pytestmark = pytest.mark.gpu
 
@@ -234,5 +235,18 @@ def test_device_memory_of_a_context(cells, precision, per_cell):
     held = s.info()["device_bytes"] / g.info["nTCell"]
     print(f"[launches] {held:.1f} bytes per {cells} cell", flush=True)
     assert held < per_cell
+    s.close()
+    g.close()
+
+
+@pytest.mark.parametrize("precision", [mfs.MFS_FP64, mfs.MFS_MIXED], ids=["fp64", "mixed"])
+@pytest.mark.parametrize("n", [15, 40])
+def test_server_reserves_what_a_request_takes(n, precision):
+    """The serving loop's first reservation covers the context of its smallest
+    requests and of larger ones, so that the budget holds from the start."""
+    print(f"[launches] reservation {n} precision={precision}", flush=True)
+    g, p = _grid("tet", (n, n, n), (4, 512))
+    s = mfs.Solver(g, p, precision=precision)
+    assert s.info()["device_bytes"] <= Server(precision, hbm_budget=1e9).bytes_per_cell * g.info["nTCell"]
     s.close()
     g.close()
