@@ -114,7 +114,7 @@ constexpr int kDefaultTailGrid = 64;
 constexpr int kThinWaves = 2;  // waves that a workgroup of the tail grid stands for
 // Workgroups per CU of a thin launch with side work.  The fewer, the less
 // their traffic delays the thin levels' hops, and the fewer nodes' cells
-// compete for an L2 (with 4 per CU the node values read 1.9 GB instead of 1.0
+// compete for an L2 (with 4 per CU the node values read 1.88 GB instead of 0.83
 // at 6.0M cells): one, as long as the tail still hides the gradient (6.0M
 // cells take it 590 us at one per CU, so a level of 1.2 us hides 12,000
 // cells), else three.  ms per iteration, gradient at 4 / 3 / 2 / 1 per CU with

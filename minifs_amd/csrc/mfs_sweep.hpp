@@ -18,10 +18,11 @@
 // the memory system's gathers, so what counts is cells per round.  With one
 // lane per face slot (16 cells per wave, 8 on meshes with up to 6 faces per
 // cell) half the lanes had no dependency and every cell's lanes ran the
-// limiter and the update.  Wide-level launches, forward / backward, before
-// and after: 6.0M tetrahedra FP64 808 / 938 -> 690 / 770 us, 262k hexahedra
-// FP64 190 / 203 -> 146 / 148 us, a mixed batch of 2.3M cells 603 / 686 ->
-// 433 / 452 us.
+// limiter and the update.  Wide-level launches, forward / backward, with one
+// lane per face slot and now: 6.0M tetrahedra FP64 808 / 938 -> 650 / 745 us,
+// 262k hexahedra FP64 190 / 203 -> 111 / 112 us (fewer levels are wide), a
+// mixed batch of 2.3M cells, whose sweeps are one launch each, 603 / 686 ->
+// 384 / 487 us.
 //
 // Schedule: cells are stored by tile (4096 consecutive mesh ids, a compact
 // region in TDTree numbering), then forward level; a chunk is as many cells
@@ -688,8 +689,8 @@ struct XcdArgs {
 // The side blocks fill the CUs that the sweep leaves idle without sharing its
 // XCD's issue slots and L2: on a second stream their workgroups landed there
 // too, and a tail of 303 us took 605 us beside the node values and 436 beside
-// the gradient (6.0M cells, FP64); inside, the two launches take 340 us with
-// the node values (292 us alone) and 481 with the gradient (397 alone).
+// the gradient (6.0M cells, FP64); inside, the two launches take 325 us with
+// the node values (292 us alone) and 450 with the gradient (397 alone).
 template <bool FWD, int MAXF, typename R>
 __global__ __launch_bounds__(kBlock) void k_sweep_xcd(XcdArgs<R> P) {
     const SweepArgs<R>& A = P.A;
